@@ -256,6 +256,7 @@ class Engine {
   int32_t* d_acolidx_ = nullptr;
   double* d_vals_ = nullptr;
   double* d_scale_ = nullptr;  // equilibration s_i (FP32 mode)
+  double* d_norm_ = nullptr;   // ||A||_inf (FP32 mode)
   double* d_arena64_ = nullptr;
   void* d_dinv_ = nullptr;     // inverted 16x16 diagonal tiles of the factor
   void* d_garena_ = nullptr;   // partitioned-inverse solve factor G (panel shapes, factor precision)
