@@ -63,10 +63,12 @@ typedef struct spk_options {
   int verbose;
   int profile;        /* time every kernel launch with HIP events */
   int device;         /* HIP device ordinal */
-  int merge_updates;  /* 1 (default): a chain child's update outside its parent's columns is
-                         computed inside the parent's Schur update (one scatter instead of two)
-                         on etree levels with enough update tiles to fill the GPU; 2: on every
-                         level; 0: every supernode scatters its whole update */
+  int merge_updates;  /* 1 (default): along a chain of supernodes (each the main child of the
+                         next) the updates beyond the chain's columns are applied once, by the
+                         chain's last member, and inside the chain a child's update beyond its
+                         parent's columns is computed with the parent's on etree levels with
+                         enough update tiles to fill the GPU; 2: on every level and for
+                         supernodes of any width; 0: every supernode applies its whole update */
   int solve_dataflow; /* must be 0 (default): one launch per etree level and kernel kind.
                          The dependency-driven sweeps (one persistent launch each) are
                          disabled in this build; Solve rejects 1 */
@@ -83,7 +85,7 @@ typedef struct spk_options {
                          lose accuracy).  0: block substitution, four launches per level */
   int autotune;       /* 1: the first spk_factorize of a structure with at least 1e9
                          Schur-update flops times every etree level's Schur launch under each
-                         kernel (64 x 64 tiles staged through LDS, 128 x 64 tiles, 64 x 64 tiles
+                         kernel (64 x 64 or 128 x 128 tiles staged through LDS, 64 x 64 tiles
                          with one wave per tile), task order (plan / longest first) and k split
                          (1-8 workgroups per tile) on the device and keeps the fastest
                          (spk_get_autotune), for structures factored many times (tuning costs
@@ -91,8 +93,9 @@ typedef struct spk_options {
                          reference counterpart */
   int schur_kernel;   /* 0 (default): the Schur-update kernel the autotuner (or, untuned, the
                          plan) chooses per level; 1: 64 x 64 tiles staged through LDS, 2: 128 x
-                         64 tiles, 3: 64 x 64 tiles with one wave per tile, on every level (no
-                         tuning); other values are rejected by spk_init */
+                         128 tiles, 3: 64 x 64 tiles with one wave per tile (1 on levels where an
+                         update spans more than two supernodes), on every level (no tuning);
+                         other values are rejected by spk_init */
 } spk_options;
 
 typedef struct spk_stats {
@@ -145,7 +148,7 @@ int spk_get_launch_trace(spk_handle h, int32_t* kinds, int64_t* grids, double* m
 int spk_get_launch_levels(spk_handle h, int32_t* levels, int max);
 /* The autotuner's choice per Schur launch (one per etree level with updates)
  * after the first factorization: level, k split (workgroups per tile), launch
- * variant (bit 0: tasks longest first instead of plan order; bit 1: 128 x 64
+ * variant (bit 0: tasks longest first instead of plan order; bit 1: 128 x 128
  * output tiles; bit 2: 64 x 64 tiles with one wave per tile; neither: 64 x 64
  * tiles staged through LDS), best time of the default configuration
  * and of the chosen one (ms); returns the number of records (<= max), 0 when
@@ -219,8 +222,17 @@ int spk_get_cells(spk_handle h, int32_t* cell_K, int32_t* cell_I, int32_t* cell_
 /* Schur-update merging chosen by the plan (no counterpart in the reference,
  * whose tasks update each target cell from one source supernode):
  * deferred_into[I] = 0-based parent that computes the part of supernode I's
- * update outside the parent's columns, -1 where I scatters its whole update. */
+ * update outside the parent's columns (what lies beyond the columns of their
+ * chain: together with the chain's last member), -1 for none. */
 int spk_get_update_merges(spk_handle h, int32_t* deferred_into /* nsuper */);
+/* The Schur update that supernode I (0-based) applies at its etree level:
+ * nseg[I] supernodes contribute to it (0: none), to its output columns (its
+ * off-diagonal rows) below bcut[I]; those below excl[I] lie in panels that no
+ * other supernode of the level updates.  spk_get_update_segment: contributor
+ * s of supernode I and, per off-diagonal row of I, the row of the
+ * contributor's panel (-1: it has no such row). */
+int spk_get_update_schedule(spk_handle h, int32_t* nseg, int32_t* bcut, int32_t* excl /* nsuper each */);
+int spk_get_update_segment(spk_handle h, int32_t I, int32_t s, int32_t* sn, int32_t* rows);
 /* Checks the task lists of the dependency-driven solve (no counterpart in
  * the reference): 0 when a single worker taking tasks in ticket order never
  * waits and every counter drains, < 0 with spk_last_error() otherwise. */

@@ -541,6 +541,41 @@ int spk_get_update_merges(spk_handle h, int32_t* deferred_into) {
   });
 }
 
+int spk_get_update_schedule(spk_handle h, int32_t* nseg, int32_t* bcut, int32_t* excl) {
+  if (!h || !nseg || !bcut || !excl) return fail("null argument");
+  return guarded([&]() {
+    const spk::Plan& p = h->engine.plan();
+    if ((int)p.chain_end.size() != p.nsuper) throw std::logic_error("no symbolic factorization");
+    std::fill_n(nseg, p.nsuper, 0);
+    std::fill_n(bcut, p.nsuper, 0);
+    std::fill_n(excl, p.nsuper, 0);
+    for (const spk::SchurEmit& e : p.schur_emit) {
+      const spk::SchurHead& hd = p.schur_heads[e.head];
+      nseg[e.I] = hd.nseg;
+      bcut[e.I] = hd.bcut;
+      excl[e.I] = hd.excl;
+    }
+    return 0;
+  });
+}
+
+int spk_get_update_segment(spk_handle h, int32_t I, int32_t s, int32_t* sn, int32_t* rows) {
+  if (!h || !sn || !rows) return fail("null argument");
+  return guarded([&]() {
+    const spk::Plan& p = h->engine.plan();
+    for (const spk::SchurEmit& e : p.schur_emit) {
+      if (e.I != I) continue;
+      const spk::SchurHead& hd = p.schur_heads[e.head];
+      if (s < 0 || s >= hd.nseg) break;
+      const spk::SchurSeg& g = p.schur_segs[hd.seg0 + s];
+      *sn = g.sn;
+      for (int32_t a = 0; a < p.sn[I].r - p.sn[I].w; ++a) rows[a] = g.moff < 0 ? g.shift + a : p.mmap[g.moff + a];
+      return 0;
+    }
+    throw std::out_of_range("no such update segment");
+  });
+}
+
 int spk_get_cell_counts(spk_handle h, int64_t* ncells, int64_t* nblocks) {
   if (!h || !ncells || !nblocks) return fail("null argument");
   return guarded([&]() {

@@ -310,7 +310,8 @@ void Engine::free_device() {
   dfree(d_tcol_);
   dfree(d_tmap_);
   dfree(d_rel_);
-  dfree(d_merges_);
+  dfree(d_heads_);
+  dfree(d_segs_);
   dfree(d_mmap_);
   dfree(d_amap_);
   dfree(d_invp0_);
@@ -367,7 +368,7 @@ void Engine::init(const EngineOptions& o) {
 int64_t Engine::device_bytes(int nrhs) const {
   auto vb = [](const auto& v) { return (int64_t)(v.size() * sizeof(v[0])); };
   const Plan& p = plan_;
-  int64_t b = vb(p.sn) + vb(p.lindx0) + p.upd_size * 16 + p.rel_size * 4 + vb(p.merges) + vb(p.mmap) + vb(p.amap) + vb(p.perm0) +
+  int64_t b = vb(p.sn) + vb(p.lindx0) + p.upd_size * 16 + p.rel_size * 4 + vb(p.schur_heads) + vb(p.schur_segs) + vb(p.mmap) + vb(p.amap) + vb(p.perm0) +
               vb(p.potrf_tasks) + vb(p.trsm_tasks) + vb(p.inpanel_tasks) +
               2 * (p.n_schur + p.n_schur_wide) * (int64_t)sizeof(Task4) + vb(p.fused_tasks) +
               vb(p.sdiag_tasks) + vb(p.soffm_tasks);
@@ -450,7 +451,8 @@ void Engine::ensure_device() {
     dfree(bad);
     if (hbad) throw std::logic_error("symbolic structure is not closed under elimination");
   }
-  d_merges_ = dupload(plan_.merges, s);
+  d_heads_ = dupload(plan_.schur_heads, s);
+  d_segs_ = dupload(plan_.schur_segs, s);
   d_mmap_ = dupload(plan_.mmap, s);
   d_amap_ = dupload(plan_.amap, s);
   {
@@ -838,14 +840,17 @@ void Engine::launch_diagtrsm(int bucket, bool ldl, unsigned g, const Task4* t, T
 #undef SPK_FUSED
 }
 
-// One Schur launch of range r: 64 x 64 tiles staged through LDS (k_update),
-// 128 x 64 tiles (k_schur_wide, alt bit 1) or 64 x 64 tiles with one wave per
-// tile (k_schur_w1, alt bit 2), plan or longest-first task order (alt bit 0),
+// One Schur launch of range r: 64 x 64 tiles staged through LDS (k_schur),
+// 128 x 128 tiles (alt bit 1) or 64 x 64 tiles with one wave per tile
+// (k_schur_w1, alt bit 2), plan or longest-first task order (alt bit 0),
 // each tile's k chunks split over ks workgroups (waves for k_schur_w1).
 template <typename T>
 void Engine::launch_schur(const LaunchRange& r, int alt, int ks, T* arena, hipStream_t st) {
   const SnInfo* sn = (const SnInfo*)d_sn_;
   const bool ldl = opt_.ldl != 0;
+  // k_schur_w1 takes tasks of at most two segments, and addresses panels
+  // through 32-bit buffer offsets: below 2 GiB
+  if ((alt & 4) && (r.nsegmax > 2 || plan_.max_panel * (int64_t)sizeof(T) >= (int64_t(1) << 31))) alt &= 1;
   const bool wide = (alt & 2) != 0;
   const int64_t cnt = wide ? r.count_w : r.count;
   if (cnt == 0) return;
@@ -853,24 +858,22 @@ void Engine::launch_schur(const LaunchRange& r, int alt, int ks, T* arena, hipSt
                                               : ((alt & 1) ? TA_SCHUR_LPT : TA_SCHUR)] +
                    (wide ? r.first_w : r.first);
   const unsigned gs = (unsigned)(cnt * ks);
-  // k_schur_w1 addresses panels through 32-bit buffer offsets: below 2 GiB
-  if ((alt & 4) && plan_.max_panel * (int64_t)sizeof(T) >= (int64_t(1) << 31)) alt &= 1;
   if (alt & 4) {  // one wave per (task, part): four per workgroup
     const unsigned gw = (unsigned)((cnt * ks + 3) / 4);
     if (ldl)
-      dev::k_schur_w1<T, true><<<gw, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, cnt, ks);
+      dev::k_schur_w1<T, true><<<gw, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_heads_, d_segs_, d_mmap_, cnt, ks);
     else
-      dev::k_schur_w1<T, false><<<gw, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, cnt, ks);
+      dev::k_schur_w1<T, false><<<gw, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_heads_, d_segs_, d_mmap_, cnt, ks);
   } else if (wide) {
     if (ldl)
-      dev::k_schur_wide<T, true><<<gs, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, cnt, ks);
+      dev::k_schur<T, true, dev::Tile128><<<gs, 512, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_heads_, d_segs_, d_mmap_, ks);
     else
-      dev::k_schur_wide<T, false><<<gs, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, cnt, ks);
+      dev::k_schur<T, false, dev::Tile128><<<gs, 512, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_heads_, d_segs_, d_mmap_, ks);
   } else {
     if (ldl)
-      dev::k_update<T, 1, true><<<gs, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, cnt, ks);
+      dev::k_schur<T, true, dev::Tile64><<<gs, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_heads_, d_segs_, d_mmap_, ks);
     else
-      dev::k_update<T, 1, false><<<gs, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, cnt, ks);
+      dev::k_schur<T, false, dev::Tile64><<<gs, 256, 0, st>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_heads_, d_segs_, d_mmap_, ks);
   }
 }
 
@@ -901,9 +904,9 @@ void Engine::factor_sequence(T* arena) {
       case 1: {
         const Task4* t = (const Task4*)d_tasks_[TA_INPANEL] + r.first;
         if (ldl)
-          dev::k_update<T, 0, true><<<g, 256, 0, stream_>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, r.count, 1);
+          dev::k_update<T, true><<<g, 256, 0, stream_>>>(sn, t, arena);
         else
-          dev::k_update<T, 0, false><<<g, 256, 0, stream_>>>(sn, t, arena, d_tcol_, d_tmap_, d_rel_, d_merges_, d_mmap_, r.count, 1);
+          dev::k_update<T, false><<<g, 256, 0, stream_>>>(sn, t, arena);
         break;
       }
       case 2:
@@ -977,6 +980,7 @@ void Engine::autotune_schur(T* arena) {
       for (int ks : {1, 2, 3, 4, 6, 8}) {
         const int64_t tiles = (alt & 2) ? r.count_w : r.count;
         if (tiles == 0 || ks > nqmin || tiles * ks > 8192) continue;
+        if (alt > 3 && r.nsegmax > 2) continue;
         if (alt == rec.alt0 && ks == rec.split0) continue;
         const double ms = time_of(r, alt, ks);
         ++rec.candidates;

@@ -34,14 +34,15 @@ struct EngineOptions {
   int device = 0;
   int profile = 0;        // record HIP events around every launch
   int verbose = 0;
-  int merge_updates = 1;  // 0 off, 1 on levels that fill the GPU, 2 every qualifying chain child
+  int merge_updates = 1;  // 0 off, 1 chains of wide supernodes, 2 every chain (see build_plan)
   int solve_dataflow = 0; // dependency-driven solve sweeps: disabled, requesting it is an error
   int solve_inverse = 1;  // partitioned-inverse solve where every supernode is <= kStep wide
   int refine = 0;         // 10*ordflag + altflag of the supernode reordering, 0 = none
   int autotune = 1;       // time the Schur launch configurations of every level on the first
                           // factorization of a plan with at least kAutotuneMinFlops Schur flops
-  int schur_kernel = 0;   // 0: tuner / plan default; 1, 2, 3: k_update, k_schur_wide, k_schur_w1
-                          // on every level (no tuning when set)
+  int schur_kernel = 0;   // 0: tuner / plan default; 1, 2, 3: k_schur with 64 x 64 or 128 x 128 tiles,
+                          // k_schur_w1 on every level (no tuning when set; k_schur where the
+                          // launch has tasks of more than two segments)
   std::vector<Int> user_perm;
 };
 
@@ -231,7 +232,8 @@ class Engine {
   int64_t* d_tcol_ = nullptr;
   int64_t* d_tmap_ = nullptr;
   int32_t* d_rel_ = nullptr;
-  MergeInfo* d_merges_ = nullptr;
+  SchurHead* d_heads_ = nullptr;
+  SchurSeg* d_segs_ = nullptr;
   int32_t* d_mmap_ = nullptr;
   int64_t* d_amap_ = nullptr;
   int32_t* d_invp0_ = nullptr;  // original -> permuted row, 0-based

@@ -14,11 +14,11 @@
 //  k_ptrsm       panel TRSM of 64 rows below that block on MFMA with the
 //                inverted 16x16 diagonal tiles (blockCell_t::trsm, :1104-1178).
 //  k_diagtrsm    both, one workgroup per 64-row tile (each factors the block).
-//  k_update<0>   trailing update of a panel wider than 160 inside itself.
-//  k_update<1>   Schur update of ancestors: -P P^T (LDL: -P D P^T) on FP64 /
-//                FP32 MFMA 16x16x4, scattered straight from registers into the
-//                target panels through precomputed relative indices with
-//                hardware atomics (blockCell_t::update, :1180-1466).
+//  k_update      trailing update of a panel wider than 160 inside itself.
+//  k_schur       Schur update of ancestors: -P P^T (LDL: -P D P^T) on FP64 /
+//                FP32 MFMA 16x16x4, written straight from registers into the
+//                target panels through precomputed relative indices
+//                (blockCell_t::update, :1180-1466).
 //  k_sdiag4 / k_sdiag3 / k_sdiag_fwd / k_soffm_fwd / k_scale_d / k_soffm_bwd /
 //  k_sdiag_bwd   supernodal forward/backward solve (forward_update[_contrib],
 //                back_update[_contrib], :1486-1797).
@@ -154,31 +154,39 @@ __global__ __launch_bounds__(256) void k_build_rel(const SnInfo* __restrict__ sn
 }
 
 // Schur task lists from the per-supernode records: one workgroup per
-// supernode writes its 64 x 64 tiles (plan order and longest-first
-// positions) and its 128 x 64 tiles; a thread per row tile.
+// supernode writes its 64 x 64 and its 128 x 128 tiles (plan order and
+// longest-first positions), a thread per row tile, each tile's k parts one
+// after another.  The tiles of a supernode go in blocks of 8 x 8 (see
+// xcd_unit), block rows first, inside a block row tile by row tile.
+constexpr int kSuper = 8;
+__device__ __forceinline__ void emit_tiles(const SchurEmit& e, int nt, int ntj, int split,
+                                           Task4* __restrict__ plan, Task4* __restrict__ lpt) {
+  for (int ti = (int)threadIdx.x; ti < nt; ti += (int)blockDim.x) {
+    const int t_lo = ti / kSuper * kSuper, t_hi = min(t_lo + kSuper, nt);
+    const int64_t row0 = schur_tiles_before(t_lo, ntj);
+    for (int j0 = 0; j0 < min(ti + 1, ntj); j0 += kSuper) {
+      int64_t at = row0;  // tiles of the block row left of this block, and of the block's rows above
+      for (int q = t_lo; q < t_hi; ++q) {
+        const int lim = min(q + 1, ntj);
+        at += min(lim, j0) + (q < ti ? min(max(lim - j0, 0), kSuper) : 0);
+      }
+      for (int tj = j0; tj < min(min(ti + 1, ntj), j0 + kSuper); ++tj, ++at) {
+        for (int p = 0; p < split; ++p) {
+          const Task4 t{e.I, ti, tj | (p << kTileBits), e.head};
+          plan[at * split + p] = t;
+          lpt[at * split + p] = t;
+        }
+      }
+    }
+  }
+}
 __global__ __launch_bounds__(256) void k_emit_schur(const SchurEmit* __restrict__ emit, int64_t nemit,
                                                     Task4* __restrict__ t0, Task4* __restrict__ t1,
                                                     Task4* __restrict__ t2, Task4* __restrict__ t3) {
   for (int64_t q = blockIdx.x; q < nemit; q += gridDim.x) {
     const SchurEmit e = emit[q];
-    for (int ti = (int)threadIdx.x; ti < e.nt; ti += (int)blockDim.x) {
-      const int64_t at = schur_tiles_before(ti, e.ntj);
-      const int ntj = min(ti + 1, e.ntj);
-      for (int tj = 0; tj < ntj; ++tj) {
-        const Task4 t{e.I, ti, tj, e.d};
-        t0[e.first[0] + at + tj] = t;
-        t1[e.first[1] + at + tj] = t;
-      }
-    }
-    for (int ti = (int)threadIdx.x; ti < e.ntw; ti += (int)blockDim.x) {
-      const int64_t at = schur_wide_before(ti, e.ntj);
-      const int ntj = min(2 * ti + 2, e.ntj);
-      for (int tj = 0; tj < ntj; ++tj) {
-        const Task4 t{e.I, ti, tj, e.d};
-        t2[e.first[2] + at + tj] = t;
-        t3[e.first[3] + at + tj] = t;
-      }
-    }
+    emit_tiles(e, e.nt, e.ntj, e.split, t0 + e.first[0], t1 + e.first[1]);
+    emit_tiles(e, e.ntw, e.ntjw, 1, t2 + e.first[2], t3 + e.first[3]);
   }
 }
 
@@ -773,483 +781,389 @@ __global__ __launch_bounds__(NT) void k_diagtrsm(const SnInfo* __restrict__ sn,
 }
 
 // ---------------------------------------------------------------------------
-// MFMA tile update.  The 64x64 output tile C[a][b] = sum_k Pa[a][k] Pb[b][k]
+// MFMA tile updates.  The 64x64 output tile C[a][b] = sum_k Pa[a][k] Pb[b][k]
 // (times D[k] for LDL) is computed by 4 waves, each owning a 32x32 quarter as
 // 2x2 blocks of 16x16x4 MFMA.  MFMA operand A is the b side and operand B the
 // a side, so an accumulator element (lane l, slot v) holds b = Mfma<T>::row(l,v)
 // and a = l%16 within its block: 16 consecutive lanes own 16 consecutive
-// target rows, which keeps the scatter coalesced.
-// MODE 0: in-panel trailing update of step t.b (direct read-modify-write).
-// MODE 1: Schur update of ancestor panels (atomic scatter).
+// target rows, which keeps the stores coalesced.  K goes through LDS in chunks
+// of 32 columns; the next chunk's loads are in flight during the products.
 // ---------------------------------------------------------------------------
-template <typename T, int MODE, bool LDL>
-__global__ __launch_bounds__(NT) void k_update(const SnInfo* __restrict__ sn,
-                                                const Task4* __restrict__ tasks,
-                                                T* __restrict__ arena,
-                                                const int64_t* __restrict__ tcol,
-                                                const int64_t* __restrict__ tmap,
-                                                const int32_t* __restrict__ rel,
-                                                const MergeInfo* __restrict__ merges,
-                                                const int32_t* __restrict__ mmap, int64_t ntasks,
-                                                int ksplit) {
+// Work unit of workgroup `b` of a grid of n units: workgroups go to the eight
+// XCDs in turn, each with an L2 of its own, so every XCD takes runs of 64
+// consecutive units (an 8 x 8 block of tiles: 16 operand stripes for 64
+// tiles).
+__device__ __forceinline__ unsigned xcd_unit(unsigned b, unsigned n) {
+  constexpr unsigned XCDS = 8, RUN = kSuper * kSuper, WIN = XCDS * RUN;
+  const unsigned w0 = b / WIN * WIN, r = b - w0;
+  const unsigned len = min(n - w0, WIN), per = len / XCDS, rem = len % XCDS;
+  const unsigned x = r % XCDS;
+  return w0 + x * per + min(x, rem) + r / XCDS;
+}
+
+// Shape of a workgroup's output tile: E x E, WA x WB waves over (rows a,
+// columns b), KC k columns per LDS chunk.
+struct Tile64 {
+  static constexpr int E = 64, WA = 2, WB = 2, KC = 32;
+};
+struct Tile128 {
+  static constexpr int E = 128, WA = 4, WB = 2, KC = 16;
+};
+template <typename T, class S>
+struct TileLds {
+  T As[S::KC][S::E + 1];  // odd pitch: the 4 k rows a wave reads hit different banks
+  T Bs[S::KC][S::E + 1];
+  T Dk[S::KC];
+};
+
+// acc += the chunk's products over its first 4 nkk k columns; wave (wa, wb)
+// owns rows E / WA * wa .. and output columns E / WB * wb ..  The LDS reads
+// run one step of 4 columns ahead of the products.
+template <typename T, bool LDL, class S>
+__device__ __forceinline__ void tile_products(const TileLds<T, S>& L,
+                                              typename Mfma<T>::v4 (&acc)[S::E / S::WB / 16][S::E / S::WA / 16],
+                                              int nkk, int wa, int wb, int lane) {
+  constexpr int BA = S::E / S::WA / 16, BB = S::E / S::WB / 16;
+  T bf[2][BB], af[2][BA], dk[2];
+  auto load = [&](int kk, int h) {
+    const int k = kk * 4 + (lane >> 4);
+#pragma unroll
+    for (int bi = 0; bi < BB; ++bi) bf[h][bi] = L.Bs[k][(wb * BB + bi) * 16 + (lane & 15)];
+    if (LDL) dk[h] = L.Dk[k];
+#pragma unroll
+    for (int aj = 0; aj < BA; ++aj) af[h][aj] = L.As[k][(wa * BA + aj) * 16 + (lane & 15)];
+  };
+  auto mma = [&](int h) {
+#pragma unroll
+    for (int bi = 0; bi < BB; ++bi) {
+      const T b = LDL ? bf[h][bi] * dk[h] : bf[h][bi];
+#pragma unroll
+      for (int aj = 0; aj < BA; ++aj) acc[bi][aj] = Mfma<T>::mma(b, af[h][aj], acc[bi][aj]);
+    }
+  };
+  load(0, 0);
+#pragma unroll
+  for (int kk = 0; kk < S::KC / 4; ++kk) {
+    if (kk >= nkk) break;  // uniform over the wave
+    if (kk + 1 < S::KC / 4) load(kk + 1, (kk + 1) & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(kk & 1);
+  }
+}
+
+// In-panel trailing update of step t.b of a panel wider than kStep (direct
+// read-modify-write).  Task {sn, step, ti, tj}.
+template <typename T, bool LDL>
+__global__ __launch_bounds__(NT) void k_update(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+                                               T* __restrict__ arena) {
   typedef typename Mfma<T>::v4 v4;
-  constexpr int KC = kSchurKC;
-  constexpr int LDS_LD = TILE + 1;  // odd pitch: the 4 k rows a wave reads hit different banks
-  __shared__ T As[KC][LDS_LD];
-  __shared__ T Bs[KC][LDS_LD];
-  __shared__ T Dk[KC];
-  __shared__ int64_t sTc[TILE], sTm[TILE];  // MODE 1: scatter bases of the tile's output columns
-  // grid-stride over (task, k part) pairs (the launches use one workgroup
-  // per pair); part `part` of a task covers k chunks [q_lo, q_hi)
-  for (int64_t gi = blockIdx.x; gi < ntasks * ksplit; gi += gridDim.x) {
-  const int64_t task = gi / ksplit;
-  const int part = (int)(gi - task * ksplit);
-  const Task4 t = tasks[task];
+  constexpr int KC = kSchurKC, NQ = KC / 4;
+  __shared__ TileLds<T, Tile64> L;
+  const Task4 t = tasks[blockIdx.x];
   const SnInfo s = sn[t.a];
   T* __restrict__ P = arena + s.off;
   const int64_t ld = s.r;
-  int kbeg, K, arow0, brow0, alim, blim, ti, tj;
-  if (MODE == 0) {
-    kbeg = t.b * kStep;
-    K = min(kStep, s.w - kbeg);
-    const int rb = kbeg + K;
-    ti = t.c;
-    tj = t.d;
-    arow0 = rb + ti * TILE;
-    brow0 = rb + tj * TILE;
-    alim = s.r;
-    blim = s.w;
-  } else {
-    kbeg = 0;
-    K = s.w;
-    ti = t.b;
-    tj = t.c;
-    arow0 = s.w + ti * TILE;
-    brow0 = s.w + tj * TILE;
-    alim = s.r;
-    blim = s.r;
-  }
+  const int kbeg = t.b * kStep, K = min(kStep, s.w - kbeg), rb0 = kbeg + K;
+  const int arow0 = rb0 + t.c * TILE, brow0 = rb0 + t.d * TILE;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wb = wave >> 1, wa = wave & 1;
+  const int arow = min(arow0 + lane, s.r - 1), brow = min(brow0 + lane, s.w - 1);
   v4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
-
-  // loader mapping: a wave reads 64 consecutive rows of one k column
-  const int lrow = tid & 63, lk = tid >> 6;
-  const bool arow_ok = arow0 + lrow < alim;
-  const bool brow_ok = brow0 + lrow < blim;
-  const int arow = min(arow0 + lrow, alim - 1), brow = min(brow0 + lrow, blim - 1);
-  constexpr int NQ = KC / 4;
-  // MODE 1 with t.d > 0: after the K columns of this panel, K2 more k
-  // columns from a merged child's panel, whose rows are gathered through
-  // the row map (rows the child lacks are zero)
-  int K2 = 0;
-  const T* __restrict__ P2 = P;
-  int64_t ld2 = 1;
-  int arow2 = 0, brow2 = 0;
-  bool arow2_ok = false, brow2_ok = false;
-  if (MODE == 1 && t.d > 0) {
-    const MergeInfo mg = merges[t.d - 1];
-    K2 = mg.w;
-    P2 = arena + mg.off;
-    ld2 = mg.ld;
-    const int ma = mmap[mg.moff + (arow - s.w)];
-    const int mb = mmap[mg.moff + (brow - s.w)];
-    arow2_ok = arow_ok && ma >= 0;
-    brow2_ok = brow_ok && mb >= 0;
-    arow2 = max(ma, 0);
-    brow2 = max(mb, 0);
-  }
-  const int nq1 = (K + KC - 1) / KC;
-  const int nq = nq1 + (K2 + KC - 1) / KC;
-  const int q_lo = (int)((int64_t)part * nq / ksplit), q_hi = (int)((int64_t)(part + 1) * nq / ksplit);
-  if (q_lo >= q_hi) continue;  // uniform over the workgroup
-  // A chunk is loaded from clamped (valid) addresses into ra/rb with its
-  // validity bits in mk; the bits are applied when the chunk is written to
-  // LDS, a chunk later, so nothing consumes the loads before the MFMAs of
-  // the current chunk have issued.  LDL: dv holds d_k of k column tid.
   T ra[NQ], rb[NQ], dv = T(0);
-  unsigned mk = 0;
-  auto fetch = [&](int qc) {
-    unsigned m = 0;
-    if (qc < nq1) {
-      const int kc = qc * KC;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        const int kg = kc + lk + 4 * q;
-        const T* col = P + (int64_t)(kbeg + min(kg, K - 1)) * ld;
-        ra[q] = col[arow];
-        rb[q] = col[brow];
-        m |= (unsigned)((kg < K) & arow_ok) << q;
-        m |= (unsigned)((kg < K) & brow_ok) << (q + NQ);
-      }
-      if (LDL) {
-        const int kg = min(kc + (tid & (KC - 1)), K - 1);
-        dv = P[(int64_t)(kbeg + kg) * ld + kbeg + kg];
-        m |= (unsigned)(kc + (tid & (KC - 1)) < K) << (2 * NQ);
-      }
-    } else {
-      const int kc = (qc - nq1) * KC;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        const int kg = kc + lk + 4 * q;
-        const T* col = P2 + (int64_t)min(kg, K2 - 1) * ld2;
-        ra[q] = col[arow2];
-        rb[q] = col[brow2];
-        m |= (unsigned)((kg < K2) & arow2_ok) << q;
-        m |= (unsigned)((kg < K2) & brow2_ok) << (q + NQ);
-      }
-      if (LDL) {
-        const int kg = min(kc + (tid & (KC - 1)), K2 - 1);
-        dv = P2[(int64_t)kg * ld2 + kg];
-        m |= (unsigned)(kc + (tid & (KC - 1)) < K2) << (2 * NQ);
-      }
-    }
-    mk = m;
-  };
-  // On a diagonal tile (ti == tj) the wave holding rows b of the upper half
-  // and columns a of the lower half (wb > wa) only produces entries a < b,
-  // which are never stored: it skips its products.
-  const bool idle = (ti == tj) && (wb > wa);
-  // MODE 1: the scatter bases tcol / tmap of the tile's 64 output columns b
-  // are loaded with the first chunk and kept in LDS, so the epilogue needs
-  // one memory round trip (rel) instead of two, and that one is issued
-  // before the last chunk's products
-  int64_t tcv = 0, tmv = 0;
-  const int m = s.r - s.w;
-  if (MODE == 1 && tid < TILE) {
-    const int bc = min(tj * TILE + tid, m - 1);
-    tcv = tcol[s.upd + bc];
-    tmv = tmap[s.upd + bc];
-  }
-  fetch(q_lo);
-  auto stage = [&](int qc) {
+  auto fetch = [&](int kc) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      As[lk + 4 * q][lrow] = ((mk >> q) & 1u) ? ra[q] : T(0);
-      Bs[lk + 4 * q][lrow] = ((mk >> (q + NQ)) & 1u) ? rb[q] : T(0);
+      const T* col = P + (int64_t)(kbeg + min(kc + wave + 4 * q, K - 1)) * ld;
+      ra[q] = col[arow];
+      rb[q] = col[brow];
     }
-    if (LDL && tid < KC) Dk[tid] = ((mk >> (2 * NQ)) & 1u) ? dv : T(0);
-    if (MODE == 1 && qc == q_lo && tid < TILE) {
-      sTc[tid] = tcv;
-      sTm[tid] = tmv;
-    }
-    __syncthreads();
-  };
-  auto products = [&](int qc) {
-    // k steps of 4 that hold valid columns in this chunk (the last chunk of
-    // each part is partial: its zero-filled tail is not multiplied)
-    const int krem = qc < nq1 ? K - qc * KC : K2 - (qc - nq1) * KC;
-    const int nkk = idle ? 0 : min(KC / 4, (krem + 3) >> 2);
-#pragma unroll
-    for (int kk = 0; kk < KC / 4; ++kk) {
-      if (kk >= nkk) break;  // uniform over the wave
-      const int k = kk * 4 + (lane >> 4);
-      T bf[2], af[2];
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi) {
-        bf[bi] = Bs[k][wb * 32 + bi * 16 + (lane & 15)];
-        if (LDL) bf[bi] *= Dk[k];
-      }
-#pragma unroll
-      for (int aj = 0; aj < 2; ++aj) af[aj] = As[k][wa * 32 + aj * 16 + (lane & 15)];
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int aj = 0; aj < 2; ++aj) acc[bi][aj] = Mfma<T>::mma(bf[bi], af[aj], acc[bi][aj]);
+    if (LDL) {
+      const int kg = kbeg + min(kc + (tid & (KC - 1)), K - 1);
+      dv = P[(int64_t)kg * ld + kg];
     }
   };
-  for (int qc = q_lo; qc < q_hi - 1; ++qc) {
-    stage(qc);
-    fetch(qc + 1);  // next chunk in flight during the MFMAs
-    products(qc);
+  // On a diagonal tile the wave holding columns b of the upper half and rows
+  // a of the lower half only produces entries a < b, which are never stored
+  const bool idle = (t.c == t.d) && (wb > wa);
+  fetch(0);
+  for (int kc = 0; kc < K; kc += KC) {
+    const int kv = min(KC, K - kc);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const bool in = wave + 4 * q < kv;
+      L.As[wave + 4 * q][lane] = in ? ra[q] : T(0);
+      L.Bs[wave + 4 * q][lane] = in ? rb[q] : T(0);
+    }
+    if (LDL && tid < KC) L.Dk[tid] = tid < kv ? dv : T(0);
+    __syncthreads();
+    if (kc + KC < K) fetch(kc + KC);
+    tile_products<T, LDL, Tile64>(L, acc, idle ? 0 : (kv + 3) >> 2, wa, wb, lane);
     __syncthreads();
   }
-  // last chunk (peeled: the prefetch registers are free, the scatter
-  // offsets take their place)
-  stage(q_hi - 1);
-  // MODE 1: scatter offsets of the 16 outputs of this lane, target column
-  // base from LDS plus the relative row (rel is defined for rows a >= the
-  // first row of b's target group: clamped, unconditional loads)
-  int64_t off[2][4][2];
-  if (MODE == 1) {
+  // every load first (clamped, unconditional, one wait), then the stores
+  T cur[2][2][4];
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+  for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+    for (int aj = 0; aj < 2; ++aj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int bl = wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
-        const int bc = min(tj * TILE + bl, m - 1);
-        const int64_t tc = sTc[bl], tmb = sTm[bl];
-#pragma unroll
-        for (int aj = 0; aj < 2; ++aj) {
-          const int aoff = ti * TILE + wa * 32 + aj * 16 + (lane & 15);
-          const int ac = min(max(aoff, bc), m - 1);
-          off[bi][v][aj] = tc + rel[tmb + ac];
-        }
+        const int bg = brow0 + wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
+        const int ag = arow0 + wa * 32 + aj * 16 + (lane & 15);
+        cur[bi][aj][v] = P[(int64_t)min(bg, s.w - 1) * ld + min(ag, s.r - 1)];
       }
-  }
-  products(q_hi - 1);
-
-  // Epilogue: every load first (clamped, unconditional, one wait), then the
-  // predicated stores / atomics.
-  if (MODE == 0) {
-    T cur[2][2][4];
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+  for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-      for (int aj = 0; aj < 2; ++aj)
+    for (int aj = 0; aj < 2; ++aj)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int bg = brow0 + wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
-          const int ag = arow0 + wa * 32 + aj * 16 + (lane & 15);
-          cur[bi][aj][v] = P[(int64_t)min(bg, s.w - 1) * ld + min(ag, s.r - 1)];
-        }
+      for (int v = 0; v < 4; ++v) keep(cur[bi][aj][v]);
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+  for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-      for (int aj = 0; aj < 2; ++aj)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) keep(cur[bi][aj][v]);
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-      for (int aj = 0; aj < 2; ++aj)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int bg = brow0 + wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
-          const int ag = arow0 + wa * 32 + aj * 16 + (lane & 15);
-          if (ag < s.r && bg < s.w && ag >= bg)
-            P[(int64_t)bg * ld + ag] = cur[bi][aj][v] - acc[bi][aj][v];
-        }
-  } else {
-    // a deferred supernode scatters only the output columns in its parent
-    const int bcut = t.d < 0 ? -t.d : m;
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+    for (int aj = 0; aj < 2; ++aj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int boff = tj * TILE + wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
-#pragma unroll
-        for (int aj = 0; aj < 2; ++aj) {
-          const int aoff = ti * TILE + wa * 32 + aj * 16 + (lane & 15);
-          if (boff < bcut && aoff < m && aoff >= boff) atomic_add(arena + off[bi][v][aj], -acc[bi][aj][v]);
-        }
+        const int bg = brow0 + wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
+        const int ag = arow0 + wa * 32 + aj * 16 + (lane & 15);
+        if (ag < s.r && bg < s.w && ag >= bg) P[(int64_t)bg * ld + ag] = cur[bi][aj][v] - acc[bi][aj][v];
       }
-  }
-  // a workgroup that takes another (task, part) rewrites As / Bs / sTc only
-  // after every wave has finished reading them
-  if (gi + gridDim.x < ntasks * ksplit) __syncthreads();
-  }
 }
 
-// ---------------------------------------------------------------------------
-// Schur update with 128 x 64 output tiles (rows a x columns b; the
-// autotuner's wide candidate).  Same algorithm as k_update<T,1,LDL>: C =
-// -P_a P_b^T (LDL: -P_a D P_b^T) over the supernode's k columns (and a merged
-// child's, gathered through the row map), K in chunks of 32 staged through
-// LDS with the next chunk in flight, scatter through tcol/tmap/rel with
-// atomics.  Each wave owns 64 a-rows x 32 b-columns, 4 x 2 MFMA 16x16x4
-// blocks: every k step reads 6 LDS operands for 8 products (4 for 4 in the
-// 64 x 64 tile), and a tile reads 192 rows of operands for 8192 outputs
-// (128 for 4096).  Task {sn, 128-row tile ti, 64-column tile tj, d} with
-// 64 tj <= 128 ti + 127; d as in k_update.
-// ---------------------------------------------------------------------------
-template <typename T, bool LDL>
-__global__ __launch_bounds__(NT) void k_schur_wide(const SnInfo* __restrict__ sn,
-                                                    const Task4* __restrict__ tasks,
-                                                    T* __restrict__ arena,
-                                                    const int64_t* __restrict__ tcol,
-                                                    const int64_t* __restrict__ tmap,
-                                                    const int32_t* __restrict__ rel,
-                                                    const MergeInfo* __restrict__ merges,
-                                                    const int32_t* __restrict__ mmap, int64_t ntasks,
-                                                    int ksplit) {
+// Schur update of ancestor panels: task {sn, ti, tj, head}, one workgroup per
+// (task, k part).  The k columns run over the head's segments (the supernode
+// itself, then chain members whose updates it takes over; see SchurSeg), each
+// segment's last chunk partial; k part p covers chunks [q_lo, q_hi).
+// Targets are arena[tcol[b] + rel[tmap[b] + a]].
+// Bound by the matrix cores where k is long: 54 TFLOP/s at m = 3600, k =
+// 1800 in FP64 (a loop without the operand loads: 66; the chip's 16x16x4
+// rate: 71-78), by the writes where k is short (see `plain` below).  64 x 64
+// tiles in 122 registers and 34 KB of LDS leave four workgroups per CU, which
+// cover each other's barriers, row lookups and writes.
+template <typename T, bool LDL, class S>
+__global__ __launch_bounds__(64 * S::WA * S::WB, 4) void k_schur(
+    const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, T* __restrict__ arena,
+    const int64_t* __restrict__ tcol, const int64_t* __restrict__ tmap, const int32_t* __restrict__ rel,
+    const SchurHead* __restrict__ heads, const SchurSeg* __restrict__ segs, const int32_t* __restrict__ mmap,
+    int ksplit) {
   typedef typename Mfma<T>::v4 v4;
-  constexpr int KC = kSchurKC;
-  constexpr int TA = 2 * TILE, TB = TILE;
-  constexpr int NQ = KC / 4;
-  __shared__ T As[KC][TA + 1];  // odd pitches: the 4 k rows a wave reads hit different banks
-  __shared__ T Bs[KC][TB + 1];
-  __shared__ T Dk[KC];
-  __shared__ int64_t sTc[TB], sTm[TB];
-  for (int64_t gi = blockIdx.x; gi < ntasks * ksplit; gi += gridDim.x) {
-    const int64_t task = gi / ksplit;
-    const int part = (int)(gi - task * ksplit);
-    const Task4 t = tasks[task];
-    const SnInfo s = sn[t.a];
-    const T* __restrict__ P = arena + s.off;
-    const int64_t ld = s.r;
-    const int K = s.w, m = s.r - s.w;
-    const int ti = t.b, tj = t.c;
-    const int arow0 = s.w + ti * TA, brow0 = s.w + tj * TB;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wb = wave >> 1, wa = wave & 1;
-    v4 acc[2][4];
+  constexpr int E = S::E, KC = S::KC, NW = S::WA * S::WB, NQ = KC / NW, NR = E / 64;
+  constexpr int BA = E / S::WA / 16, BB = E / S::WB / 16;
+  __shared__ TileLds<T, S> L;
+  __shared__ int64_t sTc[E], sTm[E];  // scatter bases of the tile's output columns
+  const unsigned unit = xcd_unit(blockIdx.x, gridDim.x);
+  const unsigned task = unit / (unsigned)ksplit;
+  const int part = (int)(unit - task * (unsigned)ksplit);
+  const Task4 t = tasks[task];
+  const SnInfo s = sn[t.a];
+  const SchurHead hd = heads[t.d];
+  const int m = s.r - s.w, ti = t.b, tj = t.c & kTileMask;
+  const int nq = E == 64 ? hd.nq : hd.nq16;
+  // k parts: the task's own part and the launch's
+  const int np = (E == 64 ? hd.split : 1) * ksplit, p = (t.c >> kTileBits) * ksplit + part;
+  const int q_lo = (int)((int64_t)p * nq / np), q_hi = (int)((int64_t)(p + 1) * nq / np);
+  if (q_lo >= q_hi) return;  // the whole workgroup
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wb = wave / S::WA, wa = wave % S::WA;
+  // the segment being loaded: rows ar / br of its panel for this lane's
+  // off-diagonal rows (past m: clamped, they only reach outputs that are
+  // never stored), column kc next
+  int seg = hd.seg0, kc = 0, Ks, ar[NR], br[NR];
+  bool mapped = false;  // its rows go through the row map
+  int64_t ld;
+  const T* __restrict__ P;
+  auto open_segment = [&]() {
+    const SchurSeg g = segs[seg];
+    P = arena + g.off;
+    ld = g.ld;
+    Ks = g.w;
+    mapped = g.moff >= 0;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = v4{0, 0, 0, 0};
-    // loader: a wave reads 64 consecutive rows of one k column; A rows in two
-    // halves of 64
-    const int lrow = tid & 63, lk = tid >> 6;
-    bool aok[2];
-    int arow[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      aok[h] = arow0 + h * 64 + lrow < s.r;
-      arow[h] = min(arow0 + h * 64 + lrow, s.r - 1);
+    for (int h = 0; h < NR; ++h) {
+      const int am = min(ti * E + h * 64 + lane, m - 1), bm = min(tj * E + h * 64 + lane, m - 1);
+      if (!mapped) {
+        ar[h] = g.shift + am;
+        br[h] = g.shift + bm;
+      } else {
+        ar[h] = mmap[g.moff + am];
+        br[h] = mmap[g.moff + bm];
+      }
     }
-    const bool bok = brow0 + lrow < s.r;
-    const int brow = min(brow0 + lrow, s.r - 1);
-    int K2 = 0;
-    const T* __restrict__ P2 = P;
-    int64_t ld2 = 1;
-    int arow2[2] = {0, 0}, brow2 = 0;
-    bool aok2[2] = {false, false}, bok2 = false;
-    if (t.d > 0) {
-      const MergeInfo mg = merges[t.d - 1];
-      K2 = mg.w;
-      P2 = arena + mg.off;
-      ld2 = mg.ld;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int ma = mmap[mg.moff + (arow[h] - s.w)];
-        aok2[h] = aok[h] && ma >= 0;
-        arow2[h] = max(ma, 0);
-      }
-      const int mb = mmap[mg.moff + (brow - s.w)];
-      bok2 = bok && mb >= 0;
-      brow2 = max(mb, 0);
+  };
+  if (np > 1) {  // the part's first chunk
+    int q = q_lo;
+    for (;;) {
+      const int n = (segs[seg].w + KC - 1) / KC;
+      if (q < n) break;
+      q -= n;
+      ++seg;
     }
-    const int nq1 = (K + KC - 1) / KC;
-    const int nq = nq1 + (K2 + KC - 1) / KC;
-    const int q_lo = (int)((int64_t)part * nq / ksplit), q_hi = (int)((int64_t)(part + 1) * nq / ksplit);
-    if (q_lo >= q_hi) continue;  // uniform over the workgroup
-    // chunk registers: A halves, B; validity bits applied at the LDS write
-    T ra[2][NQ], rb[NQ], dv = T(0);
-    unsigned mk = 0;
-    auto fetch = [&](int qc) {
-      unsigned mm = 0;
-      const bool own = qc < nq1;
-      const int kc = (own ? qc : qc - nq1) * KC;
-      const int Kp = own ? K : K2;
-      const T* __restrict__ Pp = own ? P : P2;
-      const int64_t ldp = own ? ld : ld2;
+    kc = q * KC;
+  }
+  open_segment();
+  int64_t tcv = 0, tmv = 0;
+  if (tid < E) {
+    const int b = min(tj * E + tid, m - 1);
+    tcv = tcol[s.upd + b];
+    tmv = tmap[s.upd + b];
+  }
+  v4 acc[BB][BA];
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        const int kg = kc + lk + 4 * q;
-        const T* col = Pp + (int64_t)min(kg, Kp - 1) * ldp;
+  for (int i = 0; i < BB; ++i)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          ra[h][q] = col[own ? arow[h] : arow2[h]];
-          mm |= (unsigned)((kg < Kp) & (own ? aok[h] : aok2[h])) << (h * NQ + q);
-        }
-        rb[q] = col[own ? brow : brow2];
-        mm |= (unsigned)((kg < Kp) & (own ? bok : bok2)) << (2 * NQ + q);
-      }
-      if (LDL) {
-        const int kg = min(kc + (tid & (KC - 1)), Kp - 1);
-        dv = Pp[(int64_t)kg * ldp + kg];
-        mm |= (unsigned)(kc + (tid & (KC - 1)) < Kp) << (3 * NQ);
-      }
-      mk = mm;
-    };
-    // a wave whose 64 x 32 block lies wholly above the diagonal (every a < b)
-    // skips its products
-    const bool idle = ti * TA + wa * 64 + 63 < tj * TB + wb * 32;
-    int64_t tcv = 0, tmv = 0;
-    if (tid < TB) {
-      const int bc = min(tj * TB + tid, m - 1);
-      tcv = tcol[s.upd + bc];
-      tmv = tmap[s.upd + bc];
+    for (int j = 0; j < BA; ++j) acc[i][j] = v4{0, 0, 0, 0};
+  // A wave loads 64 rows of one k column at a time, from clamped (valid)
+  // addresses; columns past the segment (kv) and rows that the segment lacks
+  // are zeroed when the chunk is written to LDS, a chunk later.
+  T ra[NQ][NR], rb[NQ][NR], dv = T(0);
+  int kv = 0;
+  bool aok[NR], bok[NR], whole = false;
+  auto fetch = [&](int q) {
+    kv = min(KC, Ks - kc);
+    whole = kv == KC && !mapped;
+    int ac[NR], bc[NR];
+#pragma unroll
+    for (int h = 0; h < NR; ++h) {
+      aok[h] = ar[h] >= 0;
+      bok[h] = br[h] >= 0;
+      ac[h] = max(ar[h], 0);
+      bc[h] = max(br[h], 0);
     }
-    fetch(q_lo);
-    auto stage = [&](int qc) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
+    for (int i = 0; i < NQ; ++i) {
+      const T* col = P + (int64_t)min(kc + wave + NW * i, Ks - 1) * ld;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) As[lk + 4 * q][h * 64 + lrow] = ((mk >> (h * NQ + q)) & 1u) ? ra[h][q] : T(0);
-        Bs[lk + 4 * q][lrow] = ((mk >> (2 * NQ + q)) & 1u) ? rb[q] : T(0);
+      for (int h = 0; h < NR; ++h) {
+        ra[i][h] = col[ac[h]];
+        rb[i][h] = col[bc[h]];
       }
-      if (LDL && tid < KC) Dk[tid] = ((mk >> (3 * NQ)) & 1u) ? dv : T(0);
-      if (qc == q_lo && tid < TB) {
-        sTc[tid] = tcv;
-        sTm[tid] = tmv;
-      }
-      __syncthreads();
-    };
-    auto products = [&](int qc) {
-      const int krem = qc < nq1 ? K - qc * KC : K2 - (qc - nq1) * KC;
-      const int nkk = idle ? 0 : min(KC / 4, (krem + 3) >> 2);
-#pragma unroll
-      for (int kk = 0; kk < KC / 4; ++kk) {
-        if (kk >= nkk) break;  // uniform over the wave
-        const int k = kk * 4 + (lane >> 4);
-        T bf[2], af[4];
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-          bf[bi] = Bs[k][wb * 32 + bi * 16 + (lane & 15)];
-          if (LDL) bf[bi] *= Dk[k];
-        }
-#pragma unroll
-        for (int aj = 0; aj < 4; ++aj) af[aj] = As[k][wa * 64 + aj * 16 + (lane & 15)];
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-          for (int aj = 0; aj < 4; ++aj) acc[bi][aj] = Mfma<T>::mma(bf[bi], af[aj], acc[bi][aj]);
-      }
-    };
-    for (int qc = q_lo; qc < q_hi - 1; ++qc) {
-      stage(qc);
-      fetch(qc + 1);
-      products(qc);
-      __syncthreads();
     }
-    stage(q_hi - 1);
-    // scatter offsets: column base from LDS, relative row per output (rel is
-    // defined for rows a >= the first row of b's target group: clamped,
-    // unconditional loads), issued before the last chunk's products
-    int64_t tcb[2][4];
-    int32_t relv[2][4][4];
+    if (LDL) {
+      const int kg = min(kc + (tid & (KC - 1)), Ks - 1);
+      dv = P[(int64_t)kg * ld + kg];
+    }
+    kc += KC;
+    if (kc >= Ks && q + 1 < q_hi) {  // the next chunk opens the next segment
+      ++seg;
+      kc = 0;
+      open_segment();
+    }
+  };
+  fetch(q_lo);
+  if (tid < E) {
+    sTc[tid] = tcv;
+    sTm[tid] = tmv;
+  }
+  __syncthreads();
+  // Relative rows of this lane's outputs (rel is defined for rows a >= the
+  // first row of b's target group: clamped, unconditional loads).  The
+  // 64 x 64 tile has the registers to hold them from the start and to load
+  // its targets ahead of the last chunk's products.
+  constexpr bool AHEAD = E == 64;
+  constexpr int HB = AHEAD ? BB : 1;  // 16-column blocks whose rows and targets are held at a time
+  int32_t rv[HB][4][BA];
+  auto load_rows = [&](int b0) {
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+    for (int bi = 0; bi < HB; ++bi)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int bl = wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
-        const int bc = min(tj * TB + bl, m - 1);
-        tcb[bi][v] = sTc[bl];
+        const int bl = (wb * BB + b0 + bi) * 16 + Mfma<T>::row(lane, v);
+        const int bc = min(tj * E + bl, m - 1);
         const int64_t tmb = sTm[bl];
 #pragma unroll
-        for (int aj = 0; aj < 4; ++aj) {
-          const int aoff = ti * TA + wa * 64 + aj * 16 + (lane & 15);
-          relv[bi][v][aj] = rel[tmb + min(max(aoff, bc), m - 1)];
+        for (int aj = 0; aj < BA; ++aj) {
+          const int aoff = ti * E + (wa * BA + aj) * 16 + (lane & 15);
+          rv[bi][v][aj] = rel[tmb + min(max(aoff, bc), m - 1)];
         }
       }
-    products(q_hi - 1);
-    const int bcut = t.d < 0 ? -t.d : m;  // deferred supernode: its parent's columns only
+  };
+  if (AHEAD) load_rows(0);
+  int nkk = 0;
+  // a wave wholly above the diagonal of a diagonal tile stores nothing
+  const bool idle = ti * E + (wa + 1) * (16 * BA) - 1 < tj * E + wb * (16 * BB);
+  auto stage = [&]() {
+    if (whole) {
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+      for (int i = 0; i < NQ; ++i)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int boff = tj * TB + wb * 32 + bi * 16 + Mfma<T>::row(lane, v);
+        for (int h = 0; h < NR; ++h) {
+          L.As[wave + NW * i][h * 64 + lane] = ra[i][h];
+          L.Bs[wave + NW * i][h * 64 + lane] = rb[i][h];
+        }
+    } else {
 #pragma unroll
-        for (int aj = 0; aj < 4; ++aj) {
-          const int aoff = ti * TA + wa * 64 + aj * 16 + (lane & 15);
-          if (boff < bcut && aoff < m && aoff >= boff)
-            atomic_add(arena + tcb[bi][v] + relv[bi][v][aj], -acc[bi][aj][v]);
+      for (int i = 0; i < NQ; ++i) {
+        const int k = wave + NW * i;
+#pragma unroll
+        for (int h = 0; h < NR; ++h) {
+          L.As[k][h * 64 + lane] = (k < kv && aok[h]) ? ra[i][h] : T(0);
+          L.Bs[k][h * 64 + lane] = (k < kv && bok[h]) ? rb[i][h] : T(0);
         }
       }
-    if (gi + gridDim.x < ntasks * ksplit) __syncthreads();
+    }
+    if (LDL && tid < KC) L.Dk[tid] = tid < kv ? dv : T(0);
+    nkk = idle ? 0 : (kv + 3) >> 2;
+    __syncthreads();
+  };
+  for (int q = q_lo; q < q_hi - 1; ++q) {
+    stage();
+    fetch(q + 1);
+    tile_products<T, LDL, S>(L, acc, nkk, wa, wb, lane);
+    __syncthreads();
+  }
+  stage();
+  // A tile whose columns no other workgroup of the launch writes is read and
+  // written plainly, the others use device-scope atomics: every XCD sends
+  // those past its L2 (64 x 64 tiles of unaligned targets, whole chip: 122e9
+  // entries/s, against 317e9/s for plain loads and stores).
+  const bool plain = np == 1 && min(tj * E + E, hd.bcut) <= hd.excl;
+  T cur[HB][4][BA];
+  auto target = [&](int b0, int bi, int v, int aj) {
+    return arena + sTc[(wb * BB + b0 + bi) * 16 + Mfma<T>::row(lane, v)] + rv[bi][v][aj];
+  };
+  auto load_targets = [&](int b0) {
+#pragma unroll
+    for (int bi = 0; bi < HB; ++bi)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int aj = 0; aj < BA; ++aj) cur[bi][v][aj] = *target(b0, bi, v, aj);
+  };
+  if (AHEAD && plain) load_targets(0);
+  tile_products<T, LDL, S>(L, acc, nkk, wa, wb, lane);
+#pragma unroll
+  for (int b0 = 0; b0 < BB; b0 += HB) {
+    if (!AHEAD) {
+      compiler_fence();  // keeps the loads of later blocks out of the registers
+      load_rows(b0);
+      if (plain) load_targets(b0);
+    }
+#pragma unroll
+    for (int bi = 0; bi < HB; ++bi)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int aj = 0; aj < BA; ++aj) {
+          const int boff = tj * E + (wb * BB + b0 + bi) * 16 + Mfma<T>::row(lane, v);
+          const int aoff = ti * E + (wa * BA + aj) * 16 + (lane & 15);
+          if (boff < hd.bcut && aoff < m && aoff >= boff) {
+            if (plain)
+              *target(b0, bi, v, aj) = cur[bi][v][aj] - acc[b0 + bi][aj][v];
+            else
+              atomic_add(target(b0, bi, v, aj), -acc[b0 + bi][aj][v]);
+          }
+        }
   }
 }
 
 // ---------------------------------------------------------------------------
 // Schur update with one wave per 64 x 64 output tile (the autotuner's
 // candidate without LDS staging).  The same C = -P_a P_b^T (LDL:
-// -P_a D P_b^T) as k_update<T,1,LDL>, but each wave owns a whole tile as 4 x 4
+// -P_a D P_b^T) as k_schur, but each wave owns a whole tile as 4 x 4
 // MFMA 16x16x4 blocks (16 independent accumulators: one wave keeps the
 // matrix core busy on its own) and streams its operands from memory straight
 // into registers, two k steps of 4 ahead of the products, so there is no
@@ -1306,7 +1220,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 // need no masks.  Panels are below 2 GiB (the launch checks it).
 template <typename T, bool LDL, int SHAPE, bool MERGED>
 __device__ __forceinline__ void w1_body(const SnInfo& s, const Task4& t, T* __restrict__ arena,
-                                        const int32_t* __restrict__ rel, const MergeInfo* __restrict__ merges,
+                                        const int32_t* __restrict__ rel, const SchurHead* __restrict__ heads,
+        const SchurSeg* __restrict__ segs,
                                         const int32_t* __restrict__ mmap, const int64_t* __restrict__ sTc,
                                         const int64_t* __restrict__ sTm, int g_lo, int g_hi, int ng1, int nbi,
                                         int nbj) {
@@ -1330,13 +1245,15 @@ __device__ __forceinline__ void w1_body(const SnInfo& s, const Task4& t, T* __re
   uint32_t ld2 = 1;
   uint32_t aoff2[4] = {0, 0, 0, 0}, boff2[4] = {0, 0, 0, 0};
   if (MERGED) {
-    const MergeInfo mg = merges[t.d - 1];
+    const SchurSeg mg = segs[heads[t.d].seg0 + 1];
+    const bool map = mg.moff >= 0;
     rC = make_rsrc(arena + mg.off, (uint32_t)mg.ld * (uint32_t)mg.w * TB);
     ld2 = (uint32_t)mg.ld;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int ma = mmap[mg.moff + (aoff[i] / TB - s.w)];
-      const int mb = mmap[mg.moff + (boff[i] / TB - s.w)];
+      const int a = (int)(aoff[i] / TB) - s.w, b = (int)(boff[i] / TB) - s.w;
+      const int ma = map ? mmap[mg.moff + a] : mg.shift + a;
+      const int mb = map ? mmap[mg.moff + b] : mg.shift + b;
       aoff2[i] = ma >= 0 ? (uint32_t)ma * TB : 0xffffffffu;
       boff2[i] = mb >= 0 ? (uint32_t)mb * TB : 0xffffffffu;
     }
@@ -1400,7 +1317,7 @@ __device__ __forceinline__ void w1_body(const SnInfo& s, const Task4& t, T* __re
   // scatter: bases from LDS, relative rows from rel (defined for rows a >=
   // the first row of b's target group: clamped, unconditional loads), one
   // 16-column block at a time
-  const int bcut = t.d < 0 ? -t.d : m;
+  const int bcut = heads[t.d].bcut;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     int32_t rv[4][4];
@@ -1433,7 +1350,8 @@ template <typename T, bool LDL>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, T* __restrict__ arena,
                 const int64_t* __restrict__ tcol, const int64_t* __restrict__ tmap,
-                const int32_t* __restrict__ rel, const MergeInfo* __restrict__ merges,
+                const int32_t* __restrict__ rel, const SchurHead* __restrict__ heads,
+        const SchurSeg* __restrict__ segs,
                 const int32_t* __restrict__ mmap, int64_t ntasks, int ksplit) {
   constexpr int KC = kSchurKC;
   __shared__ int64_t sTc[NT / 64][TILE], sTm[NT / 64][TILE];
@@ -1443,11 +1361,14 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
   if (gi >= ntasks * ksplit) return;  // the whole wave
   const int64_t task = gi / ksplit;
   const int part = (int)(gi - task * ksplit);
-  const Task4 t = tasks[task];
+  Task4 t = tasks[task];
   const SnInfo s = sn[t.a];
+  const SchurHead hd = heads[t.d];
+  const int np = hd.split * ksplit, p = (t.c >> kTileBits) * ksplit + part;
+  t.c &= kTileMask;
   const int K = s.w, m = s.r - s.w, ti = t.b, tj = t.c;
-  int K2 = 0;
-  if (t.d > 0) K2 = merges[t.d - 1].w;
+  const bool merged = hd.nseg > 1;
+  const int K2 = merged ? segs[hd.seg0 + 1].w : 0;
   // scatter bases of the tile's 64 output columns (wave-private LDS: the
   // wave's own LDS accesses complete in order, no barrier)
   {
@@ -1459,7 +1380,7 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
   // the k split, as in k_update
   constexpr int SPC = KC / 4;
   const int nq1 = (K + KC - 1) / KC, nq = nq1 + (K2 + KC - 1) / KC;
-  const int q_lo = (int)((int64_t)part * nq / ksplit), q_hi = (int)((int64_t)(part + 1) * nq / ksplit);
+  const int q_lo = (int)((int64_t)p * nq / np), q_hi = (int)((int64_t)(p + 1) * nq / np);
   if (q_lo >= q_hi) return;
   const int ng1 = (K + 3) / 4, ng2 = (K2 + 3) / 4;
   const int g_lo = q_lo < nq1 ? SPC * q_lo : ng1 + SPC * (q_lo - nq1);
@@ -1467,26 +1388,26 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
   // blocks of this tile that hold stored outputs
   const bool diag = ti == tj;
   const int nbi = min(4, (m - ti * TILE + 15) / 16);
-  const int bcut = t.d < 0 ? -t.d : m;
+  const int bcut = hd.bcut;
   const int nbj = min(4, (min(bcut, m) - tj * TILE + 15) / 16);
   const int64_t* c = sTc[wv];
   const int64_t* mm = sTm[wv];
   if (nbi == 4 && nbj == 4 && !diag) {
-    if (t.d > 0)
-      w1_body<T, LDL, 0, true>(s, t, arena, rel, merges, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
+    if (merged)
+      w1_body<T, LDL, 0, true>(s, t, arena, rel, heads, segs, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
     else
-      w1_body<T, LDL, 0, false>(s, t, arena, rel, merges, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
+      w1_body<T, LDL, 0, false>(s, t, arena, rel, heads, segs, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
   } else if (nbi == 4 && nbj == 4) {
-    if (t.d > 0)
-      w1_body<T, LDL, 1, true>(s, t, arena, rel, merges, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
+    if (merged)
+      w1_body<T, LDL, 1, true>(s, t, arena, rel, heads, segs, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
     else
-      w1_body<T, LDL, 1, false>(s, t, arena, rel, merges, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
+      w1_body<T, LDL, 1, false>(s, t, arena, rel, heads, segs, mmap, c, mm, g_lo, g_hi, ng1, 4, 4);
   } else {
     const int nbi_enc = diag ? -nbi : nbi;
-    if (t.d > 0)
-      w1_body<T, LDL, 2, true>(s, t, arena, rel, merges, mmap, c, mm, g_lo, g_hi, ng1, nbi_enc, nbj);
+    if (merged)
+      w1_body<T, LDL, 2, true>(s, t, arena, rel, heads, segs, mmap, c, mm, g_lo, g_hi, ng1, nbi_enc, nbj);
     else
-      w1_body<T, LDL, 2, false>(s, t, arena, rel, merges, mmap, c, mm, g_lo, g_hi, ng1, nbi_enc, nbj);
+      w1_body<T, LDL, 2, false>(s, t, arena, rel, heads, segs, mmap, c, mm, g_lo, g_hi, ng1, nbi_enc, nbj);
   }
 }
 

@@ -183,7 +183,9 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   p.upd_size = upd;
   p.rel_groups.clear();
   p.rel_size = 0;
+  std::vector<int64_t> group0(ns + 1, 0);  // first RelGroup of every supernode
   for (Int I = 0; I < ns; ++I) {
+    group0[I] = (int64_t)p.rel_groups.size();
     const SnInfo& si = p.sn[I];
     const int32_t* st = &p.lindx0[si.lx];
     int32_t m = si.r - si.w;
@@ -200,91 +202,128 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
       p.rel_size += m - gb;
     }
   }
+  group0[ns] = (int64_t)p.rel_groups.size();
 
-  // Deferred (merged) updates along supernode chains (see MergeInfo).  The
-  // parent P of C is the supernode of C's first off-diagonal row; the rows of
-  // struct(C) inside P's columns form a prefix of length n1, the remaining
-  // rows R2 all lie in struct(P).  P absorbs at most one child, and a
-  // supernode that absorbs a child is not itself deferred, so each merged
-  // update has exactly two k segments.  A child qualifies when R2 covers most
-  // of P's off-diagonal rows (the merged tiles then carry few zero rows).
-  // Merging moves work from the child's level to the parent's and lengthens
-  // the parent's tiles' k loop, which only pays where both levels have
-  // enough tiles to keep every CU busy (3 workgroups per CU x 256 CUs); near
-  // the root, where a level holds one or two supernodes, it would lengthen
-  // the critical path instead.
-  constexpr int32_t kMergeMinRows = 32;
-  constexpr double kMergeMinFill = 0.85;
-  const int64_t kMergeMinLevelTiles = merge_updates >= 2 ? 0 : 768;
-  std::vector<int64_t> level_tiles(p.nlevels, 0);
-  for (Int I = 0; I < ns; ++I) {
-    const int64_t t = ceil_div(p.sn[I].r - p.sn[I].w, kTile);
-    level_tiles[p.level[I]] += t * (t + 1) / 2;
-  }
+  // Chains (see SchurSeg).  The parent P of C is the supernode of C's first
+  // off-diagonal row; the rows of struct(C) inside P's columns form a prefix
+  // of length n1, the remaining rows r2 all lie in struct(P).  C continues
+  // its chain into P when its remaining rows cover most of P's (the chain's
+  // products then carry few zero rows: 1% of the flops on 3D nested
+  // dissection grids) and no other child of P comes near it in rows: where
+  // two separators of similar size meet, their parent's columns are outside
+  // both chains.  Members narrower than one k chunk are left out in mode 1:
+  // a segment costs a whole chunk's staging.
+  constexpr double kChainMinFill = 0.85, kChainMaxSibling = 0.5;
+  std::vector<int32_t> par(ns, -1), n1(ns, 0);
+  std::vector<int32_t> link(ns, -1), prev(ns, -1);  // next / previous member of the chain
   std::vector<int32_t> pos(n, -1);
-  p.deferred_into.assign(ns, -1);
-  std::vector<int32_t> merge_of(ns, 0);  // per supernode: 1 + index into merges, 0 = none
-  std::vector<int32_t> ncut(ns, 0);      // per deferred supernode: n1
   if (merge_updates > 0) {
-    std::vector<int32_t> par(ns, -1), n1(ns, 0);
-    std::vector<std::vector<Int>> kids(ns);
+    std::vector<int32_t> big(ns, -1), second(ns, 0);  // per parent: child with most rows, next one's rows
+    auto rows_of = [&](Int I) { return p.sn[I].r - p.sn[I].w; };
     for (Int I = 0; I < ns; ++I) {
       const SnInfo& si = p.sn[I];
       const int32_t m = si.r - si.w;
       if (m <= 0) continue;
       const int32_t* st = &p.lindx0[si.lx + si.w];
       const Int P = row_sup[st[0]];
-      const int32_t end = p.sn[P].fc + p.sn[P].w;
-      int32_t k = 0;
-      while (k < m && st[k] < end) ++k;
       par[I] = P;
-      n1[I] = k;
-      kids[P].push_back(I);
-    }
-    std::vector<char> is_merger(ns, 0);
-    std::vector<int32_t> map;
-    for (Int P = 0; P < ns; ++P) {  // children precede parents
-      const SnInfo& sp = p.sn[P];
-      const int32_t mP = sp.r - sp.w;
-      if (mP <= 0 || level_tiles[p.level[P]] < kMergeMinLevelTiles) continue;
-      Int best = -1;
-      int32_t bv = 0;
-      for (Int C : kids[P]) {
-        if (is_merger[C] || level_tiles[p.level[C]] < kMergeMinLevelTiles) continue;
-        const int32_t r2 = (p.sn[C].r - p.sn[C].w) - n1[C];
-        if (r2 >= kMergeMinRows && (double)r2 >= kMergeMinFill * mP && r2 > bv) {
-          best = C;
-          bv = r2;
-        }
+      n1[I] = (int32_t)(std::lower_bound(st, st + m, p.sn[P].fc + p.sn[P].w) - st);
+      if (big[P] < 0 || m > rows_of(big[P])) {
+        if (big[P] >= 0) second[P] = std::max(second[P], rows_of(big[P]));
+        big[P] = I;
+      } else {
+        second[P] = std::max(second[P], m);
       }
-      if (best < 0) continue;
-      const SnInfo& sc = p.sn[best];
-      const int32_t* stC = &p.lindx0[sc.lx];
-      for (int32_t q = 0; q < sc.r; ++q) pos[stC[q]] = q;
-      map.assign(mP, -1);
-      int32_t found = 0;
-      for (int32_t a = 0; a < mP; ++a) {
-        const int32_t q = pos[p.lindx0[sp.lx + sp.w + a]];
-        if (q >= sc.w) {
-          map[a] = q;
-          ++found;
-        }
-      }
-      for (int32_t q = 0; q < sc.r; ++q) pos[stC[q]] = -1;
-      if (found != bv) continue;  // R2 not inside struct(P): keep the plain update
-      MergeInfo mi{};
-      mi.off = sc.off;
-      mi.moff = (int64_t)p.mmap.size();
-      mi.ld = sc.r;
-      mi.w = sc.w;
-      mi.child = best;
-      p.mmap.insert(p.mmap.end(), map.begin(), map.end());
-      is_merger[P] = 1;
-      p.deferred_into[best] = P;
-      ncut[best] = n1[best];
-      merge_of[P] = (int32_t)p.merges.size() + 1;
-      p.merges.push_back(mi);
     }
+    for (Int P = 0; P < ns; ++P) {
+      const Int C = big[P];
+      if (C < 0) continue;
+      const int32_t mC = rows_of(C), mP = rows_of(P), r2 = mC - n1[C];
+      if (merge_updates < 2 && p.sn[C].w < kSchurKC) continue;
+      if (second[P] > kChainMaxSibling * mC || r2 < kChainMinFill * mP) continue;
+      // the remaining rows must be rows of P
+      const int32_t* c = &p.lindx0[p.sn[C].lx + p.sn[C].w] + n1[C];
+      const int32_t* q = &p.lindx0[p.sn[P].lx + p.sn[P].w];
+      if (!std::includes(q, q + mP, c, c + r2)) continue;
+      link[C] = P;
+      prev[P] = C;
+    }
+  }
+  p.chain_end.resize(ns);
+  for (Int I = ns - 1; I >= 0; --I) p.chain_end[I] = link[I] >= 0 ? p.chain_end[link[I]] : I;
+
+  // Inside a chain, a child's update beyond its parent's columns can be taken
+  // over by the parent as a second segment; a supernode that takes one over
+  // is not itself taken over.  That moves work to the parent's level and
+  // lengthens its tiles' k loop, which only pays where both levels have
+  // enough tiles to keep every CU busy (3 workgroups per CU x 256 CUs); near
+  // the root, where a level holds one or two supernodes, it would lengthen
+  // the critical path instead.
+  constexpr int32_t kMergeMinRows = 32;
+  const int64_t kMergeMinLevelTiles = merge_updates >= 2 ? 0 : 768;
+  std::vector<int64_t> level_tiles(p.nlevels, 0);
+  for (Int I = 0; I < ns; ++I) {
+    const int64_t t = ceil_div(p.sn[I].r - p.sn[I].w, kTile);
+    level_tiles[p.level[I]] += t * (t + 1) / 2;
+  }
+  p.deferred_into.assign(ns, -1);
+  std::vector<int32_t> absorbs(ns, -1);  // per supernode: the child it takes over
+  for (Int P = 0; P < ns; ++P) {  // children precede parents
+    const Int C = prev[P];
+    if (C < 0 || p.sn[P].r <= p.sn[P].w || absorbs[C] >= 0) continue;
+    if (level_tiles[p.level[P]] < kMergeMinLevelTiles || level_tiles[p.level[C]] < kMergeMinLevelTiles) continue;
+    if ((p.sn[C].r - p.sn[C].w) - n1[C] < kMergeMinRows) continue;
+    absorbs[P] = C;
+    p.deferred_into[C] = P;
+  }
+
+  // heads and their segments
+  auto add_segment = [&](Int H, Int S) {
+    const SnInfo& sh = p.sn[H];
+    const SnInfo& sg = p.sn[S];
+    const int32_t mH = sh.r - sh.w;
+    SchurSeg g{};
+    g.off = sg.off;
+    g.moff = -1;
+    g.ld = sg.r;
+    g.w = sg.w;
+    g.sn = S;
+    const int32_t* st = &p.lindx0[sg.lx];
+    const int32_t first = (int32_t)(std::lower_bound(st + sg.w, st + sg.r, sh.fc + sh.w) - st);
+    g.shift = first;  // S has exactly H's rows there, or:
+    if (sg.r - first != mH) {
+      g.moff = (int64_t)p.mmap.size();
+      for (int32_t q = first; q < sg.r; ++q) pos[st[q]] = q;
+      for (int32_t a = 0; a < mH; ++a) p.mmap.push_back(pos[p.lindx0[sh.lx + sh.w + a]]);
+      for (int32_t q = first; q < sg.r; ++q) pos[st[q]] = -1;
+    }
+    p.schur_segs.push_back(g);
+    p.schur_heads.back().nseg++;
+    p.schur_heads.back().nq += (int32_t)ceil_div(sg.w, kSchurKC);
+    p.schur_heads.back().nq16 += (int32_t)ceil_div(sg.w, 16);
+  };
+  std::vector<int32_t> head_of(ns, -1);
+  for (Int I = 0; I < ns; ++I) {
+    const SnInfo& si = p.sn[I];
+    const int32_t m = si.r - si.w;
+    if (m <= 0) continue;
+    head_of[I] = (int32_t)p.schur_heads.size();
+    SchurHead h{};
+    h.seg0 = (int32_t)p.schur_segs.size();
+    h.bcut = m;
+    if (p.deferred_into[I] >= 0) {
+      h.bcut = n1[I];
+    } else if (p.chain_end[I] != I) {
+      const SnInfo& se = p.sn[p.chain_end[I]];
+      const int32_t* st = &p.lindx0[si.lx + si.w];
+      h.bcut = (int32_t)(std::lower_bound(st, st + m, se.fc + se.w) - st);
+    }
+    p.schur_heads.push_back(h);
+    add_segment(I, I);
+    if (p.chain_end[I] == I)
+      for (Int C = prev[I]; C >= 0; C = prev[C]) add_segment(I, C);
+    else if (absorbs[I] >= 0)
+      add_segment(I, absorbs[I]);
   }
 
   amap_thread.join();
@@ -302,8 +341,24 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   // ---- factorization task lists, level by level ----
   std::vector<std::vector<Int>> by_level(p.nlevels);
   for (Int I = 0; I < ns; ++I) by_level[p.level[I]].push_back(I);
+  std::vector<int32_t> writers(ns, 0);  // per panel: supernodes of the level that update it
   for (int L = 0; L < p.nlevels; ++L) {
     const auto& sns = by_level[L];
+    auto each_target = [&](Int I, auto&& f) {
+      if (head_of[I] < 0) return;
+      const int32_t cut = p.schur_heads[head_of[I]].bcut;
+      for (int64_t g = group0[I]; g < group0[I + 1] && p.rel_groups[g].gb < cut; ++g)
+        if (!f(p.rel_groups[g])) break;
+    };
+    for (Int I : sns) each_target(I, [&](const RelGroup& g) { return ++writers[g.J], true; });
+    for (Int I : sns)
+      each_target(I, [&](const RelGroup& g) {
+        SchurHead& h = p.schur_heads[head_of[I]];
+        if (writers[g.J] != 1) return false;
+        h.excl = std::min(g.ge, h.bcut);
+        return true;
+      });
+    for (Int I : sns) each_target(I, [&](const RelGroup& g) { return writers[g.J] = 0, true; });
     const size_t level_first = p.factor_seq.size();
     int smax = 0;
     for (Int I : sns) smax = std::max<int>(smax, (int)ceil_div(p.sn[I].w, kStep));
@@ -374,39 +429,45 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     LaunchRange sr{2, p.n_schur, 0};
     sr.first_w = p.n_schur_wide;
     const size_t emit_first = p.schur_emit.size();
+    // A head with a long k loop (a chain's last member) is split into parts of
+    // at least kPartChunks chunks, so that every resident workgroup gets
+    // about four: 1,827 tiles of 60 chunks on 1,024 slots (60^3 27-point,
+    // level 36) 541 us whole, 529 us in two parts.  Shorter parts cost more
+    // in atomics than the balance gains.
+    constexpr int64_t kPartChunks = 20, kSlots = 1024;
+    int64_t units = 0;  // chunks of all tiles of the level
+    for (Int I : sns) {
+      if (head_of[I] < 0) continue;
+      const SchurHead& h = p.schur_heads[head_of[I]];
+      units += h.nq * schur_tiles_before(ceil_div(p.sn[I].r - p.sn[I].w, kTile), ceil_div(h.bcut, kTile));
+    }
+    const int64_t part_chunks = std::max(kPartChunks, units / (4 * kSlots));
     int nqmin = INT_MAX, nqmax = 0;
     for (Int I : sns) {
       const SnInfo& si = p.sn[I];
       int64_t m = si.r - si.w;
       if (m <= 0) continue;
+      SchurHead& h = p.schur_heads[head_of[I]];
+      h.split = (int32_t)std::max<int64_t>(1, h.nq / part_chunks);
       SchurEmit e{};
       e.I = I;
       e.nt = (int32_t)ceil_div(m, kTile);
+      e.ntj = (int32_t)ceil_div(h.bcut, kTile);
       e.ntw = (int32_t)ceil_div(m, 2 * kTile);
-      if (p.deferred_into[I] >= 0) {
-        // only the output columns in the parent's columns; the rest is
-        // computed by the parent's merged update
-        const int32_t n1 = ncut[I];
-        e.ntj = (int32_t)ceil_div(n1, kTile);
-        e.d = -n1;
-        p.schur_entries += (int64_t)n1 * m - (int64_t)n1 * (n1 - 1) / 2;
-      } else {
-        e.ntj = e.nt;
-        e.d = merge_of[I];
-        p.schur_entries += m * (m + 1) / 2;
-      }
+      e.ntjw = (int32_t)ceil_div(h.bcut, 2 * kTile);
+      e.head = head_of[I];
+      e.split = h.split;
+      p.schur_entries += (int64_t)h.bcut * m - (int64_t)h.bcut * (h.bcut - 1) / 2;
       e.first[0] = p.n_schur;
       e.first[2] = p.n_schur_wide;
-      p.n_schur += schur_tiles_before(e.nt, e.ntj);
-      p.n_schur_wide += schur_wide_before(e.ntw, e.ntj);
-      int nq = (int)ceil_div(si.w, kSchurKC);
-      if (e.d > 0) nq += (int)ceil_div(p.merges[e.d - 1].w, kSchurKC);
-      nqmin = std::min(nqmin, nq);
-      nqmax = std::max(nqmax, nq);
-      e.nq = nq;
+      p.n_schur += schur_tiles_before(e.nt, e.ntj) * e.split;
+      p.n_schur_wide += schur_tiles_before(e.ntw, e.ntjw);
+      nqmin = std::min(nqmin, h.nq / h.split);
+      nqmax = std::max(nqmax, h.nq);
+      sr.nsegmax = std::max(sr.nsegmax, h.nseg);
       p.schur_emit.push_back(e);
       // algorithmic flops stay those of the supernode's whole update, wherever
-      // its deferred part is computed
+      // its parts are computed
       p.schur_flops += (double)si.w * (double)m * (double)(m + 1);
     }
     sr.count = p.n_schur - sr.first;
@@ -417,20 +478,25 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     // supernode's tiles in their plan order
     {
       std::vector<int64_t> cnt(nqmax + 2, 0);
-      for (size_t q = emit_first; q < p.schur_emit.size(); ++q) ++cnt[nqmax - p.schur_emit[q].nq + 1];
+      for (size_t q = emit_first; q < p.schur_emit.size(); ++q) ++cnt[nqmax - p.schur_heads[p.schur_emit[q].head].nq + 1];
       for (int i = 1; i <= nqmax + 1; ++i) cnt[i] += cnt[i - 1];
       std::vector<size_t> order(p.schur_emit.size() - emit_first);
       for (size_t q = emit_first; q < p.schur_emit.size(); ++q)
-        order[cnt[nqmax - p.schur_emit[q].nq]++] = q;
+        order[cnt[nqmax - p.schur_heads[p.schur_emit[q].head].nq]++] = q;
       int64_t f1 = sr.first, f3 = sr.first_w;
       for (size_t q : order) {
         SchurEmit& e = p.schur_emit[q];
         e.first[1] = f1;
         e.first[3] = f3;
-        f1 += schur_tiles_before(e.nt, e.ntj);
-        f3 += schur_wide_before(e.ntw, e.ntj);
+        f1 += schur_tiles_before(e.nt, e.ntj) * e.split;
+        f3 += schur_tiles_before(e.ntw, e.ntjw);
       }
     }
+    // longest first: the same as plan order where all tasks are as long; 64 x
+    // 64 tiles: 128 x 128 ones read half the operands but fill the last round
+    // of workgroups worse (60^3 27-point, whole Schur: 8.58 against 9.95 ms;
+    // 80^3 LDL^T: 39.8 against 43.0 ms; ahead by 3% on three of its levels)
+    sr.alt = 1;
     if (sr.count && sr.count < kSplitTarget) {
       // few output tiles: each task's k chunks are split over S workgroups
       // (partial sums meet in the atomic scatter), S <= the fewest chunks of

@@ -49,18 +49,36 @@ struct Task4 {
   int32_t a, b, c, d;
 };
 
-// A child supernode C whose Schur update is split in two: the part landing in
-// its parent P's columns is applied at C's level; the rest (rows and columns
-// both in struct(P)) is deferred and computed inside P's Schur update as
-// extra k columns, so those target entries are scattered once instead of
-// twice.  mmap[moff + a] = row of C's panel holding P's off-diagonal row a
-// (-1 where C has no such row).
-struct MergeInfo {         // mirrored on the device
-  int64_t off;             // C's panel offset
-  int64_t moff;            // offset of the row map in mmap
-  int32_t ld;              // C's panel leading dimension (rows)
-  int32_t w;               // C's width (extra k columns)
-  int32_t child;           // C
+// Schur updates along chains.  A separator wider than the supernode limit is
+// a chain of supernodes, each the main child of the next, and the rows of
+// every member below the chain's columns are rows of the chain's last member
+// E.  A member applies its update at its own level only inside the chain's
+// columns; the rest is applied once for the whole chain, at E's level, as
+// one product over the columns of all members.  Each target entry outside
+// the chain is then written once per chain instead of once per member, and
+// the product runs over a long k.
+//
+// The update that a supernode H computes at its level (its "head") is
+//   C(a,b) = sum over its segments of  S(a,:) S(b,:)^T   (LDL: S D S^T)
+// for H's off-diagonal rows a >= b, b < bcut.  Segment 0 is H itself; a row
+// a of H is row shift + a of the segment's panel, or mmap[moff + a] where
+// moff >= 0 (-1: the segment has no such row).
+struct SchurSeg {          // mirrored on the device
+  int64_t off;             // panel offset of the segment's supernode
+  int64_t moff;            // offset of the row map in mmap, -1: shift
+  int32_t ld;              // its panel's leading dimension (rows)
+  int32_t w;               // its width (k columns)
+  int32_t shift;
+  int32_t sn;
+};
+struct SchurHead {         // mirrored on the device; one per supernode with an update
+  int32_t seg0, nseg;      // segments [seg0, seg0 + nseg)
+  int32_t bcut;            // output columns (off-diagonal rows b) below bcut only
+  int32_t nq, nq16;        // k chunks of kSchurKC / of 16 columns over all segments
+  // output columns below excl lie in panels that no other supernode of the
+  // same etree level (the same launch) updates: no atomics needed there
+  int32_t excl;
+  int32_t split;           // k parts of its 64 x 64 tiles, tasks of their own
   int32_t pad;
 };
 
@@ -83,27 +101,25 @@ struct RelGroup {          // mirrored on the device
 #define SPK_HD
 #endif
 
-// Schur output tiles of one supernode with m off-diagonal rows: 64 x 64
-// tiles (ti, tj), tj <= ti, tj < ntj (ntj = the column-tile count, fewer for
-// a deferred supernode's column cut), in order ti then tj; 128 x 64 tiles
-// (ti, tj), ti < ceil(m / 128), tj <= 2 ti + 1, tj < ntj.  *_before(ti, ntj):
-// tiles of the rows before row tile ti.
+// Schur output tiles (ti, tj), tj <= ti, tj < ntj, of one supernode (ntj =
+// the column-tile count, fewer than the row tiles where the head's columns
+// are cut): those of the row tiles before ti.
 SPK_HD inline int64_t schur_tiles_before(int64_t ti, int64_t ntj) {
   return ti <= ntj ? ti * (ti + 1) / 2 : ntj * (ntj + 1) / 2 + (ti - ntj) * ntj;
 }
-SPK_HD inline int64_t schur_wide_before(int64_t ti, int64_t ntj) {
-  const int64_t c = ntj / 2;  // row tiles whose 2 ti + 2 columns all lie below the cap
-  return ti <= c ? ti * (ti + 1) : c * (c + 1) + (ti - c) * ntj;
-}
 
-// Per supernode with a Schur update: where its tasks {sn, ti, tj, d} go in
+// A Schur task is {sn, ti, tj | part << kTileBits, head}.
+constexpr int kTileBits = 20, kTileMask = (1 << kTileBits) - 1;
+
+// Per supernode with a Schur update: where its tasks go in
 // the four Schur task arrays (64 x 64 tiles in plan order and longest first,
-// 128 x 64 tiles in plan order and longest first).  nt = ceil(m / 64) row
-// tiles, ntw = ceil(m / 128).
+// 128 x 128 tiles in plan order and longest first); nt x ntj and ntw x ntjw
+// row x column tiles.
 struct SchurEmit {         // mirrored on the device
   int64_t first[4];
-  int32_t I, nt, ntw, ntj;
-  int32_t d, nq, pad1, pad2;  // nq: k chunks of each task (panel and merged child)
+  int32_t I, nt, ntj, ntw;
+  int32_t ntjw, head;      // head: index of its SchurHead (the tasks' d)
+  int32_t split, pad;      // as in the SchurHead
 };
 
 struct LaunchRange {
@@ -116,10 +132,11 @@ struct LaunchRange {
   int aux = 0;       // kinds 0, 7, 9, 3, 6: diagonal-block bucket (diag_bucket);
                      // kind 2: k-chunk split factor (0 or 1 = none)
   int level = 0;     // etree level of the launch (factor sequence)
-  int alt = 0;       // kind 2: bit 0 = tasks in longest-first order, bit 1 = 128 x 64
-                     // tiles (k_schur_wide), bit 2 = one wave per 64 x 64 tile (k_schur_w1)
-  int64_t first_w = 0, count_w = 0;  // kind 2: the level's 128 x 64 tile tasks
+  int alt = 0;       // kind 2: bit 0 = tasks in longest-first order, bit 1 = 128 x 128
+                     // tiles, bit 2 = one wave per 64 x 64 tile (k_schur_w1)
+  int64_t first_w = 0, count_w = 0;  // kind 2: the level's 128 x 128 tile tasks
   int nqmin = 0;     // kind 2: fewest k chunks of any task of the range
+  int nsegmax = 0;   // kind 2: most segments of any task of the range
 };
 
 struct Plan {
@@ -145,19 +162,21 @@ struct Plan {
   std::vector<int64_t> inv_base;   // per supernode: first inverse tile (tile t of 16-column block t)
   std::vector<Task4> inpanel_tasks;// {sn, step, ti, tj}
   std::vector<Task4> fused_tasks;  // {sn, row tiles, row_tile, inverse-tile offset}: block factor + TRSM
-  // Schur tasks {sn, ti, tj, d}: 64x64 output tiles; d = 0 plain, d > 0 the
-  // update also carries merges[d-1] (a deferred child), d < 0 only output
-  // columns b < -d (parent columns of a deferred supernode).  Four arrays,
+  // Schur tasks: 64x64 output tiles (and k parts).  Four arrays,
   // written on the device from schur_emit: 64 x 64 tiles in plan order; the
   // same with every launch range's supernodes ordered by their k chunks,
-  // longest first (stable: an alternative task order for the autotuner,
-  // workgroups are dispatched in index order); 128 x 64 tiles {sn, 128-row
-  // tile, 64-column tile, d} in plan order and longest first.
+  // longest first (stable; workgroups are dispatched in index order);
+  // 128 x 128 tiles in plan order and longest first.
   int64_t n_schur = 0, n_schur_wide = 0;
   std::vector<SchurEmit> schur_emit;
-  std::vector<MergeInfo> merges;
+  std::vector<SchurHead> schur_heads;
+  std::vector<SchurSeg> schur_segs;
   std::vector<int32_t> mmap;
-  std::vector<int32_t> deferred_into;  // per supernode: parent absorbing its update, -1 = none
+  std::vector<int32_t> chain_end;      // per supernode: last member of its chain (itself: a chain of one)
+  // per supernode: the parent (in the same chain) that takes over its update
+  // beyond the parent's columns, -1 = none.  The parent has it as a second
+  // segment; beyond the chain's columns the chain's last member has both.
+  std::vector<int32_t> deferred_into;
   std::vector<LaunchRange> factor_seq;
   // solve
   std::vector<Task4> sdiag_tasks;  // {sn, 0, 0, 0}: diagonal-block solves
@@ -188,9 +207,11 @@ struct Plan {
 };
 
 // Build the plan from the symbolic analysis and the caller's CSC pattern
-// (lower triangle, any base).  merge_updates: 0 no merged updates, 1 merge
-// qualifying chain children on levels with enough tiles to fill the GPU,
-// 2 merge every qualifying chain child.
+// (lower triangle, any base).  merge_updates: 0 every supernode applies its
+// whole update at its own level; 1 chains of supernodes at least kSchurKC
+// wide, and inside a chain a child's update taken over by its parent where
+// both levels have enough tiles to fill the GPU; 2 both wherever the
+// structure allows.
 void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, int baseval,
                 Plan& p, int merge_updates = 1);
 

@@ -96,7 +96,7 @@ class symPACKOptions:
         # factorization (structures with >= 1e9 Schur flops)
         self.autotune = autotune
         # Schur-update kernel on every level: 0 autotuner / plan, 1 64 x 64 tiles staged
-        # through LDS, 2 128 x 64 tiles, 3 64 x 64 tiles with one wave per tile
+        # through LDS, 2 128 x 128 tiles, 3 64 x 64 tiles with one wave per tile
         self.schur_kernel = schur_kernel
 
     @classmethod
@@ -339,7 +339,7 @@ class symPACKMatrix2D:
 
     def autotune_log(self, max_records=4096):
         """The autotuner's record per Schur launch: dicts with level, split,
-        order (bit 0: longest first instead of plan order, bit 1: 128 x 64
+        order (bit 0: longest first instead of plan order, bit 1: 128 x 128
         output tiles, bit 2: 64 x 64 tiles with one wave per tile), ms_default
         and ms_best."""
         lv, sp_, od = (np.zeros(max_records, np.int32) for _ in range(3))
@@ -430,10 +430,30 @@ class symPACKMatrix2D:
 
     def GetUpdateMerges(self):
         """deferred_into[I] (0-based): the parent that computes supernode I's
-        update outside the parent's columns, -1 where I scatters all of it."""
+        update outside the parent's columns (beyond their chain's columns:
+        together with the chain's last member), -1 for none."""
         d = np.zeros(self.TotalSupernodeCnt(), np.int32)
         _lib.check(self._lib.spk_get_update_merges(self._h, _ptr(d, ctypes.c_int32)), "merges")
         return d
+
+    def GetUpdateSchedule(self):
+        """Per supernode (0-based) the Schur update applied at its level: the
+        number of contributing supernodes, the cut of its output columns and
+        the part of them in panels that no other supernode of the level
+        updates."""
+        a = [np.zeros(self.TotalSupernodeCnt(), np.int32) for _ in range(3)]
+        _lib.check(self._lib.spk_get_update_schedule(self._h, *[_ptr(x, ctypes.c_int32) for x in a]), "schedule")
+        return a
+
+    def GetUpdateSegment(self, I, s, m):
+        """Contributor s of supernode I's update: (supernode, its panel row
+        per off-diagonal row of I, -1 where it has none); m = number of
+        off-diagonal rows of I."""
+        sn = ctypes.c_int32()
+        rows = np.zeros(m, np.int32)
+        _lib.check(self._lib.spk_get_update_segment(self._h, I, s, ctypes.byref(sn), _ptr(rows, ctypes.c_int32)),
+                   "segment")
+        return sn.value, rows
 
     def ValidateSolvePlan(self):
         """Raise if the dependency-driven solve's task lists are inconsistent."""
