@@ -1196,22 +1196,29 @@ void Engine::ginv_sequence(T* Y, T* X, T* Xf, int nrhs) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nblk, (kGinvGrid + tiles - 1) / tiles));
   };
   for (const LaunchRange& r : plan_.gfwd_seq) {
-    const dim3 grid((unsigned)r.count, grid_y(r.count));
+    // narrow supernodes on a level with many tiles keep 64 rows per
+    // workgroup: little of the time is latency there, and four times the
+    // workgroups cost more to start (60^3 27-point, level 0, 6,931 tiles of
+    // at most 32 columns: 45 against 60 us)
+    const bool rows64 = r.aux <= 2 && r.count > kGinvFew;
+    const int64_t wgs = rows64 ? r.count : 4 * r.count;
+    const dim3 grid((unsigned)wgs, grid_y(wgs));
     const Task4* t = tiles + r.first;
     launch_begin(10, r.count, nullptr, r.level);
-#define SPK_GF(NBM)                                                                                        \
-  case NBM:                                                                                                \
-    if (ldl)                                                                                               \
-      dev::k_gsolve_fwd<T, true, NBM><<<grid, 256, 0, stream_>>>(sn, t, G, arena, d_lindx0_, Y, Xf, nrhs); \
-    else                                                                                                   \
-      dev::k_gsolve_fwd<T, false, NBM><<<grid, 256, 0, stream_>>>(sn, t, G, arena, d_lindx0_, Y, Xf, nrhs); \
-    break;
-    switch (r.aux) {
-      SPK_GF(1)
-      SPK_GF(2)
-      SPK_GF(4)
-      SPK_GF(6)
-      SPK_GF(10)
+#define SPK_GF(KERNEL, NBM)                                                                           \
+  if (ldl)                                                                                            \
+    dev::KERNEL<T, true, NBM><<<grid, 256, 0, stream_>>>(sn, t, G, arena, d_lindx0_, Y, Xf, nrhs);    \
+  else                                                                                                \
+    dev::KERNEL<T, false, NBM><<<grid, 256, 0, stream_>>>(sn, t, G, arena, d_lindx0_, Y, Xf, nrhs);   \
+  break;
+    switch (rows64 ? -r.aux : r.aux) {
+      case -1: SPK_GF(k_gsolve_fwd, 1)
+      case -2: SPK_GF(k_gsolve_fwd, 2)
+      case 1: SPK_GF(k_gsolve_fwd4, 1)
+      case 2: SPK_GF(k_gsolve_fwd4, 2)
+      case 4: SPK_GF(k_gsolve_fwd4, 4)
+      case 6: SPK_GF(k_gsolve_fwd4, 6)
+      case 10: SPK_GF(k_gsolve_fwd4, 10)
       default:
         throw std::logic_error("bad diagonal-block bucket");
     }
@@ -1219,17 +1226,10 @@ void Engine::ginv_sequence(T* Y, T* X, T* Xf, int nrhs) {
     launch_end(10);
   }
   for (const LaunchRange& r : plan_.gbwd_seq) {
-    const dim3 grid((unsigned)r.count, grid_y(r.count));
-    const Task4* t = tiles + r.first;
+    const unsigned gz = (unsigned)((r.aux + 3) / 4);  // four 16-column blocks per workgroup
+    const dim3 grid((unsigned)r.count, grid_y(r.count * gz), gz);
     launch_begin(11, r.count, nullptr, r.level);
-    switch (r.aux) {
-      case 1: dev::k_gsolve_bwd<T, 1><<<grid, 256, 0, stream_>>>(sn, t, G, d_lindx0_, Xf, X, nrhs); break;
-      case 2: dev::k_gsolve_bwd<T, 2><<<grid, 256, 0, stream_>>>(sn, t, G, d_lindx0_, Xf, X, nrhs); break;
-      case 4: dev::k_gsolve_bwd<T, 4><<<grid, 256, 0, stream_>>>(sn, t, G, d_lindx0_, Xf, X, nrhs); break;
-      case 6: dev::k_gsolve_bwd<T, 6><<<grid, 256, 0, stream_>>>(sn, t, G, d_lindx0_, Xf, X, nrhs); break;
-      case 10: dev::k_gsolve_bwd<T, 10><<<grid, 256, 0, stream_>>>(sn, t, G, d_lindx0_, Xf, X, nrhs); break;
-      default: throw std::logic_error("bad diagonal-block bucket");
-    }
+    dev::k_gsolve_bwd<T><<<grid, 256, 0, stream_>>>(sn, tiles + r.first, G, d_lindx0_, Xf, X, nrhs);
     launch_end(11);
   }
   HIP_OK(hipGetLastError());

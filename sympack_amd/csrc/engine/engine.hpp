@@ -18,6 +18,9 @@ constexpr int kGmresRestart = 20;  // GMRES restart length of the LDL^T refineme
 // partitioned-inverse sweeps: workgroups a level launch aims at before it
 // splits its right-hand-side blocks over the grid
 constexpr int64_t kGinvGrid = 1024;
+// a level of supernodes at most 32 wide takes k_gsolve_fwd (64 rows per
+// workgroup) above this many 64-row tiles, k_gsolve_fwd4 otherwise
+constexpr int64_t kGinvFew = 256;
 // Size of the per-device array behind Engine::solve_noalloc: Y, X and Xf,
 // 3 n nrhs doubles, at most 128 MiB (n nrhs <= 5592405).
 constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;

@@ -2088,40 +2088,102 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd(const SnInfo* __restrict__ sn
   }
 }
 
+// Forward level, 16 rows per workgroup, the k columns spread over its four
+// waves (4 NBM each), partial sums through LDS.  A launch is bound by one
+// chain of latencies (task, supernode, operands, products, stores), on which
+// k_gsolve_fwd puts 40 operand loads and 38 dependent products of a
+// 160-column supernode and this kernel 10 (one supernode, 150 columns: 10.3
+// -> 6.7 us with events, of which an empty launch takes 4-5); in 84 registers
+// rather than 304 it also leaves room for more workgroups where a level has
+// hundreds of tiles (48^3, 600 tiles: 27 -> 19 us).  Task as k_gsolve_fwd's;
+// workgroup 4 t + q takes rows 16 q .. of task t's tile.
+template <typename T, bool LDL, int NBM>
+__global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+                                                    const T* __restrict__ garena, const T* __restrict__ arena,
+                                                    const int32_t* __restrict__ lindx0, T* Y, T* __restrict__ Xf,
+                                                    int nrhs) {
+  typedef typename Mfma<T>::v4 v4;
+  __shared__ T part[4][4][64];
+  const Task4 t = tasks[blockIdx.x >> 2];
+  const SnInfo s = sn[t.a];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int a0 = t.b * TILE + 16 * (int)(blockIdx.x & 3);
+  if (a0 >= s.r) return;  // the whole workgroup
+  const int w = s.w, k0 = 4 * NBM * wave;
+  const int64_t ld = s.r;
+  const int mi = lane & 15, g = lane >> 4;
+  const T* __restrict__ Ga = garena + s.off + min(a0 + mi, s.r - 1);
+  T av[NBM];
+#pragma unroll
+  for (int q = 0; q < NBM; ++q) {
+    const int k = k0 + 4 * q + g;
+    av[q] = Ga[(int64_t)min(k, w - 1) * ld];
+  }
+  // after the reduction this wave holds output slot `wave` of every lane
+  const int a = a0 + Mfma<T>::row(lane, wave);
+  const int orow = (a >= w && a < s.r) ? lindx0[s.lx + min(a, s.r - 1)] : -1;
+  T dinv = T(1);
+  if (LDL && a < w) dinv = T(1) / arena[s.off + (int64_t)a * ld + a];
+  const int nblk = (nrhs + SUB - 1) / SUB;
+  for (int jb = blockIdx.y; jb < nblk; jb += gridDim.y) {
+    const int jn = jb * SUB + mi;
+    const int jc = min(jn, nrhs - 1);
+    const T* __restrict__ Yk = Y + (int64_t)s.fc * nrhs + jc;
+    T bv[NBM];
+#pragma unroll
+    for (int q = 0; q < NBM; ++q) bv[q] = Yk[(int64_t)min(k0 + 4 * q + g, w - 1) * nrhs];
+#pragma unroll
+    for (int q = 0; q < NBM; ++q) keep(bv[q]);
+    v4 acc = v4{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < NBM; ++q) {
+      const int k = k0 + 4 * q + g;
+      if (k0 + 4 * q < w)  // uniform: chunks wholly beyond w are skipped
+        acc = Mfma<T>::mma(k < w ? av[q] : T(0), jn < nrhs && k < w ? bv[q] : T(0), acc);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) part[wave][v][lane] = acc[v];
+    __syncthreads();
+    const T x = (part[0][wave][lane] + part[1][wave][lane]) + (part[2][wave][lane] + part[3][wave][lane]);
+    if (jn < nrhs) {
+      if (a < w)
+        Xf[(int64_t)(s.fc + a) * nrhs + jn] = LDL ? x * dinv : x;
+      else if (orow >= 0)
+        atomic_add(Y + (int64_t)orow * nrhs + jn, -x);
+    }
+    __syncthreads();
+  }
+}
+
 // Backward level: X_I += G_I(tile rows, :)^T V(tile rows), V(a) = Xf(a) on
 // the diagonal rows and -X(struct row a) below (the ancestors' final
-// values).  Lane (m, g) reads rows 16g..16g+15 of one G column (a cache
-// line), wave q the 16-column blocks q, q+4, q+8; the G values stay in
-// registers while the workgroup walks its right-hand-side blocks (as in the
-// forward level); every load of a block is issued before its first product;
-// partial sums of the tile go to X_I with atomics (X zeroed before the
-// sweep).
-template <typename T, int NBM>
+// values).  Each wave takes one 16-column block, blockIdx.z four of them (a
+// latency chain as in the forward level: one block's loads and products per
+// wave rather than three, 10.0 -> 7.0 us for a 150-column supernode).  Lane
+// (m, g) reads rows 16g..16g+15 of one G column (a cache line); the G values
+// stay in registers while the workgroup walks its right-hand-side blocks;
+// every load of a block is issued before its first product; partial sums of
+// the tile go to X_I with atomics (X zeroed before the sweep).
+template <typename T>
 __global__ __launch_bounds__(NT) void k_gsolve_bwd(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
                                                    const T* __restrict__ garena,
                                                    const int32_t* __restrict__ lindx0, const T* __restrict__ Xf,
                                                    T* X, int nrhs) {
   typedef typename Mfma<T>::v4 v4;
-  constexpr int MKB = (NBM + 3) / 4;  // column blocks per wave
   const Task4 t = tasks[blockIdx.x];
   const SnInfo s = sn[t.a];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, kb = 4 * blockIdx.z + (threadIdx.x >> 6);
   const int w = s.w;
-  const int nkb = (w + 15) >> 4;
-  if (wave >= nkb) return;
+  if (16 * kb >= w) return;  // no barrier follows
   const int a0 = t.b * TILE;
   const int mi = lane & 15, g = lane >> 4;
   int rowi[16];
 #pragma unroll
   for (int st = 0; st < 16; ++st) rowi[st] = lindx0[s.lx + min(a0 + 16 * g + st, s.r - 1)];
-  T av[MKB][16];
+  T av[16];
+  const T* __restrict__ Gc = garena + s.off + (int64_t)min(16 * kb + mi, w - 1) * s.r;
 #pragma unroll
-  for (int i = 0; i < MKB; ++i) {
-    const int kcol = min((wave + 4 * i) * 16 + mi, w - 1);
-    const T* __restrict__ Gc = garena + s.off + (int64_t)kcol * s.r;
-#pragma unroll
-    for (int st = 0; st < 16; ++st) av[i][st] = Gc[min(a0 + 16 * g + st, s.r - 1)];
-  }
+  for (int st = 0; st < 16; ++st) av[st] = Gc[min(a0 + 16 * g + st, s.r - 1)];
   const int nblk = (nrhs + SUB - 1) / SUB;
   for (int jb = blockIdx.y; jb < nblk; jb += gridDim.y) {
     const int jn = jb * SUB + mi;
@@ -2137,20 +2199,14 @@ __global__ __launch_bounds__(NT) void k_gsolve_bwd(const SnInfo* __restrict__ sn
     }
 #pragma unroll
     for (int st = 0; st < 16; ++st) keep(bv[st]);
+    v4 acc = v4{0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < MKB; ++i) {
-      const int kb = wave + 4 * i;
-      if (kb < nkb) {
-        v4 acc = v4{0, 0, 0, 0};
+    for (int st = 0; st < 16; ++st) acc = Mfma<T>::mma(av[st], bv[st], acc);
+    if (jn < nrhs) {
 #pragma unroll
-        for (int st = 0; st < 16; ++st) acc = Mfma<T>::mma(av[i][st], bv[st], acc);
-        if (jn < nrhs) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int k = kb * 16 + Mfma<T>::row(lane, v);
-            if (k < w) atomic_add(X + (int64_t)(s.fc + k) * nrhs + jn, acc[v]);
-          }
-        }
+      for (int v = 0; v < 4; ++v) {
+        const int k = kb * 16 + Mfma<T>::row(lane, v);
+        if (k < w) atomic_add(X + (int64_t)(s.fc + k) * nrhs + jn, acc[v]);
       }
     }
   }
