@@ -77,12 +77,12 @@ typedef struct spk_options {
                          10*ordflag + altflag: 10, 11, 20, 21, 30, 31 for SET10 .. SET31
                          (SET = 31), 40 = TSPB (traveling-salesman tour with skeleton
                          compression), 41 = any other TSPB* name (tour without it) */
-  int solve_inverse;  /* 1 (default): where every supernode is at most 160 columns wide, the
-                         solve uses the partitioned inverse G_I = [I; L_off] L_II^{-1} of each
-                         supernode (prepared once per factorization), one launch per etree level
-                         and sweep; for LL^T and for the FP32 factor under refinement, not for
-                         FP64 static LDL^T (explicit inverses of its indefinite diagonal blocks
-                         lose accuracy).  0: block substitution, four launches per level */
+  int solve_inverse;  /* 1 (default): the solve uses the partitioned inverse G = [I; L_off] L_diag^{-1}
+                         of each panel of at most 160 columns of a supernode (prepared once per
+                         factorization), one launch per level of panels and sweep; for LL^T and
+                         for the FP32 factor under refinement, not for FP64 static LDL^T (explicit
+                         inverses of its indefinite diagonal blocks lose accuracy).  0: block
+                         substitution, four launches per level */
   int autotune;       /* 1: the first spk_factorize of a structure with at least 1e9
                          Schur-update flops times every etree level's Schur launch under each
                          kernel (64 x 64 or 128 x 128 tiles staged through LDS, 64 x 64 tiles
@@ -156,7 +156,8 @@ int spk_get_launch_levels(spk_handle h, int32_t* levels, int max);
 int spk_get_autotune(spk_handle h, int32_t* level, int32_t* split, int32_t* order, double* ms_default,
                      double* ms_best, int max);
 /* Etree level of every supernode (0-based supernode index, 0 = leaves): the
- * level whose launches factor it and solve with it.  No reference
+ * level whose launches factor it and (where no supernode is wider than 160
+ * columns) solve with it.  No reference
  * counterpart (the reference schedules tasks, not levels). */
 int spk_get_supernode_levels(spk_handle h, int32_t* level /* nsuper */);
 

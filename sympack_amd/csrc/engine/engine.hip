@@ -306,6 +306,7 @@ void Engine::free_device() {
   if (stream_) (void)hipStreamSynchronize(stream_);
   destroy_graphs();
   dfree(d_sn_);
+  dfree(d_panels_);
   dfree(d_lindx0_);
   dfree(d_tcol_);
   dfree(d_tmap_);
@@ -342,6 +343,7 @@ void Engine::free_device() {
   dfree(d_dinv_);
   dfree(d_garena_);
   ginv_ready_ = false;
+  ginv_fits_ = true;
   dfree(d_Y_);
   dfree(d_X_);
   dfree(d_Xf_);
@@ -371,13 +373,13 @@ int64_t Engine::device_bytes(int nrhs) const {
   int64_t b = vb(p.sn) + vb(p.lindx0) + p.upd_size * 16 + p.rel_size * 4 + vb(p.schur_heads) + vb(p.schur_segs) + vb(p.mmap) + vb(p.amap) + vb(p.perm0) +
               vb(p.potrf_tasks) + vb(p.trsm_tasks) + vb(p.inpanel_tasks) +
               2 * (p.n_schur + p.n_schur_wide) * (int64_t)sizeof(Task4) + vb(p.fused_tasks) +
-              vb(p.sdiag_tasks) + vb(p.soffm_tasks);
+              vb(p.sdiag_tasks) + vb(p.soffm_tasks) + vb(p.panels);
   b += (int64_t)(n_ + 1) * 8 + nnzA_ * (4 + 4 + 8) + (int64_t)n_ * 8;  // CSC, values, scaling
   b += (int64_t)n_ * 4 + 4;                                            // invp0, pivot flag
   if (!p.fused_tasks.empty()) b += (int64_t)p.nsuper * 4;               // fused-factor load counters
   const int64_t elem = opt_.precision == 0 ? 8 : 4;
   b += p.arena_elems * elem + std::max<int64_t>(1, p.inv_tiles) * kSub * kSub * 8;
-  if (p.ginv_ok && opt_.solve_inverse) b += p.arena_elems * elem + vb(p.gtiles);  // G and its tiles
+  if (opt_.solve_inverse) b += p.arena_elems * elem + vb(p.gtiles);  // G and its tiles
   if (opt_.precision == 1)  // full CSR of A (row pointers, columns, sources, values), at most 2 nnz
     b += (int64_t)(n_ + 1) * 8 + 2 * nnzA_ * (4 + 8 + 8);
   b += 2 * (int64_t)std::max(1, nrhs) * kRedBlocks * 8;
@@ -428,6 +430,7 @@ void Engine::ensure_device() {
   for (Int c = 0; c < n_; ++c)
     for (int64_t p = h_colptr_[c]; p < h_colptr_[c + 1]; ++p) colidx[p] = c;
   d_sn_ = dupload(plan_.sn, s);
+  d_panels_ = dupload(plan_.panels, s);
   d_lindx0_ = dupload(plan_.lindx0, s);
   {
     // scatter bases and relative indices of the Schur scatter, built on the
@@ -555,10 +558,17 @@ void Engine::ensure_device() {
   // inverted 16x16 diagonal tiles (double-sized so both precisions fit)
   d_dinv_ = dalloc<double>(std::max<int64_t>(1, plan_.inv_tiles) * kSub * kSub);
   if (use_ginv()) {
-    if (opt_.precision == 0)
-      d_garena_ = dalloc<double>(plan_.arena_elems);
-    else
-      d_garena_ = dalloc<float>(plan_.arena_elems);
+    // a second arena; where it does not fit beside one of supernodes wider
+    // than a panel (whose fill can take most of the memory), the solve
+    // substitutes
+    const size_t bytes = (size_t)std::max<int64_t>(1, plan_.arena_elems) * (opt_.precision == 0 ? 8 : 4);
+    const hipError_t e = hipMalloc(&d_garena_, bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      d_garena_ = nullptr;
+      if (e != hipErrorOutOfMemory || plan_.max_w <= kStep) HIP_OK(e);
+      ginv_fits_ = false;
+    }
   }
   ginv_ready_ = false;
   HIP_OK(hipStreamSynchronize(s));
@@ -1094,7 +1104,7 @@ void Engine::ensure_solve_capacity(int nrhs) {
 
 template <typename T, bool BWD>
 void Engine::launch_sdiag(int bucket, unsigned g, const Task4* t, const T* arena, const T* Y, T* X, int nrhs) {
-  const SnInfo* sn = (const SnInfo*)d_sn_;
+  const SolvePanel* sn = d_panels_;
   const T* dinv = (const T*)d_dinv_;
   if (nrhs <= 16) {
     // one right-hand-side group: blocks spread over the waves
@@ -1123,7 +1133,7 @@ void Engine::launch_sdiag(int bucket, unsigned g, const Task4* t, const T* arena
 // launch, (LDL) the D^{-1} scaling, one persistent backward launch.
 template <typename T>
 void Engine::solve_sequence_df(const T* arena, T* Y, T* X, int nrhs) {
-  const SnInfo* sn = (const SnInfo*)d_sn_;
+  const SolvePanel* sn = d_panels_;
   const int ns = plan_.nsuper;
   dev::DfState st;
   st.head = d_df_state_;
@@ -1155,7 +1165,7 @@ void Engine::solve_sequence_df(const T* arena, T* Y, T* X, int nrhs) {
 template <typename T>
 void Engine::ensure_ginv(const T* arena) {
   if (!use_ginv() || ginv_ready_) return;
-  const SnInfo* sn = (const SnInfo*)d_sn_;
+  const SolvePanel* sn = d_panels_;
   const Task4* tiles = (const Task4*)d_tasks_[TA_GINV];
   T* G = (T*)d_garena_;
   const T* dinv = (const T*)d_dinv_;
@@ -1181,7 +1191,7 @@ void Engine::ensure_ginv(const T* arena) {
 // level (partial sums into X).
 template <typename T>
 void Engine::ginv_sequence(T* Y, T* X, T* Xf, int nrhs) {
-  const SnInfo* sn = (const SnInfo*)d_sn_;
+  const SolvePanel* sn = d_panels_;
   const Task4* tiles = (const Task4*)d_tasks_[TA_GINV];
   const T* G = (const T*)d_garena_;
   const T* arena = opt_.precision == 0 ? (const T*)(void*)d_arena64_ : (const T*)(void*)d_arena32_;
@@ -1246,7 +1256,7 @@ void Engine::solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf) {
     solve_sequence_df<T>(arena, Y, X, nrhs);
     return;
   }
-  const SnInfo* sn = (const SnInfo*)d_sn_;
+  const SolvePanel* sn = d_panels_;
   const bool ldl = opt_.ldl != 0;
   const Task4* sd = (const Task4*)d_tasks_[TA_SDIAG];
   const Task4* sm = (const Task4*)d_tasks_[TA_SOFFM];
@@ -1254,12 +1264,7 @@ void Engine::solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf) {
     const unsigned g = (unsigned)r.count;
     launch_begin(r.kind, r.count, nullptr, r.level);
     if (r.kind == 3) {
-      if (r.aux > 0)
-        launch_sdiag<T, false>(r.aux, g, sd + r.first, arena, Y, X, nrhs);
-      else if (ldl)
-        dev::k_sdiag_fwd<T, true><<<g, 256, 0, stream_>>>(sn, sd + r.first, arena, Y, X, nrhs);
-      else
-        dev::k_sdiag_fwd<T, false><<<g, 256, 0, stream_>>>(sn, sd + r.first, arena, Y, X, nrhs);
+      launch_sdiag<T, false>(r.aux, g, sd + r.first, arena, Y, X, nrhs);
     } else {
       const dim3 grid((unsigned)r.count, (unsigned)((nrhs + 15) / 16));
       dev::k_soffm_fwd<T><<<grid, 256, 0, stream_>>>(sn, sm + r.first, arena, d_lindx0_, X, Y, nrhs);
@@ -1268,7 +1273,7 @@ void Engine::solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf) {
   }
   if (ldl) {
     launch_begin(3);
-    dev::k_scale_d<T><<<(unsigned)plan_.nsuper, 256, 0, stream_>>>(sn, sd, arena, X, nrhs);
+    dev::k_scale_d<T><<<(unsigned)plan_.panels.size(), 256, 0, stream_>>>(sn, sd, arena, X, nrhs);
     launch_end(3);
   }
   for (const LaunchRange& r : plan_.bwd_seq) {
@@ -1278,12 +1283,7 @@ void Engine::solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf) {
       const dim3 grid((unsigned)r.count, (unsigned)((nrhs + 15) / 16));
       dev::k_soffm_bwd<T><<<grid, 256, 0, stream_>>>(sn, sm + r.first, arena, d_lindx0_, X, nrhs);
     } else {
-      if (r.aux > 0)
-        launch_sdiag<T, true>(r.aux, g, sd + r.first, arena, X, X, nrhs);
-      else if (ldl)
-        dev::k_sdiag_bwd<T, true><<<g, 256, 0, stream_>>>(sn, sd + r.first, arena, X, nrhs);
-      else
-        dev::k_sdiag_bwd<T, false><<<g, 256, 0, stream_>>>(sn, sd + r.first, arena, X, nrhs);
+      launch_sdiag<T, true>(r.aux, g, sd + r.first, arena, X, X, nrhs);
     }
     launch_end(r.kind);
   }

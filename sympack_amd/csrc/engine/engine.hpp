@@ -39,7 +39,7 @@ struct EngineOptions {
   int verbose = 0;
   int merge_updates = 1;  // 0 off, 1 chains of wide supernodes, 2 every chain (see build_plan)
   int solve_dataflow = 0; // dependency-driven solve sweeps: disabled, requesting it is an error
-  int solve_inverse = 1;  // partitioned-inverse solve where every supernode is <= kStep wide
+  int solve_inverse = 1;  // partitioned-inverse solve (see use_ginv)
   int refine = 0;         // 10*ordflag + altflag of the supernode reordering, 0 = none
   int autotune = 1;       // time the Schur launch configurations of every level on the first
                           // factorization of a plan with at least kAutotuneMinFlops Schur flops
@@ -160,7 +160,7 @@ class Engine {
   void solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf = nullptr);
   template <typename T>
   void ginv_sequence(T* Y, T* X, T* Xf, int nrhs);
-  // the partitioned-inverse solve applies to this plan and is switched on.
+  // the partitioned-inverse solve applies and is switched on.
   // Not for FP64 static LDL^T: explicit inverses of its unit-lower diagonal
   // blocks (indefinite, static pivots) raise the backward error several
   // times over block substitution (80^3-like shifted Laplacians: 6x on the
@@ -168,7 +168,7 @@ class Engine {
   // drop-in's 10x bar; as the FP32 preconditioner under refinement it is
   // used, the refinement restores the accuracy
   bool use_ginv() const {
-    return plan_.ginv_ok && opt_.solve_inverse != 0 && (opt_.ldl == 0 || opt_.precision == 1);
+    return opt_.solve_inverse != 0 && ginv_fits_ && (opt_.ldl == 0 || opt_.precision == 1);
   }
   // prepares G from the current factor once per factorization
   template <typename T>
@@ -231,6 +231,7 @@ class Engine {
   std::vector<int32_t> h_rowind_;
   // device memory
   void* d_sn_ = nullptr;
+  SolvePanel* d_panels_ = nullptr;
   int32_t* d_lindx0_ = nullptr;
   int64_t* d_tcol_ = nullptr;
   int64_t* d_tmap_ = nullptr;
@@ -265,6 +266,7 @@ class Engine {
   double* d_arena64_ = nullptr;
   void* d_dinv_ = nullptr;     // inverted 16x16 diagonal tiles of the factor
   void* d_garena_ = nullptr;   // partitioned-inverse solve factor G (panel shapes, factor precision)
+  bool ginv_fits_ = true;      // its memory was there
   bool ginv_ready_ = false;    // G holds the current factor's inverse
   float* d_arena32_ = nullptr;
   // solve work

@@ -19,9 +19,10 @@
 //                FP32 MFMA 16x16x4, written straight from registers into the
 //                target panels through precomputed relative indices
 //                (blockCell_t::update, :1180-1466).
-//  k_sdiag4 / k_sdiag3 / k_sdiag_fwd / k_soffm_fwd / k_scale_d / k_soffm_bwd /
-//  k_sdiag_bwd   supernodal forward/backward solve (forward_update[_contrib],
+//  k_sdiag4 / k_sdiag3 / k_soffm_fwd / k_scale_d / k_soffm_bwd
+//                supernodal forward/backward solve (forward_update[_contrib],
 //                back_update[_contrib], :1486-1797).
+//  k_gprep / k_gsolve_fwd[4] / k_gsolve_bwd  the same with partitioned inverses.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -31,7 +32,6 @@
 namespace spk {
 namespace dev {
 
-constexpr int NB = kNB;
 constexpr int TILE = kTile;
 constexpr int NT = 256;
 
@@ -1413,104 +1413,16 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
 
 
 // ---------------------------------------------------------------------------
-// Solve.  Vectors are row-major n x nrhs in the permuted numbering.
-// Forward:  X_I = L_II^{-1} Y_I  (k_sdiag_fwd), then Y[struct rows] -= L_off X_I
-//           (k_soff_fwd, atomics).  LDL then scales by D^{-1} (k_scale_d).
-// Backward: X_I -= L_off^T X[struct rows] (k_soff_bwd, atomics into X_I),
-//           then X_I = L_II^{-T} X_I (k_sdiag_bwd).
+// Solve, panel by panel (SolvePanel: a supernode wider than kStep is a chain
+// of panels, 24^3 with MMD and widths up to 1,024: solve 1.59 -> 0.27 ms
+// against one workgroup per supernode in blocks of 64 columns).  Vectors are
+// row-major n x nrhs in the permuted numbering.
+// Forward:  X_I = L_II^{-1} Y_I, then Y[struct rows] -= L_off X_I (atomics).
+//           LDL then scales by D^{-1} (k_scale_d).
+// Backward: X_I -= L_off^T X[struct rows] (atomics into X_I), then
+//           X_I = L_II^{-T} X_I.
 // ---------------------------------------------------------------------------
-constexpr int JC = 64;  // right-hand sides per LDS chunk
 
-
-// Triangular solve of one diagonal block (bs <= 64) for right-hand sides
-// handled one per wave: lane i holds x_i, the pivot value is broadcast with
-// readlane and every lane applies one fused multiply-add per step.
-// Forward: L x = z; backward: L^T x = z.  Lk[j][k] = L(c0+k, c0+j) for k > j
-// (zero elsewhere); invd = 1/L_jj (LL) or 1 (LDL, unit diagonal).
-template <typename T, bool BWD>
-__device__ __forceinline__ void block_solve_waves(T* __restrict__ X, int64_t rowbase, int nrhs,
-                                                  int bs, T (*Lk)[NB + 1], const T* invd) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lr = min(lane, bs - 1);
-  for (int jj = wave; jj < nrhs; jj += NT / 64) {
-    T* col = X + rowbase * nrhs + jj;
-    T xi = col[(int64_t)lr * nrhs];
-    xi = (lane < bs) ? xi : T(0);
-    if (!BWD) {
-      for (int j = 0; j < bs; ++j) {
-        const T xj = readlane_t(xi, j) * invd[j];
-        xi = (lane == j) ? xj : xi - Lk[j][lane] * xj;
-      }
-    } else {
-      for (int j = bs - 1; j >= 0; --j) {
-        const T xj = readlane_t(xi, j) * invd[j];
-        xi = (lane == j) ? xj : xi - Lk[lane][j] * xj;
-      }
-    }
-    if (lane < bs) col[(int64_t)lane * nrhs] = xi;
-  }
-}
-
-// Stage diagonal block c0 of a panel in LDS: Lk[j][k] = L(c0+k, c0+j) for
-// k > j (zero elsewhere) and invd[j] = 1/L(c0+j,c0+j) (LL) or 1 (LDL).
-template <typename T, bool LDL>
-__device__ __forceinline__ void stage_diag_block(const T* __restrict__ P, int64_t ld, int c0, int bs,
-                                                 T (*Lk)[NB + 1], T* invd) {
-  for (int idx = threadIdx.x; idx < NB * NB; idx += NT) {
-    const int k = idx % NB, j = idx / NB;
-    const T v = P[(int64_t)(c0 + min(j, bs - 1)) * ld + c0 + min(k, bs - 1)];
-    Lk[j][k] = (k < bs && j < bs && k > j) ? v : T(0);
-    if (k == j) invd[j] = (j < bs) ? (LDL ? T(1) : T(1) / v) : T(0);
-  }
-}
-
-// Forward diagonal solve of a supernode: X_I = L_II^{-1} Y_I, blocked by 64
-// columns; task {sn}.  Threads own right-hand sides for the block solves and
-// (row, rhs) pairs for the updates of the supernode's remaining rows.
-template <typename T, bool LDL>
-__global__ __launch_bounds__(NT) void k_sdiag_fwd(const SnInfo* __restrict__ sn,
-                                                   const Task4* __restrict__ tasks,
-                                                   const T* __restrict__ arena,
-                                                   const T* __restrict__ Y, T* __restrict__ X,
-                                                   int nrhs) {
-  __shared__ T Lk[NB][NB + 1];
-  __shared__ T invd[NB];
-  const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
-  const int tid = threadIdx.x;
-  const T* __restrict__ P = arena + s.off;
-  const int64_t ld = s.r;
-  const int64_t base = (int64_t)s.fc * nrhs;
-  for (int64_t i = tid; i < (int64_t)s.w * nrhs; i += NT) X[base + i] = Y[base + i];
-  __syncthreads();
-  for (int c0 = 0; c0 < s.w; c0 += NB) {
-    const int bs = min(NB, s.w - c0);
-    stage_diag_block<T, LDL>(P, ld, c0, bs, Lk, invd);
-    __syncthreads();
-    block_solve_waves<T, false>(X, (int64_t)s.fc + c0, nrhs, bs, Lk, invd);
-    __syncthreads();
-    // rows of the supernode below this block: X_i -= L(i, block) x_block;
-    // fixed-length unrolled dot products (clamped columns, zero weights
-    // beyond bs) keep all loads of a row in flight.
-    const int below = s.w - c0 - bs;
-    for (int idx = tid; idx < below * nrhs; idx += NT) {
-      const int i = c0 + bs + idx / nrhs, jj = idx % nrhs;
-      const T* lrow = P + (int64_t)c0 * ld + i;
-      const T* xb = X + base + (int64_t)c0 * nrhs + jj;
-      T lv[NB], xv[NB];
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        lv[k] = lrow[(int64_t)min(k, bs - 1) * ld];
-        xv[k] = xb[(int64_t)min(k, bs - 1) * nrhs];
-      }
-      T acc = T(0);
-#pragma unroll
-      for (int k = 0; k < NB; ++k) acc += (k < bs) ? lv[k] * xv[k] : T(0);
-      X[base + (int64_t)i * nrhs + jj] -= acc;
-    }
-    __syncthreads();
-  }
-}
 
 // Diagonal-block solve on MFMA (w <= 160), the panel-TRSM recurrence with
 // right-hand sides in place of panel rows: for 16-row blocks t
@@ -1521,7 +1433,7 @@ __global__ __launch_bounds__(NT) void k_sdiag_fwd(const SnInfo* __restrict__ sn,
 // LDL: unit inverse tiles, D applied by k_scale_d.  Task {sn, inverse-tile
 // base, -, -}, blockIdx.y = chunk of 64 right-hand sides; Y may alias X.
 template <typename T, bool BWD, int NBM>
-__global__ __launch_bounds__(NT) void k_sdiag3(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_sdiag3(const SolvePanel* __restrict__ sn,
                                                const Task4* __restrict__ tasks,
                                                const T* __restrict__ arena, const T* __restrict__ dinv,
                                                const T* Y, T* X, int nrhs) {
@@ -1529,11 +1441,11 @@ __global__ __launch_bounds__(NT) void k_sdiag3(const SnInfo* __restrict__ sn,
   constexpr int NTL = NBM * (NBM + 1) / 2;
   __shared__ __attribute__((aligned(16))) T tl[NTL * TSZ];
   const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
+  const SolvePanel s = sn[t.a];
   const int w = s.w;
   const int nbt = (w + SUB - 1) / SUB;
   const T* __restrict__ P = arena + s.off;
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   {
     const int r = tid & 15, c = tid >> 4;
@@ -1634,7 +1546,7 @@ __global__ __launch_bounds__(NT) void k_sdiag3(const SnInfo* __restrict__ sn,
 // recurrence as k_sdiag3, which handles each right-hand-side group with one
 // wave.  Task {sn, inverse-tile base, -, -}; Y may alias X.
 template <typename T, bool BWD, int NBM>
-__device__ __forceinline__ void sdiag4_body(const SnInfo& s, int64_t invb,
+__device__ __forceinline__ void sdiag4_body(const SolvePanel& s, int64_t invb,
                                             const T* __restrict__ arena, const T* __restrict__ dinv,
                                             const T* Y, T* X, int nrhs, int j0, T (*xs)[4][64]) {
   typedef typename Mfma<T>::v4 v4;
@@ -1642,7 +1554,7 @@ __device__ __forceinline__ void sdiag4_body(const SnInfo& s, int64_t invb,
   const int w = s.w;
   const int nbt = (w + SUB - 1) / SUB;
   const T* __restrict__ P = arena + s.off;
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const T* __restrict__ Dv = dinv + invb * (SUB * SUB);
@@ -1736,7 +1648,7 @@ __device__ __forceinline__ void sdiag4_body(const SnInfo& s, int64_t invb,
 }
 
 template <typename T, bool BWD, int NBM>
-__global__ __launch_bounds__(NT) void k_sdiag4(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_sdiag4(const SolvePanel* __restrict__ sn,
                                                const Task4* __restrict__ tasks,
                                                const T* __restrict__ arena, const T* __restrict__ dinv,
                                                const T* Y, T* X, int nrhs) {
@@ -1751,7 +1663,7 @@ __global__ __launch_bounds__(NT) void k_sdiag4(const SnInfo* __restrict__ sn,
 // blockIdx.y = right-hand-side chunk.
 // Forward:  Y[row(a)] -= sum_k L(a,k) X_I(k)      (one atomic per output)
 template <typename T>
-__device__ __forceinline__ void soffm_fwd_body(const SnInfo& s, int rt, const T* __restrict__ arena,
+__device__ __forceinline__ void soffm_fwd_body(const SolvePanel& s, int rt, const T* __restrict__ arena,
                                                const int32_t* __restrict__ lindx0,
                                                const T* __restrict__ X, T* __restrict__ Y, int nrhs,
                                                int j0) {
@@ -1768,7 +1680,7 @@ __device__ __forceinline__ void soffm_fwd_body(const SnInfo& s, int rt, const T*
   const T jmask = T(jn < nrhs);
   const T* __restrict__ Pa = arena + s.off + s.w + ac;      // L(a, k) at Pa[k * ld]
   const T* __restrict__ Xk = X + (int64_t)s.fc * nrhs + jc;  // X_I(k, j) at Xk[k * nrhs]
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const int w = s.w;
   v4 acc = v4{0, 0, 0, 0};
   for (int k0 = 0; k0 < w; k0 += 32) {
@@ -1793,7 +1705,7 @@ __device__ __forceinline__ void soffm_fwd_body(const SnInfo& s, int rt, const T*
 }
 
 template <typename T>
-__global__ __launch_bounds__(NT) void k_soffm_fwd(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_soffm_fwd(const SolvePanel* __restrict__ sn,
                                                    const Task4* __restrict__ tasks,
                                                    const T* __restrict__ arena,
                                                    const int32_t* __restrict__ lindx0,
@@ -1807,7 +1719,7 @@ __global__ __launch_bounds__(NT) void k_soffm_fwd(const SnInfo* __restrict__ sn,
 // 64 rows, atomics into X_I).  The reduction index is permuted so that lane
 // (m, g) reads rows 16g..16g+15 of one column: one cache line per lane.
 template <typename T>
-__device__ __forceinline__ void soffm_bwd_body(const SnInfo& s, int rt, const T* __restrict__ arena,
+__device__ __forceinline__ void soffm_bwd_body(const SolvePanel& s, int rt, const T* __restrict__ arena,
                                                const int32_t* __restrict__ lindx0, T* __restrict__ X,
                                                int nrhs, int j0) {
   typedef typename Mfma<T>::v4 v4;
@@ -1818,7 +1730,7 @@ __device__ __forceinline__ void soffm_bwd_body(const SnInfo& s, int rt, const T*
   const int jn = j0 + mi;
   const int jc = min(jn, nrhs - 1);
   const T jmask = T(jn < nrhs);
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   // B operand (shared by every column block): Y rows of this tile
   int rowi[16];
 #pragma unroll
@@ -1866,7 +1778,7 @@ __device__ __forceinline__ void soffm_bwd_body(const SnInfo& s, int rt, const T*
 }
 
 template <typename T>
-__global__ __launch_bounds__(NT) void k_soffm_bwd(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_soffm_bwd(const SolvePanel* __restrict__ sn,
                                                    const Task4* __restrict__ tasks,
                                                    const T* __restrict__ arena,
                                                    const int32_t* __restrict__ lindx0,
@@ -1893,13 +1805,13 @@ __global__ __launch_bounds__(NT) void k_soffm_bwd(const SnInfo* __restrict__ sn,
 // Stage the strict lower tiles of the diagonal block (I > J) and the
 // inverse diagonal tiles (I == J) of supernode s in LDS (all 256 threads).
 template <typename T, int NBM>
-__device__ __forceinline__ void stage_block_and_inverses(const SnInfo& s, int64_t invb,
+__device__ __forceinline__ void stage_block_and_inverses(const SolvePanel& s, int64_t invb,
                                                          const T* __restrict__ arena,
                                                          const T* __restrict__ dinv, T* __restrict__ tl) {
   constexpr int NTL = NBM * (NBM + 1) / 2;
   const int w = s.w;
   const int nb = (w + SUB - 1) / SUB;
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const T* __restrict__ P = arena + s.off;
   const int tid = threadIdx.x;
   const int r = tid & 15, c = tid >> 4;
@@ -1934,19 +1846,19 @@ __device__ __forceinline__ void stage_block_and_inverses(const SnInfo& s, int64_
 // 16 rows per wave (Y^T in MFMA accumulators, as in the panel TRSM).  Task
 // {sn, row tile, inverse-tile base, -}.
 template <typename T, int NBM>
-__global__ __launch_bounds__(NT) void k_gprep(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+__global__ __launch_bounds__(NT) void k_gprep(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                               const T* __restrict__ arena, const T* __restrict__ dinv,
                                               T* __restrict__ garena) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int NTL = NBM * (NBM + 1) / 2;
   __shared__ __attribute__((aligned(16))) T tl[NTL * TSZ];
   const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
+  const SolvePanel s = sn[t.a];
   stage_block_and_inverses<T, NBM>(s, t.c, arena, dinv, tl);
   __syncthreads();
   const int w = s.w;
   const int nb = (w + SUB - 1) / SUB;
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int R0 = t.b * TILE + 16 * wave;
   if (R0 >= s.r) return;  // no barrier follows
@@ -2026,19 +1938,19 @@ __global__ __launch_bounds__(NT) void k_gprep(const SnInfo* __restrict__ sn, con
 // structure rows with atomics.  Y_I of a level's supernodes is never the
 // target of the same level's updates (targets are ancestors).
 template <typename T, bool LDL, int NBM>
-__global__ __launch_bounds__(NT) void k_gsolve_fwd(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+__global__ __launch_bounds__(NT) void k_gsolve_fwd(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                                    const T* __restrict__ garena, const T* __restrict__ arena,
                                                    const int32_t* __restrict__ lindx0, T* Y, T* __restrict__ Xf,
                                                    int nrhs) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int NQ = 4 * NBM;  // k chunks of 4
   const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
+  const SolvePanel s = sn[t.a];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int a0 = t.b * TILE + 16 * wave;
   if (a0 >= s.r) return;
   const int w = s.w;
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const int mi = lane & 15, g = lane >> 4;
   const int ac = min(a0 + mi, s.r - 1);
   const T* __restrict__ Ga = garena + s.off + ac;  // G(a, k) at Ga[k ld]
@@ -2098,19 +2010,19 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd(const SnInfo* __restrict__ sn
 // hundreds of tiles (48^3, 600 tiles: 27 -> 19 us).  Task as k_gsolve_fwd's;
 // workgroup 4 t + q takes rows 16 q .. of task t's tile.
 template <typename T, bool LDL, int NBM>
-__global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+__global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                                     const T* __restrict__ garena, const T* __restrict__ arena,
                                                     const int32_t* __restrict__ lindx0, T* Y, T* __restrict__ Xf,
                                                     int nrhs) {
   typedef typename Mfma<T>::v4 v4;
   __shared__ T part[4][4][64];
   const Task4 t = tasks[blockIdx.x >> 2];
-  const SnInfo s = sn[t.a];
+  const SolvePanel s = sn[t.a];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int a0 = t.b * TILE + 16 * (int)(blockIdx.x & 3);
   if (a0 >= s.r) return;  // the whole workgroup
   const int w = s.w, k0 = 4 * NBM * wave;
-  const int64_t ld = s.r;
+  const int64_t ld = s.ld;
   const int mi = lane & 15, g = lane >> 4;
   const T* __restrict__ Ga = garena + s.off + min(a0 + mi, s.r - 1);
   T av[NBM];
@@ -2165,13 +2077,13 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SnInfo* __restrict__ s
 // every load of a block is issued before its first product; partial sums of
 // the tile go to X_I with atomics (X zeroed before the sweep).
 template <typename T>
-__global__ __launch_bounds__(NT) void k_gsolve_bwd(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+__global__ __launch_bounds__(NT) void k_gsolve_bwd(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                                    const T* __restrict__ garena,
                                                    const int32_t* __restrict__ lindx0, const T* __restrict__ Xf,
                                                    T* X, int nrhs) {
   typedef typename Mfma<T>::v4 v4;
   const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
+  const SolvePanel s = sn[t.a];
   const int lane = threadIdx.x & 63, kb = 4 * blockIdx.z + (threadIdx.x >> 6);
   const int w = s.w;
   if (16 * kb >= w) return;  // no barrier follows
@@ -2181,7 +2093,7 @@ __global__ __launch_bounds__(NT) void k_gsolve_bwd(const SnInfo* __restrict__ sn
 #pragma unroll
   for (int st = 0; st < 16; ++st) rowi[st] = lindx0[s.lx + min(a0 + 16 * g + st, s.r - 1)];
   T av[16];
-  const T* __restrict__ Gc = garena + s.off + (int64_t)min(16 * kb + mi, w - 1) * s.r;
+  const T* __restrict__ Gc = garena + s.off + (int64_t)min(16 * kb + mi, w - 1) * s.ld;
 #pragma unroll
   for (int st = 0; st < 16; ++st) av[st] = Gc[min(a0 + 16 * g + st, s.r - 1)];
   const int nblk = (nrhs + SUB - 1) / SUB;
@@ -2302,7 +2214,7 @@ __global__ void k_df_reset(DfState st, const int* __restrict__ dcnt0, const int*
 }
 
 template <typename T>
-__global__ __launch_bounds__(NT) void k_fsolve_df(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_fsolve_df(const SolvePanel* __restrict__ sn,
                                                   const Task4* __restrict__ tasks,
                                                   const int32_t* __restrict__ tend, int ntasks,
                                                   const int32_t* __restrict__ tgt,
@@ -2317,7 +2229,7 @@ __global__ __launch_bounds__(NT) void k_fsolve_df(const SnInfo* __restrict__ sn,
     const int ti = df_ticket(st.head, &slot);
     if (ti >= ntasks) break;
     const Task4 t = tasks[ti];
-    const SnInfo s = sn[t.b];
+    const SolvePanel s = sn[t.b];
     if (t.a == 0) {
       df_wait(st.dcnt + t.b, 0, st.abort_);
       for (int j0 = 0; j0 < nrhs; j0 += SUB)
@@ -2335,7 +2247,7 @@ __global__ __launch_bounds__(NT) void k_fsolve_df(const SnInfo* __restrict__ sn,
 }
 
 template <typename T>
-__global__ __launch_bounds__(NT) void k_bsolve_df(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_bsolve_df(const SolvePanel* __restrict__ sn,
                                                   const Task4* __restrict__ tasks,
                                                   const int32_t* __restrict__ tend, int ntasks,
                                                   const int32_t* __restrict__ tgt,
@@ -2350,7 +2262,7 @@ __global__ __launch_bounds__(NT) void k_bsolve_df(const SnInfo* __restrict__ sn,
     const int ti = df_ticket(st.head + 1, &slot);
     if (ti >= ntasks) break;
     const Task4 t = tasks[ti];
-    const SnInfo s = sn[t.b];
+    const SolvePanel s = sn[t.b];
     if (t.a == 2) {
       for (int q = t.d; q < tend[ti]; ++q) df_wait(st.bflag + tgt[q], 1, st.abort_);
       for (int j0 = 0; j0 < nrhs; j0 += SUB) soffm_bwd_body<T>(s, t.c, arena, lindx0, X, nrhs, j0);
@@ -2367,62 +2279,16 @@ __global__ __launch_bounds__(NT) void k_bsolve_df(const SnInfo* __restrict__ sn,
 }
 
 template <typename T>
-__global__ __launch_bounds__(NT) void k_scale_d(const SnInfo* __restrict__ sn,
+__global__ __launch_bounds__(NT) void k_scale_d(const SolvePanel* __restrict__ sn,
                                                  const Task4* __restrict__ tasks,
                                                  const T* __restrict__ arena, T* __restrict__ X,
                                                  int nrhs) {
   const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
+  const SolvePanel s = sn[t.a];
   const T* __restrict__ P = arena + s.off;
   for (int64_t idx = threadIdx.x; idx < (int64_t)s.w * nrhs; idx += NT) {
     int i = (int)(idx / nrhs);
-    X[(int64_t)s.fc * nrhs + idx] /= P[(int64_t)i * s.r + i];
-  }
-}
-
-// Backward diagonal solve of a supernode: X_I = L_II^{-T} X_I, blocks from
-// the last one; task {sn}.
-template <typename T, bool LDL>
-__global__ __launch_bounds__(NT) void k_sdiag_bwd(const SnInfo* __restrict__ sn,
-                                                   const Task4* __restrict__ tasks,
-                                                   const T* __restrict__ arena,
-                                                   T* __restrict__ X, int nrhs) {
-  __shared__ T Lk[NB][NB + 1];
-  __shared__ T invd[NB];
-  const Task4 t = tasks[blockIdx.x];
-  const SnInfo s = sn[t.a];
-  const int tid = threadIdx.x;
-  const T* __restrict__ P = arena + s.off;
-  const int64_t ld = s.r;
-  const int64_t base = (int64_t)s.fc * nrhs;
-  const int nb = (s.w + NB - 1) / NB;
-  for (int blk = nb - 1; blk >= 0; --blk) {
-    const int c0 = blk * NB;
-    const int bs = min(NB, s.w - c0);
-    // X_block -= L(rows below the block inside the supernode, block)^T x_below
-    const int below = s.w - c0 - bs;
-    for (int idx = tid; idx < bs * nrhs; idx += NT) {
-      const int k = idx / nrhs, jj = idx % nrhs;
-      const T* lcol = P + (int64_t)(c0 + k) * ld + c0 + bs;
-      const T* xb = X + base + (int64_t)(c0 + bs) * nrhs + jj;
-      T acc = T(0);
-      for (int i0 = 0; i0 < below; i0 += NB) {
-        const int cnt = min(NB, below - i0);
-        T lv[NB], xv[NB];
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          lv[i] = lcol[i0 + min(i, cnt - 1)];
-          xv[i] = xb[(int64_t)(i0 + min(i, cnt - 1)) * nrhs];
-        }
-#pragma unroll
-        for (int i = 0; i < NB; ++i) acc += (i < cnt) ? lv[i] * xv[i] : T(0);
-      }
-      X[base + (int64_t)(c0 + k) * nrhs + jj] -= acc;
-    }
-    stage_diag_block<T, LDL>(P, ld, c0, bs, Lk, invd);
-    __syncthreads();
-    block_solve_waves<T, true>(X, (int64_t)s.fc + c0, nrhs, bs, Lk, invd);
-    __syncthreads();
+    X[(int64_t)s.fc * nrhs + idx] /= P[(int64_t)i * s.ld + i];
   }
 }
 

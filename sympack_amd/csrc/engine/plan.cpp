@@ -507,84 +507,83 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     for (size_t q = level_first; q < p.factor_seq.size(); ++q) p.factor_seq[q].level = L;
   }
 
-  // ---- solve task lists ----
-  // Per level: one diagonal task per supernode ({sn, inverse-tile base}) and
-  // one off-diagonal task per 64-row tile of the panel below the diagonal.
-  std::vector<int64_t> dfirst(p.nlevels), mfirst(p.nlevels), mcount(p.nlevels);
-  for (int L = 0; L < p.nlevels; ++L) {
-    const auto& sns = by_level[L];
-    dfirst[L] = (int64_t)p.sdiag_tasks.size();
-    for (Int I : sns) p.sdiag_tasks.push_back({I, (int32_t)p.inv_base[I], 0, 0});
-    mfirst[L] = (int64_t)p.soffm_tasks.size();
-    for (Int I : sns) {
-      int64_t m = p.sn[I].r - p.sn[I].w;
-      for (int64_t rt = 0; rt < ceil_div(m, kTile); ++rt) p.soffm_tasks.push_back({I, (int32_t)rt, 0, 0});
+  // ---- solve panels and their levels ----
+  std::vector<int32_t> slevel;       // per panel
+  std::vector<int32_t> inv_of;       // per panel: first inverse tile
+  std::vector<int32_t> child_top(ns, 0);  // per supernode: first level above its children's panels
+  for (Int I = 0; I < ns; ++I) {     // children precede parents
+    const SnInfo& si = p.sn[I];
+    int32_t L = child_top[I];
+    for (int32_t c0 = 0; c0 < si.w; c0 += kStep, ++L) {
+      p.panels.push_back({si.off + (int64_t)c0 * si.r + c0, si.r, si.r - c0, std::min(kStep, si.w - c0), si.fc + c0,
+                          si.lx + c0, 0});
+      inv_of.push_back((int32_t)(p.inv_base[I] + c0 / kSub));
+      slevel.push_back(L);
     }
-    mcount[L] = (int64_t)p.soffm_tasks.size() - mfirst[L];
+    if (si.r > si.w) {
+      int32_t& top = child_top[row_sup[p.lindx0[si.lx + si.w]]];
+      top = std::max(top, L);
+    }
   }
-  // partitioned-inverse solve: 64-row tiles over all rows of every panel,
-  // grouped by level (solve sweeps) and by diagonal-block bucket (the
-  // preparation, one launch per bucket over all supernodes)
-  p.ginv_ok = p.max_w <= kStep;
-  if (p.ginv_ok) {
-    std::vector<int> lbucket(p.nlevels, 1);
-    for (int L = 0; L < p.nlevels; ++L)
-      for (Int I : by_level[L]) lbucket[L] = std::max(lbucket[L], diag_bucket((int)ceil_div(p.sn[I].w, kSub)));
-    std::vector<int64_t> gfirst(p.nlevels), gcount(p.nlevels);
-    for (int L = 0; L < p.nlevels; ++L) {
-      gfirst[L] = (int64_t)p.gtiles.size();
-      for (Int I : by_level[L])
-        for (int64_t rt = 0; rt < ceil_div(p.sn[I].r, kTile); ++rt)
-          p.gtiles.push_back({I, (int32_t)rt, (int32_t)p.inv_base[I], 0});
-      gcount[L] = (int64_t)p.gtiles.size() - gfirst[L];
+  const Int np = (Int)p.panels.size();
+  int32_t nslevels = 0;
+  for (int32_t L : slevel) nslevels = std::max(nslevels, L + 1);
+  std::vector<std::vector<Int>> panels_at(nslevels);
+  for (Int q = 0; q < np; ++q) panels_at[slevel[q]].push_back(q);
+  auto bucket_of = [&](Int q) { return diag_bucket((int)ceil_div(p.panels[q].w, kSub)); };
+
+  // ---- solve task lists ----
+  // Per level: one diagonal task per panel, one off-diagonal task per 64-row
+  // tile below the diagonal block, and for the partitioned inverse one task
+  // per 64-row tile of the whole panel.
+  std::vector<LaunchRange> diag(nslevels), offd(nslevels), part(nslevels);
+  for (int L = 0; L < nslevels; ++L) {
+    diag[L] = {3, (int64_t)p.sdiag_tasks.size(), 0, 1, L};
+    offd[L] = {4, (int64_t)p.soffm_tasks.size(), 0, 1, L};
+    part[L] = {10, (int64_t)p.gtiles.size(), 0, 1, L};
+    for (Int q : panels_at[L]) {
+      const SolvePanel& sp = p.panels[q];
+      diag[L].aux = std::max(diag[L].aux, bucket_of(q));
+      p.sdiag_tasks.push_back({q, inv_of[q], 0, 0});
+      for (int64_t rt = 0; rt < ceil_div(sp.r - sp.w, kTile); ++rt) p.soffm_tasks.push_back({q, (int32_t)rt, 0, 0});
+      for (int64_t rt = 0; rt < ceil_div(sp.r, kTile); ++rt) p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
     }
-    for (int L = 0; L < p.nlevels; ++L) {
-      LaunchRange f{10, gfirst[L], gcount[L], lbucket[L], L};
-      if (gcount[L]) p.gfwd_seq.push_back(f);
+    diag[L].count = (int64_t)p.sdiag_tasks.size() - diag[L].first;
+    offd[L].count = (int64_t)p.soffm_tasks.size() - offd[L].first;
+    part[L].count = (int64_t)p.gtiles.size() - part[L].first;
+    offd[L].aux = part[L].aux = diag[L].aux;
+  }
+  // forward: levels bottom-up, diagonal solves then off-diagonal updates;
+  // backward: levels top-down, off-diagonal gathers then diagonal solves
+  for (int L = 0; L < nslevels; ++L) {
+    p.fwd_seq.push_back(diag[L]);
+    if (offd[L].count) p.fwd_seq.push_back(offd[L]);
+    p.gfwd_seq.push_back(part[L]);
+  }
+  for (int L = nslevels - 1; L >= 0; --L) {
+    LaunchRange d = diag[L], o = offd[L], g = part[L];
+    d.kind = 6;
+    o.kind = 5;
+    g.kind = 11;
+    if (o.count) p.bwd_seq.push_back(o);
+    p.bwd_seq.push_back(d);
+    p.gbwd_seq.push_back(g);
+  }
+  // preparation of the partitioned inverse: the same tiles, regrouped by the
+  // bucket of their own panel (appended after the level-ordered tiles)
+  for (int bk : {1, 2, 4, 6, 10}) {
+    LaunchRange r{12, (int64_t)p.gtiles.size(), 0, bk, -1};
+    for (Int q = 0; q < np; ++q) {
+      if (bucket_of(q) != bk) continue;
+      for (int64_t rt = 0; rt < ceil_div(p.panels[q].r, kTile); ++rt)
+        p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
     }
-    for (int L = p.nlevels - 1; L >= 0; --L) {
-      LaunchRange b{11, gfirst[L], gcount[L], lbucket[L], L};
-      if (gcount[L]) p.gbwd_seq.push_back(b);
-    }
-    // preparation: the same tiles, regrouped by the bucket of their own
-    // supernode (appended after the level-ordered tiles)
-    for (int bk : {1, 2, 4, 6, 10}) {
-      LaunchRange r{12, (int64_t)p.gtiles.size(), 0, bk, -1};
-      for (Int I = 0; I < ns; ++I) {
-        if (diag_bucket((int)ceil_div(p.sn[I].w, kSub)) != bk) continue;
-        for (int64_t rt = 0; rt < ceil_div(p.sn[I].r, kTile); ++rt)
-          p.gtiles.push_back({I, (int32_t)rt, (int32_t)p.inv_base[I], 0});
-      }
-      r.count = (int64_t)p.gtiles.size() - r.first;
-      if (r.count) p.gprep_seq.push_back(r);
-    }
+    r.count = (int64_t)p.gtiles.size() - r.first;
+    if (r.count) p.gprep_seq.push_back(r);
   }
 
   // the dependency-driven solve's lists are built on demand (build_dataflow_lists)
   p.df_ok = p.max_w <= kStep;
-
-  // forward: levels bottom-up, diagonal solves then off-diagonal updates.
-  std::vector<int> dbucket(p.nlevels, 1);
-  for (int L = 0; L < p.nlevels; ++L) {
-    int wmax = 1;
-    for (Int I : by_level[L]) wmax = std::max<int>(wmax, p.sn[I].w);
-    dbucket[L] = wmax > kStep ? 0 : diag_bucket((int)ceil_div(wmax, kSub));
-  }
-  for (int L = 0; L < p.nlevels; ++L) {
-    LaunchRange d{3, dfirst[L], (int64_t)by_level[L].size()};
-    d.aux = dbucket[L];
-    d.level = L;
-    p.fwd_seq.push_back(d);
-    if (mcount[L]) p.fwd_seq.push_back({4, mfirst[L], mcount[L], 0, L});
-  }
-  // backward: levels top-down, off-diagonal gathers then diagonal solves.
-  for (int L = p.nlevels - 1; L >= 0; --L) {
-    if (mcount[L]) p.bwd_seq.push_back({5, mfirst[L], mcount[L], 0, L});
-    LaunchRange d{6, dfirst[L], (int64_t)by_level[L].size()};
-    d.aux = dbucket[L];
-    d.level = L;
-    p.bwd_seq.push_back(d);
-  }
 }
 
 

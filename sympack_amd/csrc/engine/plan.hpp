@@ -20,7 +20,6 @@
 
 namespace spk {
 
-constexpr int kNB = 64;      // diagonal block width of the blocked solve
 constexpr int kTile = 64;    // update tile edge (rows x cols)
 constexpr int kStep = 160;   // panel columns factored per step (diagonal block <= 160 x 160)
 constexpr int kSub = 16;     // sub-block edge inside a diagonal block (MFMA 16x16 tiles)
@@ -47,6 +46,19 @@ struct SnInfo {            // mirrored on the device (16-byte aligned)
 
 struct Task4 {
   int32_t a, b, c, d;
+};
+
+// One panel of the solve: columns [c0, c0 + w), w <= kStep, of a supernode
+// with the rows of its structure from c0 on (so a supernode of at most kStep
+// columns is one panel, a wider one a chain of them).
+struct SolvePanel {        // mirrored on the device
+  int64_t off;             // arena offset of the panel's first diagonal entry
+  int32_t ld;              // leading dimension (rows of the whole supernode)
+  int32_t r;               // rows, w of them diagonal
+  int32_t w;
+  int32_t fc;              // first column, 0-based, permuted numbering
+  int32_t lx;              // offset of the panel's first row in lindx0
+  int32_t pad;
 };
 
 // Schur updates along chains.  A separator wider than the supernode limit is
@@ -178,18 +190,20 @@ struct Plan {
   // segment; beyond the chain's columns the chain's last member has both.
   std::vector<int32_t> deferred_into;
   std::vector<LaunchRange> factor_seq;
-  // solve
-  std::vector<Task4> sdiag_tasks;  // {sn, 0, 0, 0}: diagonal-block solves
-  std::vector<Task4> soffm_tasks;  // {sn, row_tile, 0, 0}: 64-row tiles of the off-diagonal panel
-  std::vector<LaunchRange> fwd_seq, bwd_seq;  // kind 3/6 aux: diag_bucket of the level, 0 = w > kStep
-  // Partitioned-inverse solve, available when every supernode is at most
-  // kStep wide: G_I = [I; L_off] L_II^{-1} (r_I x w_I, the panel's shape and
-  // offsets, in its own arena) is prepared once per factorization; then each
-  // etree level costs one forward launch [X_I; dY] = G_I Y_I and one
-  // backward launch X_I = G_I^T [X_I; -X_rows].  Tasks {sn, 64-row tile,
-  // inverse-tile base, 0} over all rows of every panel; kinds 10/11 per
-  // level, kind 12 (preparation) per diagonal-block bucket, aux = bucket.
-  bool ginv_ok = false;
+  // Solve, level by level over the panels (a supernode's panels follow one
+  // another; where every supernode is at most kStep wide the levels are the
+  // etree's).
+  std::vector<SolvePanel> panels;
+  std::vector<Task4> sdiag_tasks;  // {panel, inverse-tile base, 0, 0}: diagonal-block solves
+  std::vector<Task4> soffm_tasks;  // {panel, row_tile, 0, 0}: 64-row tiles of the rows below the block
+  std::vector<LaunchRange> fwd_seq, bwd_seq;  // kind 3/6 aux: diag_bucket of the level
+  // Partitioned-inverse solve: G = [I; L_off] L_diag^{-1} of every panel (its
+  // shape and offsets, in an arena of its own) is prepared once per
+  // factorization; then each level costs one forward launch
+  // [X_p; dY] = G_p Y_p and one backward launch X_p = G_p^T [X_p; -X_rows].
+  // Tasks {panel, 64-row tile, inverse-tile base, 0} over all rows of every
+  // panel; kinds 10/11 per level, kind 12 (preparation) per diagonal-block
+  // bucket, aux = bucket.
   std::vector<Task4> gtiles;
   std::vector<LaunchRange> gfwd_seq, gbwd_seq, gprep_seq;
   // dependency-driven solve (one persistent launch per sweep), available when

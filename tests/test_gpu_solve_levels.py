@@ -48,6 +48,15 @@ def test_fp32(ldl):
     _check(lambda: _cliques(97, 30, 50), [1, 17], ldl=ldl, precision="FP32_IR", ordering="NATURAL")
 
 
+@pytest.mark.parametrize("ldl,precision", [(False, "FP64"), (True, "FP64"), (False, "FP32_IR"), (True, "FP32_IR")])
+@pytest.mark.parametrize("w,m", [(161, 1), (320, 64), (321, 33), (479, 130)])
+def test_wide_supernode(w, m, ldl, precision):
+    """Wider than a panel of 160 columns: partitioned inverse and substitution."""
+    _check(lambda: _cliques(w, 30, m), [1, 17, 70], ldl=ldl, precision=precision, ordering="NATURAL")
+    if not ldl and precision == "FP64":
+        _check(lambda: _cliques(w, 30, m), [1, 17, 70], ordering="NATURAL", solve_inverse=False)
+
+
 def test_many_narrow_supernodes():
     rp = sp.RelaxationParameters()
     rp.SetMaxSize(150)
