@@ -1106,14 +1106,20 @@ template <typename T, bool BWD>
 void Engine::launch_sdiag(int bucket, unsigned g, const Task4* t, const T* arena, const T* Y, T* X, int nrhs) {
   const SolvePanel* sn = d_panels_;
   const T* dinv = (const T*)d_dinv_;
-  if (nrhs <= 16) {
-    // one right-hand-side group: blocks spread over the waves
+  // one workgroup per 16 right-hand sides, the 16-row blocks spread over its
+  // waves, where the level leaves CUs for that; otherwise one per 64, each
+  // wave a whole solve (and the block read once for all four).  80^3 LDL^T, 64
+  // right-hand sides, whole solve: 11.6 ms never, 10.7 ms up to 256
+  // workgroups, 11.0 ms always
+  const int64_t nblk = (nrhs + 15) / 16;
+  if (nblk == 1 || g * nblk <= kSdiagSpread) {
+    const dim3 grid(g, (unsigned)nblk);
     switch (bucket) {
-      case 1: dev::k_sdiag4<T, BWD, 1><<<g, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 2: dev::k_sdiag4<T, BWD, 2><<<g, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 4: dev::k_sdiag4<T, BWD, 4><<<g, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 6: dev::k_sdiag4<T, BWD, 6><<<g, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 10: dev::k_sdiag4<T, BWD, 10><<<g, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
+      case 1: dev::k_sdiag4<T, BWD, 1><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
+      case 2: dev::k_sdiag4<T, BWD, 2><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
+      case 4: dev::k_sdiag4<T, BWD, 4><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
+      case 6: dev::k_sdiag4<T, BWD, 6><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
+      case 10: dev::k_sdiag4<T, BWD, 10><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
       default: throw std::logic_error("bad diagonal-block bucket");
     }
     return;
@@ -1186,60 +1192,69 @@ void Engine::ensure_ginv(const T* arena) {
   ginv_ready_ = true;
 }
 
+// One forward launch of the rows of a level's panels (SUBST: those below the
+// diagonal blocks): 16 rows per workgroup, or 64 where narrow panels make
+// many tiles: little of the time is latency there, and four times the
+// workgroups cost more to start (60^3 27-point, level 0, 6,931 tiles of at
+// most 32 columns: 45 against 60 us).  Right-hand-side blocks of 16 per
+// workgroup: a launch with at least kGinvGrid workgroups walks every block in
+// each (G read once); one with fewer spreads the blocks over up to kGinvGrid
+// workgroups.
+static unsigned sweep_grid_y(int64_t wgs, int nrhs) {
+  const int64_t nblk = (nrhs + 15) / 16;
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nblk, (kGinvGrid + wgs - 1) / wgs));
+}
+template <typename T, bool SUBST>
+void Engine::launch_sweep_fwd(const LaunchRange& r, const Task4* t, const T* G, const T* arena, T* Y, T* Xf,
+                              int nrhs) {
+  const bool ldl = opt_.ldl != 0;
+  const bool rows64 = r.aux <= 2 && r.count > kGinvFew;
+  const int64_t wgs = rows64 ? r.count : 4 * r.count;
+  const dim3 grid((unsigned)wgs, sweep_grid_y(wgs, nrhs));
+#define SPK_GF(KERNEL, NBM)                                                                                      \
+  if (ldl && !SUBST)                                                                                             \
+    dev::KERNEL<T, !SUBST, NBM, SUBST><<<grid, 256, 0, stream_>>>(d_panels_, t, G, arena, d_lindx0_, Y, Xf, nrhs); \
+  else                                                                                                           \
+    dev::KERNEL<T, false, NBM, SUBST><<<grid, 256, 0, stream_>>>(d_panels_, t, G, arena, d_lindx0_, Y, Xf, nrhs);  \
+  break;
+  switch (rows64 ? -r.aux : r.aux) {
+    case -1: SPK_GF(k_gsolve_fwd, 1)
+    case -2: SPK_GF(k_gsolve_fwd, 2)
+    case 1: SPK_GF(k_gsolve_fwd4, 1)
+    case 2: SPK_GF(k_gsolve_fwd4, 2)
+    case 4: SPK_GF(k_gsolve_fwd4, 4)
+    case 6: SPK_GF(k_gsolve_fwd4, 6)
+    case 10: SPK_GF(k_gsolve_fwd4, 10)
+    default:
+      throw std::logic_error("bad diagonal-block bucket");
+  }
+#undef SPK_GF
+}
+template <typename T, bool SUBST>
+void Engine::launch_sweep_bwd(const LaunchRange& r, const Task4* t, const T* G, const T* Xf, T* X, int nrhs) {
+  const unsigned gz = (unsigned)((r.aux + 3) / 4);  // four 16-column blocks per workgroup
+  const dim3 grid((unsigned)r.count, sweep_grid_y(r.count * gz, nrhs), gz);
+  dev::k_gsolve_bwd<T, SUBST><<<grid, 256, 0, stream_>>>(d_panels_, t, G, d_lindx0_, Xf, X, nrhs);
+}
+
 // Partitioned-inverse sweeps: X zeroed, one forward launch per level
 // (Y accumulates the updates, Xf receives X_I), one backward launch per
 // level (partial sums into X).
 template <typename T>
 void Engine::ginv_sequence(T* Y, T* X, T* Xf, int nrhs) {
-  const SolvePanel* sn = d_panels_;
   const Task4* tiles = (const Task4*)d_tasks_[TA_GINV];
   const T* G = (const T*)d_garena_;
   const T* arena = opt_.precision == 0 ? (const T*)(void*)d_arena64_ : (const T*)(void*)d_arena32_;
-  const bool ldl = opt_.ldl != 0;
   const int64_t cnt = (int64_t)n_ * nrhs;
   dev::k_fill_zero<T><<<grid_for(cnt), 256, 0, stream_>>>(X, cnt);
-  // right-hand-side blocks of 16 per workgroup: a launch with at least
-  // kGinvGrid tiles walks every block in each workgroup (G read once); one
-  // with fewer spreads the blocks over up to kGinvGrid workgroups
-  const int64_t nblk = (nrhs + 15) / 16;
-  auto grid_y = [&](int64_t tiles) {
-    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nblk, (kGinvGrid + tiles - 1) / tiles));
-  };
   for (const LaunchRange& r : plan_.gfwd_seq) {
-    // narrow supernodes on a level with many tiles keep 64 rows per
-    // workgroup: little of the time is latency there, and four times the
-    // workgroups cost more to start (60^3 27-point, level 0, 6,931 tiles of
-    // at most 32 columns: 45 against 60 us)
-    const bool rows64 = r.aux <= 2 && r.count > kGinvFew;
-    const int64_t wgs = rows64 ? r.count : 4 * r.count;
-    const dim3 grid((unsigned)wgs, grid_y(wgs));
-    const Task4* t = tiles + r.first;
     launch_begin(10, r.count, nullptr, r.level);
-#define SPK_GF(KERNEL, NBM)                                                                           \
-  if (ldl)                                                                                            \
-    dev::KERNEL<T, true, NBM><<<grid, 256, 0, stream_>>>(sn, t, G, arena, d_lindx0_, Y, Xf, nrhs);    \
-  else                                                                                                \
-    dev::KERNEL<T, false, NBM><<<grid, 256, 0, stream_>>>(sn, t, G, arena, d_lindx0_, Y, Xf, nrhs);   \
-  break;
-    switch (rows64 ? -r.aux : r.aux) {
-      case -1: SPK_GF(k_gsolve_fwd, 1)
-      case -2: SPK_GF(k_gsolve_fwd, 2)
-      case 1: SPK_GF(k_gsolve_fwd4, 1)
-      case 2: SPK_GF(k_gsolve_fwd4, 2)
-      case 4: SPK_GF(k_gsolve_fwd4, 4)
-      case 6: SPK_GF(k_gsolve_fwd4, 6)
-      case 10: SPK_GF(k_gsolve_fwd4, 10)
-      default:
-        throw std::logic_error("bad diagonal-block bucket");
-    }
-#undef SPK_GF
+    launch_sweep_fwd<T, false>(r, tiles + r.first, G, arena, Y, Xf, nrhs);
     launch_end(10);
   }
   for (const LaunchRange& r : plan_.gbwd_seq) {
-    const unsigned gz = (unsigned)((r.aux + 3) / 4);  // four 16-column blocks per workgroup
-    const dim3 grid((unsigned)r.count, grid_y(r.count * gz), gz);
     launch_begin(11, r.count, nullptr, r.level);
-    dev::k_gsolve_bwd<T><<<grid, 256, 0, stream_>>>(sn, tiles + r.first, G, d_lindx0_, Xf, X, nrhs);
+    launch_sweep_bwd<T, false>(r, tiles + r.first, G, Xf, X, nrhs);
     launch_end(11);
   }
   HIP_OK(hipGetLastError());
@@ -1266,8 +1281,7 @@ void Engine::solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf) {
     if (r.kind == 3) {
       launch_sdiag<T, false>(r.aux, g, sd + r.first, arena, Y, X, nrhs);
     } else {
-      const dim3 grid((unsigned)r.count, (unsigned)((nrhs + 15) / 16));
-      dev::k_soffm_fwd<T><<<grid, 256, 0, stream_>>>(sn, sm + r.first, arena, d_lindx0_, X, Y, nrhs);
+      launch_sweep_fwd<T, true>(r, sm + r.first, arena, arena, Y, X, nrhs);
     }
     launch_end(r.kind);
   }
@@ -1280,8 +1294,7 @@ void Engine::solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf) {
     const unsigned g = (unsigned)r.count;
     launch_begin(r.kind, r.count, nullptr, r.level);
     if (r.kind == 5) {
-      const dim3 grid((unsigned)r.count, (unsigned)((nrhs + 15) / 16));
-      dev::k_soffm_bwd<T><<<grid, 256, 0, stream_>>>(sn, sm + r.first, arena, d_lindx0_, X, nrhs);
+      launch_sweep_bwd<T, true>(r, sm + r.first, arena, nullptr, X, nrhs);
     } else {
       launch_sdiag<T, true>(r.aux, g, sd + r.first, arena, X, X, nrhs);
     }

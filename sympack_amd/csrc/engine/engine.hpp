@@ -21,6 +21,9 @@ constexpr int64_t kGinvGrid = 1024;
 // a level of supernodes at most 32 wide takes k_gsolve_fwd (64 rows per
 // workgroup) above this many 64-row tiles, k_gsolve_fwd4 otherwise
 constexpr int64_t kGinvFew = 256;
+// block substitution: diagonal solves of a level go to workgroups of 16
+// right-hand sides up to this many of them
+constexpr int64_t kSdiagSpread = 256;
 // Size of the per-device array behind Engine::solve_noalloc: Y, X and Xf,
 // 3 n nrhs doubles, at most 128 MiB (n nrhs <= 5592405).
 constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;
@@ -160,6 +163,10 @@ class Engine {
   void solve_sequence(const T* arena, T* Y, T* X, int nrhs, T* Xf = nullptr);
   template <typename T>
   void ginv_sequence(T* Y, T* X, T* Xf, int nrhs);
+  template <typename T, bool SUBST>
+  void launch_sweep_fwd(const LaunchRange& r, const Task4* t, const T* G, const T* arena, T* Y, T* Xf, int nrhs);
+  template <typename T, bool SUBST>
+  void launch_sweep_bwd(const LaunchRange& r, const Task4* t, const T* G, const T* Xf, T* X, int nrhs);
   // the partitioned-inverse solve applies and is switched on.
   // Not for FP64 static LDL^T: explicit inverses of its unit-lower diagonal
   // blocks (indefinite, static pivots) raise the backward error several

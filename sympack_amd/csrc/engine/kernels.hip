@@ -19,10 +19,10 @@
 //                FP32 MFMA 16x16x4, written straight from registers into the
 //                target panels through precomputed relative indices
 //                (blockCell_t::update, :1180-1466).
-//  k_sdiag4 / k_sdiag3 / k_soffm_fwd / k_scale_d / k_soffm_bwd
+//  k_sdiag4 / k_sdiag3 / k_scale_d / k_gsolve_fwd[4] / k_gsolve_bwd
 //                supernodal forward/backward solve (forward_update[_contrib],
-//                back_update[_contrib], :1486-1797).
-//  k_gprep / k_gsolve_fwd[4] / k_gsolve_bwd  the same with partitioned inverses.
+//                back_update[_contrib], :1486-1797), by block substitution or,
+//                after k_gprep, with partitioned inverses.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -1535,8 +1535,8 @@ __global__ __launch_bounds__(NT) void k_sdiag3(const SolvePanel* __restrict__ sn
   }
 }
 
-// Diagonal-block solve for up to 16 right-hand sides (w <= 160), the
-// 16-row blocks spread over the four waves (block K belongs to wave K % 4,
+// Diagonal-block solve for 16 right-hand sides (w <= 160; blockIdx.y = block
+// of 16), the 16-row blocks spread over the four waves (block K belongs to wave K % 4,
 // its x^T in MFMA accumulators).  Each wave loads the tiles it needs (the
 // L tiles that fold other blocks into its own, and its inverse diagonal
 // tiles) straight from HBM into MFMA operand registers, all before the
@@ -1654,13 +1654,12 @@ __global__ __launch_bounds__(NT) void k_sdiag4(const SolvePanel* __restrict__ sn
                                                const T* Y, T* X, int nrhs) {
   __shared__ __attribute__((aligned(16))) T xs[NBM][4][64];
   const Task4 t = tasks[blockIdx.x];
-  sdiag4_body<T, BWD, NBM>(sn[t.a], t.b, arena, dinv, Y, X, nrhs, 0, xs);
+  sdiag4_body<T, BWD, NBM>(sn[t.a], t.b, arena, dinv, Y, X, nrhs, SUB * blockIdx.y, xs);
 }
 
-// Multi-RHS off-diagonal solve updates on MFMA (used for nrhs >= 4), one
-// workgroup per (64 panel rows below the diagonal block, 16 right-hand
-// sides); wave q owns rows 16q..16q+15.  Task {sn, row tile, -, -},
-// blockIdx.y = right-hand-side chunk.
+// Off-diagonal updates of the dependency-driven solve on MFMA, one workgroup
+// per (64 panel rows below the diagonal block, 16 right-hand sides); wave q
+// owns rows 16q..16q+15.
 // Forward:  Y[row(a)] -= sum_k L(a,k) X_I(k)      (one atomic per output)
 template <typename T>
 __device__ __forceinline__ void soffm_fwd_body(const SolvePanel& s, int rt, const T* __restrict__ arena,
@@ -1702,17 +1701,6 @@ __device__ __forceinline__ void soffm_fwd_body(const SolvePanel& s, int rt, cons
     const int a = a0 + Mfma<T>::row(lane, v);
     if (a < m) atomic_add(Y + (int64_t)lindx0[s.lx + s.w + a] * nrhs + jn, -acc[v]);
   }
-}
-
-template <typename T>
-__global__ __launch_bounds__(NT) void k_soffm_fwd(const SolvePanel* __restrict__ sn,
-                                                   const Task4* __restrict__ tasks,
-                                                   const T* __restrict__ arena,
-                                                   const int32_t* __restrict__ lindx0,
-                                                   const T* __restrict__ X, T* __restrict__ Y,
-                                                   int nrhs) {
-  const Task4 t = tasks[blockIdx.x];
-  soffm_fwd_body<T>(sn[t.a], t.b, arena, lindx0, X, Y, nrhs, blockIdx.y * SUB);
 }
 
 // Backward:  X_I(k) -= sum_{a in tile} L(a,k) Y[row(a)]   (partial sums over
@@ -1775,16 +1763,6 @@ __device__ __forceinline__ void soffm_bwd_body(const SolvePanel& s, int rt, cons
       }
     }
   }
-}
-
-template <typename T>
-__global__ __launch_bounds__(NT) void k_soffm_bwd(const SolvePanel* __restrict__ sn,
-                                                   const Task4* __restrict__ tasks,
-                                                   const T* __restrict__ arena,
-                                                   const int32_t* __restrict__ lindx0,
-                                                   T* __restrict__ X, int nrhs) {
-  const Task4 t = tasks[blockIdx.x];
-  soffm_bwd_body<T>(sn[t.a], t.b, arena, lindx0, X, nrhs, blockIdx.y * SUB);
 }
 
 // ---------------------------------------------------------------------------
@@ -1937,19 +1915,23 @@ __global__ __launch_bounds__(NT) void k_gprep(const SolvePanel* __restrict__ sn,
 // to Xf (LDL: divided by D_a), rows below are subtracted from Y at their
 // structure rows with atomics.  Y_I of a level's supernodes is never the
 // target of the same level's updates (targets are ancestors).
-template <typename T, bool LDL, int NBM>
+// SUBST (block substitution): the rows below the block only, G = L and the
+// solved X_I (in Xf) in place of Y_I; every right-hand-side block then reads L
+// from registers, not memory (80^3 LDL^T, 64 right-hand sides: 3.98 -> 3.28 ms
+// forward, 5.93 -> 4.26 ms backward).
+template <typename T, bool LDL, int NBM, bool SUBST>
 __global__ __launch_bounds__(NT) void k_gsolve_fwd(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                                    const T* __restrict__ garena, const T* __restrict__ arena,
-                                                   const int32_t* __restrict__ lindx0, T* Y, T* __restrict__ Xf,
+                                                   const int32_t* __restrict__ lindx0, T* Y, T* Xf,
                                                    int nrhs) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int NQ = 4 * NBM;  // k chunks of 4
   const Task4 t = tasks[blockIdx.x];
   const SolvePanel s = sn[t.a];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int a0 = t.b * TILE + 16 * wave;
-  if (a0 >= s.r) return;
   const int w = s.w;
+  const int a0 = (SUBST ? w : 0) + t.b * TILE + 16 * wave;
+  if (a0 >= s.r) return;
   const int64_t ld = s.ld;
   const int mi = lane & 15, g = lane >> 4;
   const int ac = min(a0 + mi, s.r - 1);
@@ -1968,14 +1950,14 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd(const SolvePanel* __restrict_
     const int a = a0 + Mfma<T>::row(lane, v);
     orow[v] = (a >= w && a < s.r) ? lindx0[s.lx + a] : -1;
     dinv[v] = T(1);
-    if (LDL && a < w) dinv[v] = T(1) / arena[s.off + (int64_t)a * ld + a];
+    if (LDL && !SUBST && a < w) dinv[v] = T(1) / arena[s.off + (int64_t)a * ld + a];
   }
   const int nblk = (nrhs + SUB - 1) / SUB;
   for (int jb = blockIdx.y; jb < nblk; jb += gridDim.y) {
     const int jn = jb * SUB + mi;
     const int jc = min(jn, nrhs - 1);
     const T jmask = T(jn < nrhs);
-    const T* __restrict__ Yk = Y + (int64_t)s.fc * nrhs + jc;  // Y_I(k, j) at Yk[k nrhs]
+    const T* __restrict__ Yk = (SUBST ? Xf : Y) + (int64_t)s.fc * nrhs + jc;  // Y_I(k, j) at Yk[k nrhs]
     T bv[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) bv[q] = Yk[(int64_t)min(4 * q + g, w - 1) * nrhs];
@@ -1991,7 +1973,7 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd(const SolvePanel* __restrict_
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int a = a0 + Mfma<T>::row(lane, v);
-        if (a < w)
+        if (!SUBST && a < w)
           Xf[(int64_t)(s.fc + a) * nrhs + jn] = LDL ? acc[v] * dinv[v] : acc[v];
         else if (orow[v] >= 0)
           atomic_add(Y + (int64_t)orow[v] * nrhs + jn, -acc[v]);
@@ -2009,19 +1991,19 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd(const SolvePanel* __restrict_
 // rather than 304 it also leaves room for more workgroups where a level has
 // hundreds of tiles (48^3, 600 tiles: 27 -> 19 us).  Task as k_gsolve_fwd's;
 // workgroup 4 t + q takes rows 16 q .. of task t's tile.
-template <typename T, bool LDL, int NBM>
+template <typename T, bool LDL, int NBM, bool SUBST>
 __global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                                     const T* __restrict__ garena, const T* __restrict__ arena,
-                                                    const int32_t* __restrict__ lindx0, T* Y, T* __restrict__ Xf,
+                                                    const int32_t* __restrict__ lindx0, T* Y, T* Xf,
                                                     int nrhs) {
   typedef typename Mfma<T>::v4 v4;
   __shared__ T part[4][4][64];
   const Task4 t = tasks[blockIdx.x >> 2];
   const SolvePanel s = sn[t.a];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int a0 = t.b * TILE + 16 * (int)(blockIdx.x & 3);
-  if (a0 >= s.r) return;  // the whole workgroup
   const int w = s.w, k0 = 4 * NBM * wave;
+  const int a0 = (SUBST ? w : 0) + t.b * TILE + 16 * (int)(blockIdx.x & 3);
+  if (a0 >= s.r) return;  // the whole workgroup
   const int64_t ld = s.ld;
   const int mi = lane & 15, g = lane >> 4;
   const T* __restrict__ Ga = garena + s.off + min(a0 + mi, s.r - 1);
@@ -2035,12 +2017,12 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SolvePanel* __restrict
   const int a = a0 + Mfma<T>::row(lane, wave);
   const int orow = (a >= w && a < s.r) ? lindx0[s.lx + min(a, s.r - 1)] : -1;
   T dinv = T(1);
-  if (LDL && a < w) dinv = T(1) / arena[s.off + (int64_t)a * ld + a];
+  if (LDL && !SUBST && a < w) dinv = T(1) / arena[s.off + (int64_t)a * ld + a];
   const int nblk = (nrhs + SUB - 1) / SUB;
   for (int jb = blockIdx.y; jb < nblk; jb += gridDim.y) {
     const int jn = jb * SUB + mi;
     const int jc = min(jn, nrhs - 1);
-    const T* __restrict__ Yk = Y + (int64_t)s.fc * nrhs + jc;
+    const T* __restrict__ Yk = (SUBST ? Xf : Y) + (int64_t)s.fc * nrhs + jc;
     T bv[NBM];
 #pragma unroll
     for (int q = 0; q < NBM; ++q) bv[q] = Yk[(int64_t)min(k0 + 4 * q + g, w - 1) * nrhs];
@@ -2058,7 +2040,7 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SolvePanel* __restrict
     __syncthreads();
     const T x = (part[0][wave][lane] + part[1][wave][lane]) + (part[2][wave][lane] + part[3][wave][lane]);
     if (jn < nrhs) {
-      if (a < w)
+      if (!SUBST && a < w)
         Xf[(int64_t)(s.fc + a) * nrhs + jn] = LDL ? x * dinv : x;
       else if (orow >= 0)
         atomic_add(Y + (int64_t)orow * nrhs + jn, -x);
@@ -2075,8 +2057,9 @@ __global__ __launch_bounds__(NT) void k_gsolve_fwd4(const SolvePanel* __restrict
 // (m, g) reads rows 16g..16g+15 of one G column (a cache line); the G values
 // stay in registers while the workgroup walks its right-hand-side blocks;
 // every load of a block is issued before its first product; partial sums of
-// the tile go to X_I with atomics (X zeroed before the sweep).
-template <typename T>
+// the tile go to X_I with atomics (X zeroed before the sweep).  SUBST: the
+// rows below the block only, G = L (X_I holds its right-hand side).
+template <typename T, bool SUBST>
 __global__ __launch_bounds__(NT) void k_gsolve_bwd(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                                    const T* __restrict__ garena,
                                                    const int32_t* __restrict__ lindx0, const T* __restrict__ Xf,
@@ -2087,7 +2070,7 @@ __global__ __launch_bounds__(NT) void k_gsolve_bwd(const SolvePanel* __restrict_
   const int lane = threadIdx.x & 63, kb = 4 * blockIdx.z + (threadIdx.x >> 6);
   const int w = s.w;
   if (16 * kb >= w) return;  // no barrier follows
-  const int a0 = t.b * TILE;
+  const int a0 = (SUBST ? w : 0) + t.b * TILE;
   const int mi = lane & 15, g = lane >> 4;
   int rowi[16];
 #pragma unroll
@@ -2105,8 +2088,9 @@ __global__ __launch_bounds__(NT) void k_gsolve_bwd(const SolvePanel* __restrict_
 #pragma unroll
     for (int st = 0; st < 16; ++st) {
       const int a = a0 + 16 * g + st;
-      const T* src = a < w ? Xf : X;
-      const T sg = a < w ? T(1) : T(-1);
+      const bool own = !SUBST && a < w;
+      const T* src = own ? Xf : X;
+      const T sg = own ? T(1) : T(-1);
       bv[st] = src[(int64_t)rowi[st] * nrhs + jc] * (jmask * T(a < s.r) * sg);
     }
 #pragma unroll
