@@ -51,7 +51,7 @@ inline unsigned grid_for(int64_t n, int block = 256) {
 }
 // k_gather_rhs / k_scatter_sol: one workgroup per 64 rows
 inline unsigned grid_rows64(int n) { return (unsigned)std::max(1, (n + 63) / 64); }
-enum TaskArr { TA_POTRF = 0, TA_TRSM, TA_INPANEL, TA_SCHUR, TA_SDIAG, TA_SOFF, TA_SOFFM, TA_FUSED, TA_GINV, TA_SCHUR_LPT, TA_WIDE, TA_WIDE_LPT };
+enum TaskArr { TA_POTRF = 0, TA_TRSM, TA_INPANEL, TA_SCHUR, TA_SDIAG, TA_NARROW, TA_SOFFM, TA_FUSED, TA_GINV, TA_SCHUR_LPT, TA_WIDE, TA_WIDE_LPT };
 }  // namespace
 
 namespace {
@@ -371,7 +371,7 @@ int64_t Engine::device_bytes(int nrhs) const {
   auto vb = [](const auto& v) { return (int64_t)(v.size() * sizeof(v[0])); };
   const Plan& p = plan_;
   int64_t b = vb(p.sn) + vb(p.lindx0) + p.upd_size * 16 + p.rel_size * 4 + vb(p.schur_heads) + vb(p.schur_segs) + vb(p.mmap) + vb(p.amap) + vb(p.perm0) +
-              vb(p.potrf_tasks) + vb(p.trsm_tasks) + vb(p.inpanel_tasks) +
+              vb(p.potrf_tasks) + vb(p.narrow_tasks) + vb(p.trsm_tasks) + vb(p.inpanel_tasks) +
               2 * (p.n_schur + p.n_schur_wide) * (int64_t)sizeof(Task4) + vb(p.fused_tasks) +
               vb(p.sdiag_tasks) + vb(p.soffm_tasks) + vb(p.panels);
   b += (int64_t)(n_ + 1) * 8 + nnzA_ * (4 + 4 + 8) + (int64_t)n_ * 8;  // CSC, values, scaling
@@ -466,6 +466,7 @@ void Engine::ensure_device() {
     d_invp0_ = dupload(invp0, s);
   }
   d_tasks_[TA_POTRF] = dupload(plan_.potrf_tasks, s);
+  d_tasks_[TA_NARROW] = dupload(plan_.narrow_tasks, s);
   d_tasks_[TA_TRSM] = dupload(plan_.trsm_tasks, s);
   d_tasks_[TA_INPANEL] = dupload(plan_.inpanel_tasks, s);
   {
@@ -799,6 +800,21 @@ void Engine::launch_diag(int bucket, bool ldl, unsigned g, const Task4* t, T* ar
 }
 
 template <typename T>
+void Engine::launch_narrow(int n, bool ldl, unsigned g, const Task4* t, T* arena) {
+  const SnInfo* sn = (const SnInfo*)d_sn_;
+  T* dinv = (T*)d_dinv_;
+  const unsigned wgs = (g + 3) / 4;
+  if (n == 8 && ldl)
+    dev::k_narrow<T, true, 8><<<wgs, 256, 0, stream_>>>(sn, t, g, arena, dinv, d_info_);
+  else if (n == 8)
+    dev::k_narrow<T, false, 8><<<wgs, 256, 0, stream_>>>(sn, t, g, arena, dinv, d_info_);
+  else if (ldl)
+    dev::k_narrow<T, true, 16><<<wgs, 256, 0, stream_>>>(sn, t, g, arena, dinv, d_info_);
+  else
+    dev::k_narrow<T, false, 16><<<wgs, 256, 0, stream_>>>(sn, t, g, arena, dinv, d_info_);
+}
+
+template <typename T>
 void Engine::launch_ptrsm(int bucket, bool ldl, unsigned g, const Task4* t, T* arena) {
   const SnInfo* sn = (const SnInfo*)d_sn_;
   const T* dinv = (const T*)d_dinv_;
@@ -897,8 +913,11 @@ void Engine::factor_sequence(T* arena) {
     launch_begin(r.kind, r.count, st, r.level);
     switch (r.kind) {
       case 0: {
-        const Task4* t = (const Task4*)d_tasks_[TA_POTRF] + r.first;
-        launch_diag<T>(r.aux, ldl, g, t, arena);
+        const Task4* t = (const Task4*)d_tasks_[r.aux > 0 ? TA_POTRF : TA_NARROW] + r.first;
+        if (r.aux > 0)
+          launch_diag<T>(r.aux, ldl, g, t, arena);
+        else
+          launch_narrow<T>(-r.aux, ldl, g, t, arena);
         break;
       }
       case 7: {

@@ -156,6 +156,8 @@ class Engine {
   template <typename T, bool BWD>
   void launch_sdiag(int bucket, unsigned g, const Task4* t, const T* arena, const T* Y, T* X, int nrhs);
   template <typename T>
+  void launch_narrow(int n, bool ldl, unsigned g, const Task4* t, T* arena);
+  template <typename T>
   void launch_ptrsm(int bucket, bool ldl, unsigned g, const Task4* t, T* arena);
   template <typename T>
   void launch_diagtrsm(int bucket, bool ldl, unsigned g, const Task4* t, T* arena);
@@ -248,8 +250,8 @@ class Engine {
   int32_t* d_mmap_ = nullptr;
   int64_t* d_amap_ = nullptr;
   int32_t* d_invp0_ = nullptr;  // original -> permuted row, 0-based
-  void* d_tasks_[12] = {nullptr};  // diag, trsm, inpanel, schur, sdiag, soff, soffm, fused, partitioned-inverse tiles,
-                                   // schur longest first, schur 128 x 64 (plan order, longest first)
+  void* d_tasks_[12] = {nullptr};  // diag, trsm, inpanel, schur, sdiag, narrow, soffm, fused, partitioned-inverse tiles,
+                                   // schur longest first, schur 128 x 128 (plan order, longest first)
   int* d_info_ = nullptr;
   int* d_fcnt_ = nullptr;  // per supernode: loads of the fused block factor + TRSM
   // dependency-driven solve

@@ -14,6 +14,7 @@
 //  k_ptrsm       panel TRSM of 64 rows below that block on MFMA with the
 //                inverted 16x16 diagonal tiles (blockCell_t::trsm, :1104-1178).
 //  k_diagtrsm    both, one workgroup per 64-row tile (each factors the block).
+//  k_narrow      both for a supernode of at most 16 columns, one wave.
 //  k_update      trailing update of a panel wider than 160 inside itself.
 //  k_schur       Schur update of ancestors: -P P^T (LDL: -P D P^T) on FP64 /
 //                FP32 MFMA 16x16x4, written straight from registers into the
@@ -313,6 +314,71 @@ struct DiagLds {
   int store;  // fused: this workgroup writes the factored block back
 };
 
+// The pivots of N columns held one row per lane: lanes 0 .. N-1 hold the rows
+// of the N x N diagonal tile, the others rows below it; a[] goes from the
+// unfactored to the factored row (LL: L_ij; LDL: l_ij below the diagonal, d_j
+// on it).  cb: the wave's LDS buffer.
+template <typename T, bool LDL, int N>
+__device__ __forceinline__ void chain_core(T (*__restrict__ cb)[SUB], int lane, T (&a)[N]) {
+  const bool diag_lane = lane < N;
+  // Column j of the diagonal rows (still unscaled) is broadcast through
+  // this wave's LDS buffer: LDS operations of one wave complete in order,
+  // so no barrier is needed between the write and the reads.  Column j+1
+  // is final on the diagonal rows as soon as step j has updated it (the
+  // first thing step j does), so it is published and read back in step j,
+  // a step ahead of its use: the LDS round trip stays off the wave's path.
+  T u[N];  // u[k], k >= j+3: column j of diagonal row k
+  if (diag_lane) cb[0][lane] = a[0];
+  compiler_fence();
+#pragma unroll
+  for (int k = 3; k < N; ++k) u[k] = cb[0][k];
+  compiler_fence();
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    // The dependency chain from one pivot to the next runs through
+    // readlane(pivot) -> 1/pivot -> the next row's diagonal entry; the
+    // next row's entry comes by readlane, and the scaling 1/sqrt(pivot)
+    // stays off the chain.
+    const T piv = readlane_t(a[j], j);
+    // u[j+1] and u[j+2] feed the next two pivots: readlane
+    if (j + 1 < N) u[j + 1] = readlane_t(a[j], j + 1);
+    if (j + 2 < N) u[j + 2] = readlane_t(a[j], j + 2);
+    // 1/piv from the hardware estimate y0 and e = 1 - piv y0:
+    // inv = y0 (1 + s) with s = e + e^2 (f64; |e| < 2^-24, so the error is
+    // e^3) or s = e (f32)
+    const T y0 = rcp_est(piv);
+    const T e = fma(-piv, y0, T(1));
+    const T s = rcp_corr(e);
+    const T inv = fma(y0, s, y0);
+    // a_k -= (a_j / piv) u_k.  The entry that feeds the next pivot is
+    // a - t (1 + s) with t = a_j u_{j+1} y0: t and e are formed side by
+    // side, so it is three dependent operations after the estimate
+    if (j + 1 < N) {
+      const T t = (a[j] * u[j + 1]) * y0;
+      a[j + 1] = fma(-t, s, a[j + 1] - t);
+    }
+    // column j+1 of the diagonal rows is final: publish it, read the next
+    // step's entries (k >= j+4)
+    T un[N];
+    if (j + 1 < N) {
+      if (diag_lane) cb[(j + 1) & 1][lane] = a[j + 1];
+      compiler_fence();
+#pragma unroll
+      for (int k = j + 4; k < N; ++k) un[k] = cb[(j + 1) & 1][k];
+      compiler_fence();
+    }
+    const T l = a[j] * inv;
+#pragma unroll
+    for (int k = j + 2; k < N; ++k) a[k] -= l * u[k];
+    // LL: L_ij = a_ij / sqrt(d_j), with 1/sqrt(d_j) formed from the
+    // uniform pivot off the chain; LDL stores l = a_ij / d_j and d_j
+    if (LDL) a[j] = (lane == j) ? piv : l;
+    else a[j] = a[j] * rsqrt_nr(piv);
+#pragma unroll
+    for (int k = j + 4; k < N; ++k) u[k] = un[k];
+  }
+}
+
 // One block column J of a diagonal block held in LDS (tiles (I, J), I >= J,
 // of tl), factored lane per row by one wave: lanes 0-15 hold the 16 rows of
 // the diagonal tile (every wave that calls this keeps its own copy, so the
@@ -336,62 +402,7 @@ __device__ __forceinline__ T* chain_column(T* __restrict__ tl, T (*__restrict__ 
   for (int c = 0; c < SUB; ++c) a[c] = trow[c * TSTR];
   // every wave reads the diagonal tile: wave 0 writes the factored one
   // back only after the barrier that ends this phase
-  // Column j of the diagonal rows (still unscaled) is broadcast through
-  // this wave's LDS buffer: LDS operations of one wave complete in order,
-  // so no barrier is needed between the write and the reads.  Column j+1
-  // is final on the diagonal rows as soon as step j has updated it (the
-  // first thing step j does), so it is published and read back in step j,
-  // a step ahead of its use: the LDS round trip stays off the wave's path.
-  T u[SUB];  // u[k], k >= j+3: column j of diagonal row k
-  if (diag_lane) cb[0][lane] = a[0];
-  compiler_fence();
-#pragma unroll
-  for (int k = 3; k < SUB; ++k) u[k] = cb[0][k];
-  compiler_fence();
-#pragma unroll
-  for (int j = 0; j < SUB; ++j) {
-    // The dependency chain from one pivot to the next runs through
-    // readlane(pivot) -> 1/pivot -> the next row's diagonal entry; the
-    // next row's entry comes by readlane, and the scaling 1/sqrt(pivot)
-    // stays off the chain.
-    const T piv = readlane_t(a[j], j);
-    // u[j+1] and u[j+2] feed the next two pivots: readlane
-    if (j + 1 < SUB) u[j + 1] = readlane_t(a[j], j + 1);
-    if (j + 2 < SUB) u[j + 2] = readlane_t(a[j], j + 2);
-    // 1/piv from the hardware estimate y0 and e = 1 - piv y0:
-    // inv = y0 (1 + s) with s = e + e^2 (f64; |e| < 2^-24, so the error is
-    // e^3) or s = e (f32)
-    const T y0 = rcp_est(piv);
-    const T e = fma(-piv, y0, T(1));
-    const T s = rcp_corr(e);
-    const T inv = fma(y0, s, y0);
-    // a_k -= (a_j / piv) u_k.  The entry that feeds the next pivot is
-    // a - t (1 + s) with t = a_j u_{j+1} y0: t and e are formed side by
-    // side, so it is three dependent operations after the estimate
-    if (j + 1 < SUB) {
-      const T t = (a[j] * u[j + 1]) * y0;
-      a[j + 1] = fma(-t, s, a[j + 1] - t);
-    }
-    // column j+1 of the diagonal rows is final: publish it, read the next
-    // step's entries (k >= j+4)
-    T un[SUB];
-    if (j + 1 < SUB) {
-      if (diag_lane) cb[(j + 1) & 1][lane] = a[j + 1];
-      compiler_fence();
-#pragma unroll
-      for (int k = j + 4; k < SUB; ++k) un[k] = cb[(j + 1) & 1][k];
-      compiler_fence();
-    }
-    const T l = a[j] * inv;
-#pragma unroll
-    for (int k = j + 2; k < SUB; ++k) a[k] -= l * u[k];
-    // LL: L_ij = a_ij / sqrt(d_j), with 1/sqrt(d_j) formed from the
-    // uniform pivot off the chain; LDL stores l = a_ij / d_j and d_j
-    if (LDL) a[j] = (lane == j) ? piv : l;
-    else a[j] = a[j] * rsqrt_nr(piv);
-#pragma unroll
-    for (int k = j + 4; k < SUB; ++k) u[k] = un[k];
-  }
+  chain_core<T, LDL, SUB>(cb, lane, a);
   // rows below: every valid lane (the trailing update reads them)
   if (!diag_lane && row_ok) {
 #pragma unroll
@@ -778,6 +789,75 @@ __global__ __launch_bounds__(NT) void k_diagtrsm(const SnInfo* __restrict__ sn,
   diag_body<T, LDL, NBM, true>(t, s, arena, dinv, info, L, cnt + tk.a, tk.b);
   const int bs = min(kStep, s.w);
   ptrsm_compute<T, LDL, NBM, kTrsmRows>(s, 0, bs, (bs + SUB - 1) / SUB, tk.c, arena + s.off, L.tl, L.ysh);
+}
+
+// Supernodes of at most N columns and 64 - N rows below them, one wave each
+// (four per workgroup): block factor, inverse tile and panel TRSM in one pass,
+// the rows below ride through the pivot chain.  A launch of thousands of such
+// supernodes is bound by the instructions of their pivot chains; with a
+// workgroup each, three of four waves idle through it and a second launch
+// does the TRSM (6,000 of 4 columns and 48 rows: k_diag 65 us and k_ptrsm; 30
+// us with N = 16, 16 us with N = 8).  Task {sn, -, inverse tile, -}.
+template <typename T, bool LDL, int N>
+__global__ __launch_bounds__(NT) void k_narrow(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks,
+                                               int64_t ntasks, T* __restrict__ arena, T* __restrict__ dinv,
+                                               int* __restrict__ info) {
+  __shared__ T colb[NT / 64][2][SUB];
+  __shared__ T tile[NT / 64][N][N + 1];  // tile[wave][c][r] = factored diagonal tile (r, c)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t task = (int64_t)blockIdx.x * (NT / 64) + wave;
+  if (task >= ntasks) return;  // the whole wave; no barriers below
+  const Task4 t = tasks[task];
+  const SnInfo s = sn[t.a];
+  const int w = s.w;
+  const int64_t ld = s.r;
+  T* __restrict__ P = arena + s.off;
+  T (*lt)[N + 1] = tile[wave];
+  const bool diag_lane = lane < N;
+  const int row = diag_lane ? lane : w + lane - N;
+  const bool row_ok = diag_lane ? lane < w : row < s.r;
+  T a[N];
+#pragma unroll
+  for (int c = 0; c < N; ++c) a[c] = P[(int64_t)min(c, w - 1) * ld + min(row, s.r - 1)];
+#pragma unroll
+  for (int c = 0; c < N; ++c) keep(a[c]);
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    if (diag_lane)  // lower triangle, identity past the width
+      a[c] = (c < w && lane < w && c <= lane) ? a[c] : T(c == lane ? 1 : 0);
+    else
+      a[c] = (c < w && row_ok) ? a[c] : T(0);
+  }
+  chain_core<T, LDL, N>(colb[wave], lane, a);
+  if (row_ok) {
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+      if (c < w && (!diag_lane || c <= lane)) P[(int64_t)c * ld + row] = a[c];
+  }
+  // factored tile to LDS (one wave's LDS accesses complete in order)
+  if (diag_lane) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) lt[c][lane] = a[c];
+  }
+  compiler_fence();
+  if (lane < SUB) {
+    const T dj = lt[min(lane, N - 1)][min(lane, N - 1)];
+    const bool bad = LDL ? (dj == T(0) || dj != dj) : !(dj > T(0));
+    if (bad && lane < w) atomicMin(info, s.fc + lane + 1);
+    // inverse of the 16 x 16 tile (identity past N): lane c solves L z = e_c
+    // (LDL: unit diagonal)
+    T z[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      T acc = (lane == i) ? T(1) : T(0);
+#pragma unroll
+      for (int k = 0; k < i; ++k) acc -= lt[k][i] * z[k];
+      z[i] = LDL ? acc : acc / lt[i][i];
+    }
+    T* out = dinv + (int64_t)t.c * (SUB * SUB) + lane * SUB;
+#pragma unroll
+    for (int i = 0; i < SUB; ++i) out[i] = i < N ? z[min(i, N - 1)] : T(lane == i ? 1 : 0);
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -11,6 +11,46 @@ namespace spk {
 
 namespace {
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Splits a level's items into launches by diagonal-block bucket.  A kernel
+// compiled for wide blocks holds up to 119 KB of LDS or 40 operand registers
+// also where the block is narrow, so one wide supernode on a level of
+// hundreds of narrow ones makes them all slow: narrower buckets get a launch
+// of their own when they have more than `enough` work units, otherwise they
+// ride along with the next wider one (a launch costs 3-5 us).  315^2, level
+// 1, 1,793 supernodes of one 16-column block and one of ten: block factors
+// and TRSM 131 -> 66 us, forward sweep 37 -> 14 us.
+struct BucketGroup {
+  int bucket;
+  std::vector<Int> items;
+};
+// The next bucket has to be four times as wide: 627 supernodes of two blocks
+// beside one of six cost 37 us together and 61 us apart.
+template <class BucketOf, class UnitsOf>
+std::vector<BucketGroup> bucket_groups(const std::vector<Int>& items, int64_t enough, BucketOf&& bucket_of,
+                                       UnitsOf&& units_of) {
+  std::vector<BucketGroup> out;
+  BucketGroup cur{1, {}};
+  int64_t units = 0;
+  for (int bk : {1, 2, 4, 6, 10}) {
+    bool any = false;
+    for (Int I : items) any |= bucket_of(I) == bk;
+    if (!any) continue;
+    if (units > enough && bk >= 4 * cur.bucket) {
+      out.push_back(std::move(cur));
+      cur.items.clear();
+      units = 0;
+    }
+    cur.bucket = bk;
+    for (Int I : items)
+      if (bucket_of(I) == bk) {
+        cur.items.push_back(I);
+        units += units_of(I);
+      }
+  }
+  if (!cur.items.empty()) out.push_back(std::move(cur));
+  return out;
+}
 }  // namespace
 
 void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, int baseval,
@@ -216,7 +256,6 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   constexpr double kChainMinFill = 0.85, kChainMaxSibling = 0.5;
   std::vector<int32_t> par(ns, -1), n1(ns, 0);
   std::vector<int32_t> link(ns, -1), prev(ns, -1);  // next / previous member of the chain
-  std::vector<int32_t> pos(n, -1);
   if (merge_updates > 0) {
     std::vector<int32_t> big(ns, -1), second(ns, 0);  // per parent: child with most rows, next one's rows
     auto rows_of = [&](Int I) { return p.sn[I].r - p.sn[I].w; };
@@ -278,6 +317,8 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   }
 
   // heads and their segments
+  p.schur_heads.reserve(ns);
+  p.schur_segs.reserve(2 * (size_t)ns);
   auto add_segment = [&](Int H, Int S) {
     const SnInfo& sh = p.sn[H];
     const SnInfo& sg = p.sn[S];
@@ -293,9 +334,15 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     g.shift = first;  // S has exactly H's rows there, or:
     if (sg.r - first != mH) {
       g.moff = (int64_t)p.mmap.size();
-      for (int32_t q = first; q < sg.r; ++q) pos[st[q]] = q;
-      for (int32_t a = 0; a < mH; ++a) p.mmap.push_back(pos[p.lindx0[sh.lx + sh.w + a]]);
-      for (int32_t q = first; q < sg.r; ++q) pos[st[q]] = -1;
+      p.mmap.resize(p.mmap.size() + mH);
+      int32_t* map = &p.mmap[g.moff];
+      const int32_t* rows = &p.lindx0[sh.lx + sh.w];  // sorted, as st is
+      int32_t q = first;
+      for (int32_t a = 0; a < mH; ++a) {
+        const bool has = q < sg.r && st[q] == rows[a];
+        map[a] = has ? q : -1;
+        q += has;
+      }
     }
     p.schur_segs.push_back(g);
     p.schur_heads.back().nseg++;
@@ -367,12 +414,33 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     // workgroup factors the block again) instead of two dependent launches.
     constexpr int64_t kFuseMaxTasks = 256;
     int64_t fuse_tasks = 0;
+    // Supernodes that fit one wave, in launches of their own where they are
+    // many or all that is left of the level (otherwise they ride along with
+    // the wider ones).
+    std::vector<Int> block_sns = sns;
+    for (int N : {8, 16}) {
+      const auto mid = std::stable_partition(block_sns.begin(), block_sns.end(), [&](Int I) {
+        return p.sn[I].w > N || p.sn[I].r - p.sn[I].w > 64 - N;
+      });
+      const int64_t nn = block_sns.end() - mid;
+      if (nn == 0 || (nn <= kNarrowMany && mid != block_sns.begin())) continue;
+      LaunchRange nr{0, (int64_t)p.narrow_tasks.size(), nn, -N};
+      for (auto it = mid; it != block_sns.end(); ++it) {
+        const SnInfo& si = p.sn[*it];
+        p.narrow_tasks.push_back({*it, 0, (int32_t)p.inv_base[*it], 0});
+        p.diag_flops += (double)si.w * si.w * si.w / 3.0 + (double)si.w * si.w * (si.r - si.w);
+      }
+      p.factor_seq.push_back(nr);
+      block_sns.erase(mid, block_sns.end());
+    }
+    smax = 0;
+    for (Int I : block_sns) smax = std::max<int>(smax, (int)ceil_div(p.sn[I].w, kStep));
     if (smax == 1)
-      for (Int I : sns) fuse_tasks += std::max<int64_t>(1, ceil_div(p.sn[I].r - p.sn[I].w, kTrsmRows));
+      for (Int I : block_sns) fuse_tasks += std::max<int64_t>(1, ceil_div(p.sn[I].r - p.sn[I].w, kTrsmRows));
     if (smax == 1 && fuse_tasks <= kFuseMaxTasks) {
       LaunchRange fr{9, (int64_t)p.fused_tasks.size(), 0};
       int nbmax = 1;
-      for (Int I : sns) {
+      for (Int I : block_sns) {
         const SnInfo& si = p.sn[I];
         const int bs = si.w;
         nbmax = std::max(nbmax, (int)ceil_div(bs, kSub));
@@ -389,40 +457,45 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
       smax = 0;  // nothing left for the per-step launches below
     }
     for (int st = 0; st < smax; ++st) {
-      LaunchRange pr{0, (int64_t)p.potrf_tasks.size(), 0};
-      LaunchRange tr{7, (int64_t)p.trsm_tasks.size(), 0};
       LaunchRange ur{1, (int64_t)p.inpanel_tasks.size(), 0};
-      int nbmax = 1;
-      for (Int I : sns) {
-        const SnInfo& si = p.sn[I];
-        int nsteps = (int)ceil_div(si.w, kStep);
-        if (st >= nsteps) continue;
-        int c0 = st * kStep, bs = std::min(kStep, si.w - c0);
-        int nb = (int)ceil_div(bs, kSub);
-        nbmax = std::max(nbmax, nb);
-        int64_t rows_below = si.r - c0 - bs;
-        int32_t inv_off = (int32_t)(p.inv_base[I] + (int64_t)st * (kStep / kSub));
-        p.potrf_tasks.push_back({I, st, inv_off, 0});
-        for (int64_t rt = 0; rt < ceil_div(rows_below, kTrsmRowsWide); ++rt)
-          p.trsm_tasks.push_back({I, st, (int32_t)rt, inv_off});
-        p.diag_flops += (double)bs * bs * bs / 3.0 + (double)bs * bs * rows_below;
-        if (st < nsteps - 1) {
-          int rb = c0 + bs;  // trailing rows/cols start
-          int64_t nrow = si.r - rb, ncol = si.w - rb;
-          int64_t ntr = ceil_div(nrow, kTile), ntc = ceil_div(ncol, kTile);
-          for (int64_t ti = 0; ti < ntr; ++ti)
-            for (int64_t tj = 0; tj < ntc && tj <= ti; ++tj)
-              p.inpanel_tasks.push_back({I, st, (int32_t)ti, (int32_t)tj});
-          // flops of the lower-trapezoid update with k = bs
-          p.inpanel_flops += (double)bs * ((double)ncol * (ncol + 1) + 2.0 * (nrow - ncol) * ncol);
+      std::vector<Int> active;
+      for (Int I : block_sns)
+        if (st * kStep < p.sn[I].w) active.push_back(I);
+      auto bucket_of = [&](Int I) {
+        return diag_bucket((int)ceil_div(std::min(kStep, p.sn[I].w - st * kStep), kSub));
+      };
+      constexpr int64_t kOneRound = 256;  // blocks that CUs with one workgroup each take at once
+      for (const BucketGroup& g : bucket_groups(active, kOneRound, bucket_of, [](Int) { return 1; })) {
+        LaunchRange pr{0, (int64_t)p.potrf_tasks.size(), 0};
+        LaunchRange tr{7, (int64_t)p.trsm_tasks.size(), 0};
+        for (Int I : g.items) {
+          const SnInfo& si = p.sn[I];
+          int nsteps = (int)ceil_div(si.w, kStep);
+          int c0 = st * kStep, bs = std::min(kStep, si.w - c0);
+          int64_t rows_below = si.r - c0 - bs;
+          int32_t inv_off = (int32_t)(p.inv_base[I] + (int64_t)st * (kStep / kSub));
+          p.potrf_tasks.push_back({I, st, inv_off, 0});
+          for (int64_t rt = 0; rt < ceil_div(rows_below, kTrsmRowsWide); ++rt)
+            p.trsm_tasks.push_back({I, st, (int32_t)rt, inv_off});
+          p.diag_flops += (double)bs * bs * bs / 3.0 + (double)bs * bs * rows_below;
+          if (st < nsteps - 1) {
+            int rb = c0 + bs;  // trailing rows/cols start
+            int64_t nrow = si.r - rb, ncol = si.w - rb;
+            int64_t ntr = ceil_div(nrow, kTile), ntc = ceil_div(ncol, kTile);
+            for (int64_t ti = 0; ti < ntr; ++ti)
+              for (int64_t tj = 0; tj < ntc && tj <= ti; ++tj)
+                p.inpanel_tasks.push_back({I, st, (int32_t)ti, (int32_t)tj});
+            // flops of the lower-trapezoid update with k = bs
+            p.inpanel_flops += (double)bs * ((double)ncol * (ncol + 1) + 2.0 * (nrow - ncol) * ncol);
+          }
         }
+        pr.aux = tr.aux = g.bucket;
+        pr.count = (int64_t)p.potrf_tasks.size() - pr.first;
+        tr.count = (int64_t)p.trsm_tasks.size() - tr.first;
+        if (pr.count) p.factor_seq.push_back(pr);
+        if (tr.count) p.factor_seq.push_back(tr);
       }
-      pr.aux = tr.aux = diag_bucket(nbmax);
-      pr.count = (int64_t)p.potrf_tasks.size() - pr.first;
-      tr.count = (int64_t)p.trsm_tasks.size() - tr.first;
       ur.count = (int64_t)p.inpanel_tasks.size() - ur.first;
-      if (pr.count) p.factor_seq.push_back(pr);
-      if (tr.count) p.factor_seq.push_back(tr);
       if (ur.count) p.factor_seq.push_back(ur);
     }
     // Schur tasks: counted here, written on the device (schur_emit)
@@ -536,38 +609,43 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   // Per level: one diagonal task per panel, one off-diagonal task per 64-row
   // tile below the diagonal block, and for the partitioned inverse one task
   // per 64-row tile of the whole panel.
-  std::vector<LaunchRange> diag(nslevels), offd(nslevels), part(nslevels);
-  for (int L = 0; L < nslevels; ++L) {
-    diag[L] = {3, (int64_t)p.sdiag_tasks.size(), 0, 1, L};
-    offd[L] = {4, (int64_t)p.soffm_tasks.size(), 0, 1, L};
-    part[L] = {10, (int64_t)p.gtiles.size(), 0, 1, L};
-    for (Int q : panels_at[L]) {
-      const SolvePanel& sp = p.panels[q];
-      diag[L].aux = std::max(diag[L].aux, bucket_of(q));
-      p.sdiag_tasks.push_back({q, inv_of[q], 0, 0});
-      for (int64_t rt = 0; rt < ceil_div(sp.r - sp.w, kTile); ++rt) p.soffm_tasks.push_back({q, (int32_t)rt, 0, 0});
-      for (int64_t rt = 0; rt < ceil_div(sp.r, kTile); ++rt) p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
+  struct SolveGroup {
+    LaunchRange diag, offd, part;
+  };
+  std::vector<SolveGroup> groups;  // levels bottom-up
+  constexpr int64_t kManyTiles = 512;
+  for (int L = 0; L < nslevels; ++L)
+    for (const BucketGroup& g : bucket_groups(panels_at[L], kManyTiles, bucket_of,
+                                              [&](Int q) { return ceil_div(p.panels[q].r, kTile); })) {
+      SolveGroup sg{{3, (int64_t)p.sdiag_tasks.size(), 0, g.bucket, L},
+                    {4, (int64_t)p.soffm_tasks.size(), 0, g.bucket, L},
+                    {10, (int64_t)p.gtiles.size(), 0, g.bucket, L}};
+      for (Int q : g.items) {
+        const SolvePanel& sp = p.panels[q];
+        p.sdiag_tasks.push_back({q, inv_of[q], 0, 0});
+        for (int64_t rt = 0; rt < ceil_div(sp.r - sp.w, kTile); ++rt) p.soffm_tasks.push_back({q, (int32_t)rt, 0, 0});
+        for (int64_t rt = 0; rt < ceil_div(sp.r, kTile); ++rt) p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
+      }
+      sg.diag.count = (int64_t)p.sdiag_tasks.size() - sg.diag.first;
+      sg.offd.count = (int64_t)p.soffm_tasks.size() - sg.offd.first;
+      sg.part.count = (int64_t)p.gtiles.size() - sg.part.first;
+      groups.push_back(sg);
     }
-    diag[L].count = (int64_t)p.sdiag_tasks.size() - diag[L].first;
-    offd[L].count = (int64_t)p.soffm_tasks.size() - offd[L].first;
-    part[L].count = (int64_t)p.gtiles.size() - part[L].first;
-    offd[L].aux = part[L].aux = diag[L].aux;
-  }
   // forward: levels bottom-up, diagonal solves then off-diagonal updates;
   // backward: levels top-down, off-diagonal gathers then diagonal solves
-  for (int L = 0; L < nslevels; ++L) {
-    p.fwd_seq.push_back(diag[L]);
-    if (offd[L].count) p.fwd_seq.push_back(offd[L]);
-    p.gfwd_seq.push_back(part[L]);
+  for (const SolveGroup& g : groups) {
+    p.fwd_seq.push_back(g.diag);
+    if (g.offd.count) p.fwd_seq.push_back(g.offd);
+    p.gfwd_seq.push_back(g.part);
   }
-  for (int L = nslevels - 1; L >= 0; --L) {
-    LaunchRange d = diag[L], o = offd[L], g = part[L];
+  for (auto g = groups.rbegin(); g != groups.rend(); ++g) {
+    LaunchRange d = g->diag, o = g->offd, q = g->part;
     d.kind = 6;
     o.kind = 5;
-    g.kind = 11;
+    q.kind = 11;
     if (o.count) p.bwd_seq.push_back(o);
     p.bwd_seq.push_back(d);
-    p.gbwd_seq.push_back(g);
+    p.gbwd_seq.push_back(q);
   }
   // preparation of the partitioned inverse: the same tiles, regrouped by the
   // bucket of their own panel (appended after the level-ordered tiles)

@@ -25,6 +25,9 @@ constexpr int kStep = 160;   // panel columns factored per step (diagonal block 
 constexpr int kSub = 16;     // sub-block edge inside a diagonal block (MFMA 16x16 tiles)
 constexpr int kTrsmRows = 64;  // panel rows per fused block factor + TRSM workgroup (16 per wave)
 constexpr int kTrsmRowsWide = 128;  // panel rows per k_ptrsm workgroup (8 waves of 16 rows)
+// supernodes that fit one wave (k_narrow<N>, N = 8 or 16: at most N columns and
+// 64 - N rows below) get a launch of their own above this many
+constexpr int64_t kNarrowMany = 256;
 constexpr int kSchurKC = 32;   // k columns per LDS chunk of the Schur update
 // Schur launches with fewer tasks than this (one per CU of the 256) split
 // each task's k chunks over several workgroups; more splitting costs more in
@@ -141,7 +144,7 @@ struct LaunchRange {
                      // 10 forward / 11 backward partitioned-inverse solve, 12 its preparation
   int64_t first;     // first task in that kind's task array
   int64_t count;     // number of tasks (= grid size)
-  int aux = 0;       // kinds 0, 7, 9, 3, 6: diagonal-block bucket (diag_bucket);
+  int aux = 0;       // kinds 0, 7, 9, 3, 6: diagonal-block bucket (diag_bucket; kind 0: -N = k_narrow<N>);
                      // kind 2: k-chunk split factor (0 or 1 = none)
   int level = 0;     // etree level of the launch (factor sequence)
   int alt = 0;       // kind 2: bit 0 = tasks in longest-first order, bit 1 = 128 x 128
@@ -169,6 +172,7 @@ struct Plan {
   std::vector<int32_t> perm0;      // perm0[new] = old, 0-based
   // task arrays
   std::vector<Task4> potrf_tasks;  // {sn, step, inverse-tile offset, 0}
+  std::vector<Task4> narrow_tasks; // {sn, 0, inverse-tile offset, 0}: whole panels of k_narrow
   std::vector<Task4> trsm_tasks;   // {sn, step, row_tile, inverse-tile offset}
   int64_t inv_tiles = 0;           // 16x16 inverse diagonal tiles written by the factor
   std::vector<int64_t> inv_base;   // per supernode: first inverse tile (tile t of 16-column block t)
