@@ -1904,8 +1904,9 @@ __device__ __forceinline__ void stage_block_and_inverses(const SolvePanel& s, in
 // 16 rows per wave (Y^T in MFMA accumulators, as in the panel TRSM).  A wide
 // panel's block fills the LDS of a CU with one workgroup, so nothing else hides
 // its memory latency: the right-hand sides are loaded ahead of the staging of
-// the block, both in flight at once (FP64, 160 columns: 381 -> 362 us at 48^3,
-// 835 -> 798 us at 60^3 27-point).  Task {sn, row tile, inverse-tile base, -}.
+// the block, both in flight at once (FP64, 160 columns: 381 -> 362 us at 48^3;
+// 60^3 27-point 798 us against 806 and 835 us in two runs before; the whole
+// step there 14824 -> 14752 us).  Task {sn, row tile, inverse-tile base, -}.
 template <typename T, int NBM>
 __global__ __launch_bounds__(NT) void k_gprep(const SolvePanel* __restrict__ sn, const Task4* __restrict__ tasks,
                                               const T* __restrict__ arena, const T* __restrict__ dinv,
