@@ -529,8 +529,8 @@ def main():
                                               (5, "bwd_offdiag"), (6, "bwd_diag"),
                                               (10, "fwd_partitioned_inverse"), (11, "bwd_partitioned_inverse"),
                                               (12, "partitioned_inverse_prep")]},
-        "roofline": {"kernel": "Schur-update launches (FP64 MFMA + atomic scatter; k_update<double,1>, "
-                               "k_schur_w1 or k_schur_wide per etree level as autotuned)",
+        "roofline": {"kernel": "Schur-update launches (FP64 MFMA + scatter; k_schur with 64x64 or 128x128 "
+                               "tiles or k_schur_w1 per etree level as autotuned)",
                      "timing": "HIP events around each Schur-update launch, %d host-launched "
                                "factorizations after the graph-replayed throughput loop" % args.steps,
                      "bound": "mfma",
