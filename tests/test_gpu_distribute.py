@@ -10,6 +10,7 @@ either side: the two quotients differ by at most 32 u plus their own
 rounding."""
 import numpy as np
 import pytest
+import torch  # before the library, so that both use the HIP runtime torch brings
 
 import sympack_amd as sp
 from oracle import numeric as onum
@@ -20,8 +21,6 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("device", [False, True], ids=["host", "device"])
 @pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 1025])
 def test_norm_and_scaling(n, device):
-    import torch
-
     rng = np.random.default_rng(n)
     # band of half-width 5, rows and columns scaled over six decades
     s = 10.0 ** rng.uniform(-3, 3, n)
