@@ -167,45 +167,67 @@ __global__ __launch_bounds__(256) void k_row_scale(const int64_t* __restrict__ r
 }
 
 // out = b - A x (b given) or out = A x, A symmetric as full CSR, vectors
-// column-major n x nrhs.  One thread per row, 16 right-hand sides per pass
-// over the row's entries (each entry read once per 16 right-hand sides, 16
-// independent x loads in flight): the lanes of a wave hold 64 consecutive
-// rows, so for a banded (grid) matrix an entry position reads 64 nearly
-// consecutive x values of each column.  The entries of a row are summed in
+// column-major n x nrhs.  A workgroup takes 64 rows, one wave per four columns
+// of every 16.  The entries of the rows are consecutive in memory: they are
+// read once, coalesced, into LDS, where a thread per row walking its own
+// entries in memory touches 64 cache lines per load; the x values of an entry
+// position are nearly consecutive for a grid matrix.  Rows of more than
+// kCsrStage entries in all are walked in memory instead.  Bound by the x reads
+// through the caches (60^3 27-point, 16 right-hand sides: 309 -> 65 us, 31 us
+// of HBM traffic; 80^3 7-point, 64: 568 -> 270 us, 173).  Of the staged shapes
+// 64 x 4 and 32 x 2 rows x columns measured alike, 16 x 1 10-20% slower, a
+// stage of 512 entries 184 us at 27 points.  The entries of a row are summed in
 // CSR order; no atomics.
+constexpr int kCsrRows = 64, kCsrCols = 4, kCsrStage = 2048;
 __global__ __launch_bounds__(256) void k_csr_mv(const int64_t* __restrict__ rowptr,
                                                 const int32_t* __restrict__ col,
                                                 const double* __restrict__ val,
                                                 const double* __restrict__ x,
                                                 const double* __restrict__ b,
                                                 double* __restrict__ out, int n, int nrhs) {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= n) return;
+  constexpr int JC = 256 / kCsrRows * kCsrCols;
+  __shared__ double sv[kCsrStage];
+  __shared__ int32_t sc[kCsrStage];
+  const int r0 = blockIdx.x * kCsrRows;
+  const int64_t e0 = rowptr[r0], e1 = rowptr[min(r0 + kCsrRows, n)];
+  const bool staged = e1 - e0 <= kCsrStage;  // uniform
+  if (staged)
+    for (int i = threadIdx.x; i < (int)(e1 - e0); i += 256) {
+      sv[i] = val[e0 + i];
+      sc[i] = col[e0 + i];
+    }
+  __syncthreads();
+  const int row = r0 + threadIdx.x % kCsrRows;
+  if (row >= n) return;  // no barrier follows
   const int64_t p0 = rowptr[row], p1 = rowptr[row + 1];
-  constexpr int JC = 16;
-  for (int j0 = 0; j0 < nrhs; j0 += JC) {
-    const int jn = min(JC, nrhs - j0);
-    const double* __restrict__ xj = x + (int64_t)j0 * n;
-    double acc[JC];
+  for (int j0 = threadIdx.x / kCsrRows * kCsrCols; j0 < nrhs; j0 += JC) {
+    const int jn = min(kCsrCols, nrhs - j0);
+    const double* __restrict__ xj[kCsrCols];  // past nrhs: the last column, not used
+    double acc[kCsrCols];
 #pragma unroll
-    for (int q = 0; q < JC; ++q) acc[q] = 0.0;
-    // the next entry's value and column are loaded before this entry's x
-    // values are used, so the column-index round trip overlaps them
-    double v = p0 < p1 ? val[p0] : 0.0;
-    int32_t c = p0 < p1 ? col[p0] : 0;
-    for (int64_t p = p0; p < p1; ++p) {
-      const bool more = p + 1 < p1;
-      const double vn = more ? val[p + 1] : 0.0;
-      const int32_t cn = more ? col[p + 1] : 0;
-      const double* __restrict__ xc = xj + c;
+    for (int q = 0; q < kCsrCols; ++q) {
+      xj[q] = x + (int64_t)min(j0 + q, nrhs - 1) * n;
+      acc[q] = 0.0;
+    }
+    if (staged) {
+      const int z = (int)(p1 - e0);
+#pragma unroll 2
+      for (int p = (int)(p0 - e0); p < z; ++p) {
+        const double v = sv[p];
+        const int c = sc[p];
 #pragma unroll
-      for (int q = 0; q < JC; ++q)
-        if (q < jn) acc[q] += v * xc[(int64_t)q * n];
-      v = vn;
-      c = cn;
+        for (int q = 0; q < kCsrCols; ++q) acc[q] += v * xj[q][c];
+      }
+    } else {
+      for (int64_t p = p0; p < p1; ++p) {
+        const double v = val[p];
+        const int c = col[p];
+#pragma unroll
+        for (int q = 0; q < kCsrCols; ++q) acc[q] += v * xj[q][c];
+      }
     }
 #pragma unroll
-    for (int q = 0; q < JC; ++q) {
+    for (int q = 0; q < kCsrCols; ++q) {
       if (q < jn) {
         const int64_t o = (int64_t)(j0 + q) * n + row;
         out[o] = b ? b[o] - acc[q] : acc[q];
@@ -287,7 +309,7 @@ void Engine::coldot(const double* a, const double* b, int nrhs, double* out) {
 
 // y = A x on the full CSR (FP64, original numbering)
 void Engine::csr_mv(const double* x, const double* b, double* out, int nrhs) {
-  k_csr_mv<<<grid_for(n_), 256, 0, stream_>>>(d_crow_, d_ccol_, d_cval_, x, b, out, n_, nrhs);
+  k_csr_mv<<<(unsigned)((n_ + kCsrRows - 1) / kCsrRows), 256, 0, stream_>>>(d_crow_, d_ccol_, d_cval_, x, b, out, n_, nrhs);
 }
 
 Engine::Engine() { kind_stats.resize(13); }
