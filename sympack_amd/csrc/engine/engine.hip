@@ -137,13 +137,33 @@ __global__ void k_gather_vals(double* __restrict__ cval, const double* __restric
   if (k < nnz) cval[k] = vals[src[k]];
 }
 
+// The entries of rows [r0, r0 + kCsrRows) of a full CSR, read coalesced into LDS
+// by a workgroup of 256 threads; false (uniform, nothing staged) where they
+// are more than kCsrStage.  Ends in a barrier.
+constexpr int kCsrRows = 64, kCsrStage = 2048;
+__device__ __forceinline__ bool stage_rows(int r0, int n, const int64_t* __restrict__ rowptr,
+                                           const int32_t* __restrict__ col, const double* __restrict__ val,
+                                           double* sv, int32_t* sc) {
+  const int64_t e0 = rowptr[r0], e1 = rowptr[min(r0 + kCsrRows, n)];
+  const bool staged = e1 - e0 <= kCsrStage;
+  if (staged)
+    for (int i = threadIdx.x; i < (int)(e1 - e0); i += 256) {
+      sv[i] = val[e0 + i];
+      sc[i] = col[e0 + i];
+    }
+  __syncthreads();
+  return staged;
+}
+
 // Per row of the full CSR: the equilibration scaling s_i = 1/sqrt(|a_ii|) of
 // the FP32 factor (1 where a_ii = 0; the last of duplicate diagonal entries
 // counts) and, over all rows, ||A||_inf.  A row's absolute values are summed
 // in CSR order, so the norm does not depend on the launch.  Bound by reading
 // A once; it takes the place of copying the values to the host and walking
 // them there (60^3 27-point, 2.9e6 stored values, MI355X: DistributeMatrix
-// 4.75 -> 0.23 ms; FP64, where only the copy remains: 4.56 -> 0.02 ms).
+// 4.75 -> 0.23 ms; FP64, where only the copy remains: 4.56 -> 0.02 ms).  64 rows
+// a workgroup, their entries staged as below; one wave walks the rows (60^3
+// 27-point: 162 -> 50 us).
 // *norm holds the bits of a non-negative double, whose order is that of the
 // integers; a NaN row sum is left out, as fmax does.
 __global__ __launch_bounds__(256) void k_row_scale(const int64_t* __restrict__ rowptr,
@@ -151,13 +171,25 @@ __global__ __launch_bounds__(256) void k_row_scale(const int64_t* __restrict__ r
                                                    const double* __restrict__ val,
                                                    double* __restrict__ scale, double* __restrict__ norm,
                                                    int n) {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ double sv[kCsrStage];
+  __shared__ int32_t sc[kCsrStage];
+  const int r0 = blockIdx.x * kCsrRows;
+  const int64_t e0 = rowptr[r0];
+  const bool staged = stage_rows(r0, n, rowptr, col, val, sv, sc);
+  const int row = r0 + threadIdx.x;
   double sum = 0.0, diag = 0.0;
-  if (row < n) {
-    for (int64_t p = rowptr[row]; p < rowptr[row + 1]; ++p) {
-      const double v = val[p];
-      sum += fabs(v);
-      if (col[p] == row) diag = v;
+  if (threadIdx.x < kCsrRows && row < n) {
+    const int64_t p0 = rowptr[row], p1 = rowptr[row + 1];
+    if (staged) {
+      for (int p = (int)(p0 - e0); p < (int)(p1 - e0); ++p) {
+        sum += fabs(sv[p]);
+        if (sc[p] == row) diag = sv[p];
+      }
+    } else {
+      for (int64_t p = p0; p < p1; ++p) {
+        sum += fabs(val[p]);
+        if (col[p] == row) diag = val[p];
+      }
     }
     scale[row] = diag != 0.0 ? 1.0 / sqrt(fabs(diag)) : 1.0;
   }
@@ -178,7 +210,7 @@ __global__ __launch_bounds__(256) void k_row_scale(const int64_t* __restrict__ r
 // 64 x 4 and 32 x 2 rows x columns measured alike, 16 x 1 10-20% slower, a
 // stage of 512 entries 184 us at 27 points.  The entries of a row are summed in
 // CSR order; no atomics.
-constexpr int kCsrRows = 64, kCsrCols = 4, kCsrStage = 2048;
+constexpr int kCsrCols = 4;
 __global__ __launch_bounds__(256) void k_csr_mv(const int64_t* __restrict__ rowptr,
                                                 const int32_t* __restrict__ col,
                                                 const double* __restrict__ val,
@@ -189,14 +221,8 @@ __global__ __launch_bounds__(256) void k_csr_mv(const int64_t* __restrict__ rowp
   __shared__ double sv[kCsrStage];
   __shared__ int32_t sc[kCsrStage];
   const int r0 = blockIdx.x * kCsrRows;
-  const int64_t e0 = rowptr[r0], e1 = rowptr[min(r0 + kCsrRows, n)];
-  const bool staged = e1 - e0 <= kCsrStage;  // uniform
-  if (staged)
-    for (int i = threadIdx.x; i < (int)(e1 - e0); i += 256) {
-      sv[i] = val[e0 + i];
-      sc[i] = col[e0 + i];
-    }
-  __syncthreads();
+  const int64_t e0 = rowptr[r0];
+  const bool staged = stage_rows(r0, n, rowptr, col, val, sv, sc);
   const int row = r0 + threadIdx.x % kCsrRows;
   if (row >= n) return;  // no barrier follows
   const int64_t p0 = rowptr[row], p1 = rowptr[row + 1];
@@ -611,7 +637,8 @@ void Engine::distribute(const double* nzval, bool on_device) {
   // the whole of DistributeMatrix.
   if (opt_.precision == 1) {
     dev::k_fill_zero<unsigned long long><<<1, 64, 0, stream_>>>((unsigned long long*)d_norm_, 1);
-    k_row_scale<<<grid_for(n_), 256, 0, stream_>>>(d_crow_, d_ccol_, d_cval_, d_scale_, d_norm_, n_);
+    k_row_scale<<<(unsigned)((n_ + kCsrRows - 1) / kCsrRows), 256, 0, stream_>>>(d_crow_, d_ccol_, d_cval_, d_scale_,
+                                                                                 d_norm_, n_);
     HIP_OK(hipGetLastError());
     HIP_OK(hipMemcpyAsync(&normA_inf_, d_norm_, sizeof(double), hipMemcpyDeviceToHost, stream_));
   }
