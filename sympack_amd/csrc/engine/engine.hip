@@ -1428,32 +1428,45 @@ void Engine::precond(const double* r, double* z, int nrhs) {
   HIP_OK(hipGetLastError());
 }
 
-// One preconditioned-CG iteration for every right-hand side (FP64 vectors).
-// Scalars live on the device: rho = d_s_[0,nrhs), p.q = [nrhs,2nrhs),
-// rho_new = [2nrhs,3nrhs).
-void Engine::pcg_iteration(int nrhs) {
-  const int64_t cnt = (int64_t)n_ * nrhs;
-  const unsigned g = grid_for(cnt);
-  double* rho = d_s_;
-  double* pq = d_s_ + nrhs;
-  double* rho_new = d_s_ + 2 * nrhs;
-  csr_mv(d_p_, nullptr, d_q_, nrhs);
-  coldot(d_p_, d_q_, nrhs, pq);
-  k_pcg_xr<<<g, 256, 0, stream_>>>(d_x_, d_r_, d_p_, d_q_, rho, pq, n_, nrhs);
-  precond(d_r_, d_z_, nrhs);
-  coldot(d_r_, d_z_, nrhs, rho_new);
-  k_pcg_p<<<g, 256, 0, stream_>>>(d_p_, d_z_, rho_new, rho, n_, nrhs);
-  dev::k_copy<<<1, 256, 0, stream_>>>(rho_new, rho, (int64_t)nrhs);
-  colmax2(d_r_, d_x_, nrhs, d_red_);
-  HIP_OK(hipGetLastError());
-}
+// Preconditioned CG for every right-hand side (FP64 vectors).  Scalars live on
+// the device: rho = d_s_[0,nrhs), p.q = [nrhs,2nrhs), rho_new = [2nrhs,3nrhs).
+// An iteration is a direction (a preconditioner application, which is most of
+// its time) and a step along it.  The step's residual decides whether another
+// direction is needed, so the direction opens the iteration: k iterations take k
+// preconditioner applications, where forming the next direction before the
+// test took k + 1 (60^3 27-point, 16 right-hand sides, 3 iterations: factor and
+// solve 14.49 -> 13.32 ms).
 
-// (Re)start: r given; z = M^{-1} r; p = z; rho = r.z.
+// Direction of the first iteration: r given; z = M^{-1} r; p = z; rho = r.z.
 void Engine::pcg_restart(int nrhs) {
   const int64_t cnt = (int64_t)n_ * nrhs;
   precond(d_r_, d_z_, nrhs);
   dev::k_copy<<<grid_for(cnt), 256, 0, stream_>>>(d_z_, d_p_, cnt);
   coldot(d_r_, d_z_, nrhs, d_s_);
+  HIP_OK(hipGetLastError());
+}
+
+// Direction of a later one: z = M^{-1} r; p = z + (rho_new / rho) p.
+void Engine::pcg_direction(int nrhs) {
+  const unsigned g = grid_for((int64_t)n_ * nrhs);
+  double* rho = d_s_;
+  double* rho_new = d_s_ + 2 * nrhs;
+  precond(d_r_, d_z_, nrhs);
+  coldot(d_r_, d_z_, nrhs, rho_new);
+  k_pcg_p<<<g, 256, 0, stream_>>>(d_p_, d_z_, rho_new, rho, n_, nrhs);
+  dev::k_copy<<<1, 256, 0, stream_>>>(rho_new, rho, (int64_t)nrhs);
+  HIP_OK(hipGetLastError());
+}
+
+// Step along p: x += alpha p; r -= alpha A p; column norms of r and x.
+void Engine::pcg_step(int nrhs) {
+  const unsigned g = grid_for((int64_t)n_ * nrhs);
+  double* rho = d_s_;
+  double* pq = d_s_ + nrhs;
+  csr_mv(d_p_, nullptr, d_q_, nrhs);
+  coldot(d_p_, d_q_, nrhs, pq);
+  k_pcg_xr<<<g, 256, 0, stream_>>>(d_x_, d_r_, d_p_, d_q_, rho, pq, n_, nrhs);
+  colmax2(d_r_, d_x_, nrhs, d_red_);
   HIP_OK(hipGetLastError());
 }
 
@@ -1701,9 +1714,19 @@ SolveReport Engine::solve(const double* rhs, int nrhs, bool on_device) {
     const int maxit = std::max(1, opt_.ir_max_iter);
     if (!opt_.ldl) {
       const int64_t kit = 4 * (int64_t)nrhs + 2, kst = 4 * (int64_t)nrhs + 3;
-      run_graph(solve_graph(kst), kst, [&] { pcg_restart(nrhs); });
+      bool restart = true;
       for (int it = 0; it < maxit; ++it) {
-        run_graph(solve_graph(kit), kit, [&] { pcg_iteration(nrhs); });
+        if (restart)
+          run_graph(solve_graph(kst), kst, [&] {
+            pcg_restart(nrhs);
+            pcg_step(nrhs);
+          });
+        else
+          run_graph(solve_graph(kit), kit, [&] {
+            pcg_direction(nrhs);
+            pcg_step(nrhs);
+          });
+        restart = false;
         double berr = read_berr();
         rep.iterations = it + 1;
         if (berr <= opt_.ir_tol || it + 1 == maxit) {
@@ -1715,7 +1738,7 @@ SolveReport Engine::solve(const double* rhs, int nrhs, bool on_device) {
             rep.converged = 1;
             break;
           }
-          run_graph(solve_graph(kst), kst, [&] { pcg_restart(nrhs); });
+          restart = true;
         }
         rep.backward_error = berr;
       }

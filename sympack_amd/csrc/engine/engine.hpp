@@ -194,8 +194,9 @@ class Engine {
   void colmax2(const double* r, const double* x, int nrhs, double* out);
   void coldot(const double* a, const double* b, int nrhs, double* out);
   void precond(const double* r, double* z, int nrhs);
-  void pcg_iteration(int nrhs);
   void pcg_restart(int nrhs);
+  void pcg_direction(int nrhs);
+  void pcg_step(int nrhs);
   void gmres_ir(int nrhs, const std::vector<double>& bnorm, SolveReport& rep);
   void launch_begin(int kind, int64_t grid = 0, hipStream_t st = nullptr, int level = -1);
   void launch_end(int kind, hipStream_t st = nullptr);
