@@ -234,6 +234,9 @@ int spk_get_update_merges(spk_handle h, int32_t* deferred_into /* nsuper */);
  * contributor's panel (-1: it has no such row). */
 int spk_get_update_schedule(spk_handle h, int32_t* nseg, int32_t* bcut, int32_t* excl /* nsuper each */);
 int spk_get_update_segment(spk_handle h, int32_t I, int32_t s, int32_t* sn, int32_t* rows);
+/* parts[I]: the k parts, tasks of their own, into which supernode I's update
+ * is split (0: it has no update). */
+int spk_get_update_parts(spk_handle h, int32_t* parts /* nsuper */);
 /* Checks the task lists of the dependency-driven solve (no counterpart in
  * the reference): 0 when a single worker taking tasks in ticket order never
  * waits and every counter drains, < 0 with spk_last_error() otherwise. */

@@ -116,6 +116,7 @@ SIGNATURES = [
     ("spk_get_update_merges", _I, [_P, _PI32]),
     ("spk_get_update_schedule", _I, [_P, _PI32, _PI32, _PI32]),
     ("spk_get_update_segment", _I, [_P, _I32, _I32, _PI32, _PI32]),
+    ("spk_get_update_parts", _I, [_P, _PI32]),
     ("spk_validate_solve_plan", _I, [_P]),
     ("spk_get_cells", _I, [_P, _PI32, _PI32, _PI32, _PI32, _PI32, _PI32]),
     ("spk_get_panel_dims", _I, [_P, _I32, _PI32, _PI32]),

@@ -576,6 +576,17 @@ int spk_get_update_segment(spk_handle h, int32_t I, int32_t s, int32_t* sn, int3
   });
 }
 
+int spk_get_update_parts(spk_handle h, int32_t* parts) {
+  if (!h || !parts) return fail("null argument");
+  return guarded([&]() {
+    const spk::Plan& p = h->engine.plan();
+    if ((int)p.chain_end.size() != p.nsuper) throw std::logic_error("no symbolic factorization");
+    std::fill_n(parts, p.nsuper, 0);
+    for (const spk::SchurEmit& e : p.schur_emit) parts[e.I] = e.split;
+    return 0;
+  });
+}
+
 int spk_get_cell_counts(spk_handle h, int64_t* ncells, int64_t* nblocks) {
   if (!h || !ncells || !nblocks) return fail("null argument");
   return guarded([&]() {

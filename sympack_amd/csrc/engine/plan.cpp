@@ -521,7 +521,7 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
       int64_t m = si.r - si.w;
       if (m <= 0) continue;
       SchurHead& h = p.schur_heads[head_of[I]];
-      h.split = (int32_t)std::max<int64_t>(1, h.nq / part_chunks);
+      h.split = (int32_t)std::min(kMaxParts, std::max<int64_t>(1, h.nq / part_chunks));
       SchurEmit e{};
       e.I = I;
       e.nt = (int32_t)ceil_div(m, kTile);

@@ -123,8 +123,10 @@ SPK_HD inline int64_t schur_tiles_before(int64_t ti, int64_t ntj) {
   return ti <= ntj ? ti * (ti + 1) / 2 : ntj * (ntj + 1) / 2 + (ti - ntj) * ntj;
 }
 
-// A Schur task is {sn, ti, tj | part << kTileBits, head}.
+// A Schur task is {sn, ti, tj | part << kTileBits, head}: a non-negative field
+// holds parts below kMaxParts.
 constexpr int kTileBits = 20, kTileMask = (1 << kTileBits) - 1;
+constexpr int64_t kMaxParts = int64_t(1) << (31 - kTileBits);
 
 // Per supernode with a Schur update: where its tasks go in
 // the four Schur task arrays (64 x 64 tiles in plan order and longest first,

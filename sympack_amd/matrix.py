@@ -455,6 +455,12 @@ class symPACKMatrix2D:
                    "segment")
         return sn.value, rows
 
+    def GetUpdateParts(self):
+        """Per supernode (0-based) the k parts of its Schur update, 0 for none."""
+        p = np.zeros(self.TotalSupernodeCnt(), np.int32)
+        _lib.check(self._lib.spk_get_update_parts(self._h, _ptr(p, ctypes.c_int32)), "parts")
+        return p
+
     def ValidateSolvePlan(self):
         """Raise if the dependency-driven solve's task lists are inconsistent."""
         _lib.check(self._lib.spk_validate_solve_plan(self._h), "solve plan")
