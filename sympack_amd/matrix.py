@@ -449,6 +449,10 @@ class symPACKMatrix2D:
         """Contributor s of supernode I's update: (supernode, its panel row
         per off-diagonal row of I, -1 where it has none); m = number of
         off-diagonal rows of I."""
+        r, w = ctypes.c_int32(), ctypes.c_int32()
+        _lib.check(self._lib.spk_get_panel_dims(self._h, I + 1, ctypes.byref(r), ctypes.byref(w)), "segment")
+        if m < r.value - w.value:
+            raise ValueError("supernode %d has %d off-diagonal rows, room for %d" % (I, r.value - w.value, m))
         sn = ctypes.c_int32()
         rows = np.zeros(m, np.int32)
         _lib.check(self._lib.spk_get_update_segment(self._h, I, s, ctypes.byref(sn), _ptr(rows, ctypes.c_int32)),

@@ -2,6 +2,7 @@
 of an update are at most as many as those bits count, also for a chain of tens
 of thousands of supernodes."""
 import numpy as np
+import pytest
 
 import sympack_amd as sp
 
@@ -30,3 +31,20 @@ def test_parts_of_a_long_chain():
     parts = M.GetUpdateParts()
     assert np.array_equal(parts > 0, nseg > 0)
     assert 1024 < parts.max() <= 1 << PART_BITS
+
+
+def test_segment_rows_need_room():
+    """The library writes one row per off-diagonal row of the supernode: less
+    room than that is refused before the call."""
+    n, cp, ri, v = sp.matrices.laplacian_2d_5pt(12)
+    M = sp.symPACKMatrix2D()
+    M.Init(sp.symPACKOptions(ordering="MMD"))
+    M.SymbolicFactorization(sp.DistSparseMatrix(n, cp, ri, v))
+    xs, (xl, _) = M.GetSupernodalPartition(), M.GetStructure()
+    m = np.diff(xl) - np.diff(xs)
+    I = int(np.argmax(m))
+    assert np.array_equal(M.GetUpdateSegment(I, 0, m[I])[1], np.arange(m[I]) + xs[I + 1] - xs[I])
+    with pytest.raises(ValueError):
+        M.GetUpdateSegment(I, 0, m[I] - 1)
+    with pytest.raises(sp.SymPACKError):
+        M.GetUpdateSegment(len(m), 0, n)
