@@ -38,7 +38,7 @@ def test_segment_rows_need_room():
     room than that is refused before the call."""
     n, cp, ri, v = sp.matrices.laplacian_2d_5pt(12)
     M = sp.symPACKMatrix2D()
-    M.Init(sp.symPACKOptions(ordering="MMD"))
+    M.Init(sp.symPACKOptions(ordering="MMD", relax=sp.RelaxationParameters(0, 0, 0)))
     M.SymbolicFactorization(sp.DistSparseMatrix(n, cp, ri, v))
     xs, (xl, _) = M.GetSupernodalPartition(), M.GetStructure()
     m = np.diff(xl) - np.diff(xs)
