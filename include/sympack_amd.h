@@ -77,12 +77,15 @@ typedef struct spk_options {
                          10*ordflag + altflag: 10, 11, 20, 21, 30, 31 for SET10 .. SET31
                          (SET = 31), 40 = TSPB (traveling-salesman tour with skeleton
                          compression), 41 = any other TSPB* name (tour without it) */
-  int solve_inverse;  /* 1 (default): the solve uses the partitioned inverse G = [I; L_off] L_diag^{-1}
-                         of each panel of at most 160 columns of a supernode (prepared once per
-                         factorization), one launch per level of panels and sweep; for LL^T and
-                         for the FP32 factor under refinement, not for FP64 static LDL^T (explicit
-                         inverses of its indefinite diagonal blocks lose accuracy).  0: block
-                         substitution, four launches per level */
+  int solve_inverse;  /* 1 (default): where every supernode is at most 160 columns wide, the
+                         solve uses the partitioned inverse G_I = [I; L_off] L_II^{-1} of each
+                         supernode (prepared once per factorization), one launch per etree level
+                         and sweep; for LL^T and for the FP32 factor under refinement, not for
+                         FP64 static LDL^T (explicit inverses of its indefinite diagonal blocks
+                         lose accuracy).  The backward error grows with the condition of the
+                         diagonal blocks: 4e-9 on a 150 x 150 covariance of condition 3e11, 3e-13
+                         with 0.  0, and wider supernodes: block substitution, four launches per
+                         level of panels of at most 160 columns */
   int autotune;       /* 1: the first spk_factorize of a structure with at least 1e9
                          Schur-update flops times every etree level's Schur launch under each
                          kernel (64 x 64 or 128 x 128 tiles staged through LDS, 64 x 64 tiles

@@ -391,7 +391,6 @@ void Engine::free_device() {
   dfree(d_dinv_);
   dfree(d_garena_);
   ginv_ready_ = false;
-  ginv_fits_ = true;
   dfree(d_Y_);
   dfree(d_X_);
   dfree(d_Xf_);
@@ -607,17 +606,10 @@ void Engine::ensure_device() {
   // inverted 16x16 diagonal tiles (double-sized so both precisions fit)
   d_dinv_ = dalloc<double>(std::max<int64_t>(1, plan_.inv_tiles) * kSub * kSub);
   if (use_ginv()) {
-    // a second arena; where it does not fit beside one of supernodes wider
-    // than a panel (whose fill can take most of the memory), the solve
-    // substitutes
-    const size_t bytes = (size_t)std::max<int64_t>(1, plan_.arena_elems) * (opt_.precision == 0 ? 8 : 4);
-    const hipError_t e = hipMalloc(&d_garena_, bytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      d_garena_ = nullptr;
-      if (e != hipErrorOutOfMemory || plan_.max_w <= kStep) HIP_OK(e);
-      ginv_fits_ = false;
-    }
+    if (opt_.precision == 0)
+      d_garena_ = dalloc<double>(plan_.arena_elems);
+    else
+      d_garena_ = dalloc<float>(plan_.arena_elems);
   }
   ginv_ready_ = false;
   HIP_OK(hipStreamSynchronize(s));
@@ -1180,27 +1172,30 @@ void Engine::launch_sdiag(int bucket, unsigned g, const Task4* t, const T* arena
   // right-hand sides, whole solve: 11.6 ms never, 10.7 ms up to 256
   // workgroups, 11.0 ms always
   const int64_t nblk = (nrhs + 15) / 16;
-  if (nblk == 1 || g * nblk <= kSdiagSpread) {
-    const dim3 grid(g, (unsigned)nblk);
-    switch (bucket) {
-      case 1: dev::k_sdiag4<T, BWD, 1><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 2: dev::k_sdiag4<T, BWD, 2><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 4: dev::k_sdiag4<T, BWD, 4><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 6: dev::k_sdiag4<T, BWD, 6><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      case 10: dev::k_sdiag4<T, BWD, 10><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-      default: throw std::logic_error("bad diagonal-block bucket");
-    }
-    return;
-  }
-  const dim3 grid(g, (unsigned)((nrhs + 63) / 64));
+  const bool spread = nblk == 1 || g * nblk <= kSdiagSpread;
+  const dim3 grid(g, (unsigned)(spread ? nblk : (nrhs + 63) / 64));
+  const bool unit = opt_.ldl != 0;
+  // corrected tile solves where the plan has supernodes wider than a panel
+#define SPK_SDIAG(NBM)                                                                                        \
+  case NBM:                                                                                                   \
+    if (spread && wide_plan())                                                                                \
+      dev::k_sdiag4<T, BWD, NBM, true><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs, unit);      \
+    else if (spread)                                                                                          \
+      dev::k_sdiag4<T, BWD, NBM, false><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs, unit);     \
+    else if (wide_plan())                                                                                     \
+      dev::k_sdiag3<T, BWD, NBM, true><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs, unit);      \
+    else                                                                                                      \
+      dev::k_sdiag3<T, BWD, NBM, false><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs, unit);     \
+    break;
   switch (bucket) {
-    case 1: dev::k_sdiag3<T, BWD, 1><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-    case 2: dev::k_sdiag3<T, BWD, 2><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-    case 4: dev::k_sdiag3<T, BWD, 4><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-    case 6: dev::k_sdiag3<T, BWD, 6><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
-    case 10: dev::k_sdiag3<T, BWD, 10><<<grid, 256, 0, stream_>>>(sn, t, arena, dinv, Y, X, nrhs); break;
+    SPK_SDIAG(1)
+    SPK_SDIAG(2)
+    SPK_SDIAG(4)
+    SPK_SDIAG(6)
+    SPK_SDIAG(10)
     default: throw std::logic_error("bad diagonal-block bucket");
   }
+#undef SPK_SDIAG
 }
 
 // Dependency-driven sweeps: reset the counters, one persistent forward

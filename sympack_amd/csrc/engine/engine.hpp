@@ -169,15 +169,23 @@ class Engine {
   void launch_sweep_fwd(const LaunchRange& r, const Task4* t, const T* G, const T* arena, T* Y, T* Xf, int nrhs);
   template <typename T, bool SUBST>
   void launch_sweep_bwd(const LaunchRange& r, const Task4* t, const T* G, const T* Xf, T* X, int nrhs);
-  // the partitioned-inverse solve applies and is switched on.
-  // Not for FP64 static LDL^T: explicit inverses of its unit-lower diagonal
-  // blocks (indefinite, static pivots) raise the backward error several
-  // times over block substitution (80^3-like shifted Laplacians: 6x on the
-  // host in exact block inverses, 26x measured at 48^3), beyond the
-  // drop-in's 10x bar; as the FP32 preconditioner under refinement it is
-  // used, the refinement restores the accuracy
+  bool wide_plan() const { return plan_.max_w > kStep; }
+  // The partitioned-inverse solve applies to this plan and is switched on.
+  // Its backward error grows with the condition of the panels' diagonal blocks
+  // (see diag_operand in kernels.hip for figures), so it is left to where it
+  // is refined or has a limit of kStep columns per supernode:
+  // - a plan with wider supernodes substitutes, panel by panel, with corrected
+  //   tile solves, in either precision (24^3, MMD, any width, values + factor +
+  //   solve: 1.84 ms, 1.43 ms with inverses at eight times the error); nor does
+  //   it hold a second arena beside a fill that can take most of the memory;
+  // - FP64 static LDL^T substitutes: explicit inverses of its unit-lower
+  //   diagonal blocks (indefinite, static pivots) raise the backward error
+  //   several times over block substitution (80^3-like shifted Laplacians: 6x
+  //   on the host in exact block inverses, 26x measured at 48^3), beyond the
+  //   drop-in's 10x bar; as the FP32 preconditioner under refinement it is
+  //   used, the refinement restores the accuracy
   bool use_ginv() const {
-    return opt_.solve_inverse != 0 && ginv_fits_ && (opt_.ldl == 0 || opt_.precision == 1);
+    return !wide_plan() && opt_.solve_inverse != 0 && (opt_.ldl == 0 || opt_.precision == 1);
   }
   // prepares G from the current factor once per factorization
   template <typename T>
@@ -276,7 +284,6 @@ class Engine {
   double* d_arena64_ = nullptr;
   void* d_dinv_ = nullptr;     // inverted 16x16 diagonal tiles of the factor
   void* d_garena_ = nullptr;   // partitioned-inverse solve factor G (panel shapes, factor precision)
-  bool ginv_fits_ = true;      // its memory was there
   bool ginv_ready_ = false;    // G holds the current factor's inverse
   float* d_arena32_ = nullptr;
   // solve work

@@ -1494,8 +1494,8 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
 
 // ---------------------------------------------------------------------------
 // Solve, panel by panel (SolvePanel: a supernode wider than kStep is a chain
-// of panels, 24^3 with MMD and widths up to 1,024: solve 1.59 -> 0.27 ms
-// against one workgroup per supernode in blocks of 64 columns).  Vectors are
+// of panels, 24^3 with MMD and widths up to 1,024, values + factor + solve: 2.76
+// -> 1.84 ms against one workgroup per supernode in blocks of 64 columns).  Vectors are
 // row-major n x nrhs in the permuted numbering.
 // Forward:  X_I = L_II^{-1} Y_I, then Y[struct rows] -= L_off X_I (atomics).
 //           LDL then scales by D^{-1} (k_scale_d).
@@ -1504,19 +1504,36 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
 // ---------------------------------------------------------------------------
 
 
+// Entry (m, kp) of the operand of diagonal tile K, L_KK (BWD: its transpose),
+// identity past the width w; unit: 1 on the diagonal.
+// A product with the inverse tile alone, z = inv(L_KK) y, is off by the tile's
+// condition, which pivots that decay inside 16 columns make large; one
+// correction z += inv(L_KK) (y - L_KK z) brings it back to substitution's
+// error.  Backward error on a 480 x 480 Gaussian covariance + 1e-10 I, one
+// supernode, MI355X: column by column 2.8e-16, corrected 2.7e-16, inverse tiles
+// alone 2.3e-14, partitioned inverses of 160 columns 4.1e-10.
+template <typename T, bool BWD>
+__device__ __forceinline__ T diag_operand(const T* __restrict__ P, int64_t ld, int w, bool unit, int K, int m,
+                                          int kp) {
+  const int r = SUB * K + (BWD ? kp : m), c = SUB * K + (BWD ? m : kp);
+  const T v = P[(int64_t)min(c, w - 1) * ld + min(r, w - 1)];
+  return r == c ? (r < w && !unit ? v : T(1)) : (r < w && r > c ? v : T(0));
+}
+
 // Diagonal-block solve on MFMA (w <= 160), the panel-TRSM recurrence with
 // right-hand sides in place of panel rows: for 16-row blocks t
 //   forward   x_t = inv(L_tt) (y_t - sum_{u<t} L_tu x_u)
 //   backward  x_t = inv(L_tt)^T (y_t - sum_{u>t} L_ut^T x_u)
 // Each wave owns 16 right-hand sides (x^T in MFMA accumulators, whose
 // layout is the B operand of the next product); a workgroup covers 64.
-// LDL: unit inverse tiles, D applied by k_scale_d.  Task {sn, inverse-tile
-// base, -, -}, blockIdx.y = chunk of 64 right-hand sides; Y may alias X.
-template <typename T, bool BWD, int NBM>
+// LDL (unit): unit inverse tiles, D applied by k_scale_d.  COR: each tile's
+// solve is corrected once (see diag_operand).  Task {panel, inverse-tile base,
+// -, -}, blockIdx.y = chunk of 64 right-hand sides; Y may alias X.
+template <typename T, bool BWD, int NBM, bool COR>
 __global__ __launch_bounds__(NT) void k_sdiag3(const SolvePanel* __restrict__ sn,
                                                const Task4* __restrict__ tasks,
                                                const T* __restrict__ arena, const T* __restrict__ dinv,
-                                               const T* Y, T* X, int nrhs) {
+                                               const T* Y, T* X, int nrhs, bool unit) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int NTL = NBM * (NBM + 1) / 2;
   __shared__ __attribute__((aligned(16))) T tl[NTL * TSZ];
@@ -1552,6 +1569,14 @@ __global__ __launch_bounds__(NT) void k_sdiag3(const SolvePanel* __restrict__ sn
         const bool in = (U == J) ? (U < nbt) : (row < w && col < w);
         tl[tslot(U, J) * TSZ + c * TSTR + r] = in ? v[tslot(U, J)] : T(0);
       }
+  }
+  T lt[COR ? NBM : 1][4];
+  if (COR) {
+#pragma unroll
+    for (int K = 0; K < NBM; ++K)
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        lt[K][kk] = diag_operand<T, BWD>(P, ld, w, unit, K, lane & 15, Mfma<T>::row(lane, kk));
   }
   __syncthreads();
   const int jb = blockIdx.y * 64 + 16 * wave;
@@ -1599,6 +1624,15 @@ __global__ __launch_bounds__(NT) void k_sdiag3(const SolvePanel* __restrict__ sn
         const int kp = Mfma<T>::row(lane, kk);
         z = Mfma<T>::mma(BWD ? Li[kp] : Li[kp * TSTR], x[K][kk], z);
       }
+      if (COR) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) x[K] = Mfma<T>::mma(-lt[K][kk], z[kk], x[K]);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const int kp = Mfma<T>::row(lane, kk);
+          z = Mfma<T>::mma(BWD ? Li[kp] : Li[kp * TSTR], x[K][kk], z);
+        }
+      }
       x[K] = z;
     }
   }
@@ -1624,11 +1658,12 @@ __global__ __launch_bounds__(NT) void k_sdiag3(const SolvePanel* __restrict__ sn
 // every wave folds it into the blocks it owns that still wait for it
 // (forward: K' > K; backward: K' < K), the next block first.  Same
 // recurrence as k_sdiag3, which handles each right-hand-side group with one
-// wave.  Task {sn, inverse-tile base, -, -}; Y may alias X.
-template <typename T, bool BWD, int NBM>
+// wave.  COR as there.  Task {panel, inverse-tile base, -, -}; Y may alias X.
+template <typename T, bool BWD, int NBM, bool COR>
 __device__ __forceinline__ void sdiag4_body(const SolvePanel& s, int64_t invb,
                                             const T* __restrict__ arena, const T* __restrict__ dinv,
-                                            const T* Y, T* X, int nrhs, int j0, T (*xs)[4][64]) {
+                                            const T* Y, T* X, int nrhs, int j0, bool unit,
+                                            T (*xs)[4][64]) {
   typedef typename Mfma<T>::v4 v4;
   constexpr int NO = (NBM + 3) / 4;  // blocks per wave
   const int w = s.w;
@@ -1656,7 +1691,7 @@ __device__ __forceinline__ void sdiag4_body(const SolvePanel& s, int64_t invb,
     }
   // Li[i][kk]: inverse diagonal tile of owned block i; Lf[i][K][kk] folds
   // block K into owned block i.  L(r, c) sits at P[c ld + r].
-  T Lf[NO][NBM][4], Li[NO][4];
+  T Lf[NO][NBM][4], Li[NO][4], lt[COR ? NO : 1][4];
 #pragma unroll
   for (int i = 0; i < NO; ++i)
 #pragma unroll
@@ -1665,6 +1700,7 @@ __device__ __forceinline__ void sdiag4_body(const SolvePanel& s, int64_t invb,
       const int Kc = min(wave + 4 * i, nbt - 1);
       // forward uses inv(L_KK)(m16, kp), backward its transpose
       Li[i][kk] = Dv[(int64_t)Kc * (SUB * SUB) + (BWD ? m16 * SUB + kp : kp * SUB + m16)];
+      if (COR) lt[i][kk] = diag_operand<T, BWD>(P, ld, w, unit, wave + 4 * i, m16, kp);
     }
 #pragma unroll
   for (int Ks = 0; Ks < NBM; ++Ks) {
@@ -1694,6 +1730,12 @@ __device__ __forceinline__ void sdiag4_body(const SolvePanel& s, int64_t invb,
         v4 z = v4{0, 0, 0, 0};
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) z = Mfma<T>::mma(Li[i][kk], xo[i][kk], z);
+        if (COR) {
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) xo[i] = Mfma<T>::mma(-lt[i][kk], z[kk], xo[i]);
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) z = Mfma<T>::mma(Li[i][kk], xo[i][kk], z);
+        }
         xo[i] = z;
 #pragma unroll
         for (int v = 0; v < 4; ++v) xs[K][v][lane] = z[v];
@@ -1727,14 +1769,14 @@ __device__ __forceinline__ void sdiag4_body(const SolvePanel& s, int64_t invb,
   __syncthreads();  // xs is reused by the next call
 }
 
-template <typename T, bool BWD, int NBM>
+template <typename T, bool BWD, int NBM, bool COR>
 __global__ __launch_bounds__(NT) void k_sdiag4(const SolvePanel* __restrict__ sn,
                                                const Task4* __restrict__ tasks,
                                                const T* __restrict__ arena, const T* __restrict__ dinv,
-                                               const T* Y, T* X, int nrhs) {
+                                               const T* Y, T* X, int nrhs, bool unit) {
   __shared__ __attribute__((aligned(16))) T xs[NBM][4][64];
   const Task4 t = tasks[blockIdx.x];
-  sdiag4_body<T, BWD, NBM>(sn[t.a], t.b, arena, dinv, Y, X, nrhs, SUB * blockIdx.y, xs);
+  sdiag4_body<T, BWD, NBM, COR>(sn[t.a], t.b, arena, dinv, Y, X, nrhs, SUB * blockIdx.y, unit, xs);
 }
 
 // Off-diagonal updates of the dependency-driven solve on MFMA, one workgroup
@@ -1846,8 +1888,8 @@ __device__ __forceinline__ void soffm_bwd_body(const SolvePanel& s, int rt, cons
 }
 
 // ---------------------------------------------------------------------------
-// Partitioned-inverse solve (supernodes at most kStep wide).  Per supernode
-// I (panel r x w, column-major, ld r) the solve factor
+// Partitioned-inverse solve (plans whose supernodes are at most kStep wide: a
+// panel is a supernode).  Per supernode I (panel r x w, column-major, ld r) the solve factor
 //   G_I = [I_w; L_off] L_II^{-1}
 // (LDL: L_II unit lower) is kept in an arena of the panel's shape.  Then
 //   forward  [X_I; dY] = G_I Y_I,  Y[struct rows] -= dY   (LDL: X_I /= D)
@@ -2301,7 +2343,7 @@ __global__ __launch_bounds__(NT) void k_fsolve_df(const SolvePanel* __restrict__
     if (t.a == 0) {
       df_wait(st.dcnt + t.b, 0, st.abort_);
       for (int j0 = 0; j0 < nrhs; j0 += SUB)
-        sdiag4_body<T, false, NBM>(s, invb[t.b], arena, dinv, Y, X, nrhs, j0, xs);
+        sdiag4_body<T, false, NBM, false>(s, invb[t.b], arena, dinv, Y, X, nrhs, j0, false, xs);
       df_release();
       if (threadIdx.x == 0) st_sys(st.dflag + t.b, 1);
     } else {
@@ -2339,7 +2381,7 @@ __global__ __launch_bounds__(NT) void k_bsolve_df(const SolvePanel* __restrict__
     } else {
       df_wait(st.rcnt + t.b, 0, st.abort_);
       for (int j0 = 0; j0 < nrhs; j0 += SUB)
-        sdiag4_body<T, true, NBM>(s, invb[t.b], arena, dinv, X, X, nrhs, j0, xs);
+        sdiag4_body<T, true, NBM, false>(s, invb[t.b], arena, dinv, X, X, nrhs, j0, false, xs);
       df_release();
       if (threadIdx.x == 0) st_sys(st.bflag + t.b, 1);
     }

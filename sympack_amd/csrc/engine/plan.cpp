@@ -607,8 +607,10 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
 
   // ---- solve task lists ----
   // Per level: one diagonal task per panel, one off-diagonal task per 64-row
-  // tile below the diagonal block, and for the partitioned inverse one task
-  // per 64-row tile of the whole panel.
+  // tile below the diagonal block, and for the partitioned inverse (where no
+  // supernode is wider than a panel) one task per 64-row tile of the whole
+  // panel.
+  const bool inverse = p.max_w <= kStep;
   struct SolveGroup {
     LaunchRange diag, offd, part;
   };
@@ -624,7 +626,8 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
         const SolvePanel& sp = p.panels[q];
         p.sdiag_tasks.push_back({q, inv_of[q], 0, 0});
         for (int64_t rt = 0; rt < ceil_div(sp.r - sp.w, kTile); ++rt) p.soffm_tasks.push_back({q, (int32_t)rt, 0, 0});
-        for (int64_t rt = 0; rt < ceil_div(sp.r, kTile); ++rt) p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
+        for (int64_t rt = 0; inverse && rt < ceil_div(sp.r, kTile); ++rt)
+          p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
       }
       sg.diag.count = (int64_t)p.sdiag_tasks.size() - sg.diag.first;
       sg.offd.count = (int64_t)p.soffm_tasks.size() - sg.offd.first;
@@ -636,7 +639,7 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   for (const SolveGroup& g : groups) {
     p.fwd_seq.push_back(g.diag);
     if (g.offd.count) p.fwd_seq.push_back(g.offd);
-    p.gfwd_seq.push_back(g.part);
+    if (inverse) p.gfwd_seq.push_back(g.part);
   }
   for (auto g = groups.rbegin(); g != groups.rend(); ++g) {
     LaunchRange d = g->diag, o = g->offd, q = g->part;
@@ -645,14 +648,14 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     q.kind = 11;
     if (o.count) p.bwd_seq.push_back(o);
     p.bwd_seq.push_back(d);
-    p.gbwd_seq.push_back(q);
+    if (inverse) p.gbwd_seq.push_back(q);
   }
   // preparation of the partitioned inverse: the same tiles, regrouped by the
   // bucket of their own panel (appended after the level-ordered tiles)
   for (int bk : {1, 2, 4, 6, 10}) {
     LaunchRange r{12, (int64_t)p.gtiles.size(), 0, bk, -1};
     for (Int q = 0; q < np; ++q) {
-      if (bucket_of(q) != bk) continue;
+      if (!inverse || bucket_of(q) != bk) continue;
       for (int64_t rt = 0; rt < ceil_div(p.panels[q].r, kTile); ++rt)
         p.gtiles.push_back({q, (int32_t)rt, inv_of[q], 0});
     }

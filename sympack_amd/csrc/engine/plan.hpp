@@ -203,7 +203,9 @@ struct Plan {
   std::vector<Task4> sdiag_tasks;  // {panel, inverse-tile base, 0, 0}: diagonal-block solves
   std::vector<Task4> soffm_tasks;  // {panel, row_tile, 0, 0}: 64-row tiles of the rows below the block
   std::vector<LaunchRange> fwd_seq, bwd_seq;  // kind 3/6 aux: diag_bucket of the level
-  // Partitioned-inverse solve: G = [I; L_off] L_diag^{-1} of every panel (its
+  // Partitioned-inverse solve, for plans without a supernode wider than kStep
+  // (a panel is then a supernode; lists empty otherwise):
+  // G = [I; L_off] L_diag^{-1} of every panel (its
   // shape and offsets, in an arena of its own) is prepared once per
   // factorization; then each level costs one forward launch
   // [X_p; dY] = G_p Y_p and one backward launch X_p = G_p^T [X_p; -X_rows].

@@ -90,7 +90,7 @@ class symPACKOptions:
         # SET10, SET11, SET20, SET21, SET30, SET31, TSPB (tour with skeleton
         # compression), other TSPB* names (tour without it)
         self.order_refinement_str = order_refinement_str
-        # partitioned-inverse solve
+        # partitioned-inverse solve where every supernode is <= 160 wide
         self.solve_inverse = solve_inverse
         # time the Schur launch configurations per etree level on the first
         # factorization (structures with >= 1e9 Schur flops)
