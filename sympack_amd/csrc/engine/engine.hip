@@ -426,7 +426,7 @@ int64_t Engine::device_bytes(int nrhs) const {
   if (!p.fused_tasks.empty()) b += (int64_t)p.nsuper * 4;               // fused-factor load counters
   const int64_t elem = opt_.precision == 0 ? 8 : 4;
   b += p.arena_elems * elem + std::max<int64_t>(1, p.inv_tiles) * kSub * kSub * 8;
-  if (opt_.solve_inverse) b += p.arena_elems * elem + vb(p.gtiles);  // G and its tiles
+  if (use_ginv()) b += p.arena_elems * elem + vb(p.gtiles);  // G and its tiles
   if (opt_.precision == 1)  // full CSR of A (row pointers, columns, sources, values), at most 2 nnz
     b += (int64_t)(n_ + 1) * 8 + 2 * nnzA_ * (4 + 8 + 8);
   b += 2 * (int64_t)std::max(1, nrhs) * kRedBlocks * 8;
