@@ -18,12 +18,16 @@ namespace spk {
 
 std::string hip_error_string(hipError_t e) { return std::string(hipGetErrorString(e)); }
 
+// The error is reported here, once: left behind, the thread's next check of its
+// launches would find it again.
 #define HIP_OK(expr)                                                                       \
   do {                                                                                     \
     hipError_t e_ = (expr);                                                                \
-    if (e_ != hipSuccess)                                                                  \
+    if (e_ != hipSuccess) {                                                                \
+      (void)hipGetLastError();                                                             \
       throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_) + " at " + \
                                __FILE__ + ":" + std::to_string(__LINE__) + " (" #expr ")");  \
+    }                                                                                      \
   } while (0)
 
 namespace {
@@ -1127,6 +1131,7 @@ int Engine::factorize() {
 
 void Engine::ensure_solve_capacity(int nrhs) {
   if (nrhs <= cap_nrhs_) return;
+  cap_nrhs_ = 0;  // until every buffer is there: an allocation may fail
   // captured solves refer to the old buffers
   for (auto& g : sgraphs_) destroy_graph(g);
   sgraphs_.clear();
@@ -1485,6 +1490,7 @@ void Engine::gmres_ir(int nrhs, const std::vector<double>& bnorm, SolveReport& r
   const int64_t cnt = (int64_t)n_ * nrhs;
   if (gm_cap_ < cnt * (2 * m + 1)) {
     dfree(d_gmV_);
+    gm_cap_ = 0;
     d_gmV_ = dalloc<double>((size_t)cnt * (2 * m + 1));  // V_0..V_m then Z_0..Z_{m-1}
     gm_cap_ = cnt * (2 * m + 1);
   }
@@ -1495,8 +1501,9 @@ void Engine::gmres_ir(int nrhs, const std::vector<double>& bnorm, SolveReport& r
   const int64_t need = hsize + (int64_t)kRedBlocks * m * nrhs;
   if (gm_hcap_ < need) {
     dfree(d_gmh_);
+    gm_hcap_ = 0;
+    d_gmh_ = dalloc<double>((size_t)need);
     gm_hcap_ = need;
-    d_gmh_ = dalloc<double>((size_t)gm_hcap_);
   }
   double* V = d_gmV_;
   double* Z = d_gmV_ + cnt * (m + 1);
