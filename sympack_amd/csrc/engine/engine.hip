@@ -1406,18 +1406,6 @@ __global__ void k_pcg_p(double* __restrict__ p, const double* __restrict__ z,
   }
 }
 
-// One refinement step: d = S (SAS)^{-1} S r in the factor's precision,
-// x += d, r = b - A x and the per-RHS norms, all on the device.
-template <typename T>
-void Engine::ir_step(T* Y, T* X, int nrhs) {
-  dev::k_gather_rhs<T><<<grid_rows64(n_), 256, 0, stream_>>>(d_r_, Y, d_invp0_, n_, nrhs, d_scale_);
-  solve_sequence<T>(d_arena32_, Y, X, nrhs);
-  dev::k_scatter_sol<T><<<grid_rows64(n_), 256, 0, stream_>>>(X, d_x_, d_invp0_, n_, nrhs, d_scale_, 1);
-  residual(d_b_, d_x_, d_r_, nrhs);
-  colmax2(d_r_, d_x_, nrhs, d_red_);
-  HIP_OK(hipGetLastError());
-}
-
 // z = S (L L^T)^{-1} S r with the FP32 factor of S A S (FP64 in and out).
 void Engine::precond(const double* r, double* z, int nrhs) {
   float* Y = (float*)d_Y_;

@@ -232,8 +232,6 @@ class Engine {
   std::vector<int> cap_kinds_;
   std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> cap_events_;
   std::vector<int64_t> cap_grids_;
-  template <typename T>
-  void ir_step(T* Y, T* X, int nrhs);
 
   EngineOptions opt_;
   Symbolic sym_;

@@ -8,10 +8,11 @@
 // unit-lower factor, as in symPACK's blockCellLDL_t
 // (include/sympack/symPACKMatrix2D.hpp:2096-2139).
 //
-// Kernels (one workgroup = 256 threads = 4 wave64):
+// Kernels (one workgroup = 256 threads = 4 wave64; k_ptrsm and k_schur's 128 x
+// 128 tiles: 512):
 //  k_diag        Cholesky/LDL^T of a diagonal block of up to 160 columns in
 //                LDS (blockCell_t::factorize, symPACKMatrix2D.hpp:1052-1102).
-//  k_ptrsm       panel TRSM of 64 rows below that block on MFMA with the
+//  k_ptrsm       panel TRSM of 128 rows below that block on MFMA with the
 //                inverted 16x16 diagonal tiles (blockCell_t::trsm, :1104-1178).
 //  k_diagtrsm    both, one workgroup per 64-row tile (each factors the block).
 //  k_narrow      both for a supernode of at most 16 columns, one wave.
@@ -625,7 +626,7 @@ __global__ __launch_bounds__(NT) void k_diag(const SnInfo* __restrict__ sn,
 }
 
 // ---------------------------------------------------------------------------
-// Panel TRSM of 64 rows below a factored diagonal block (blockCell_t::trsm,
+// Panel TRSM of 128 rows below a factored diagonal block (blockCell_t::trsm,
 // symPACKMatrix2D.hpp:1104-1178; LDL: blockCellLDL_t::trsm, :2118-2139):
 // X = B L^{-T} (LDL: B L^{-T} D^{-1}, unit L), blocked by 16 columns with the
 // inverted diagonal tiles of k_diag:
@@ -1254,8 +1255,9 @@ __global__ __launch_bounds__(64 * S::WA * S::WB, 4) void k_schur(
 // never stored); k past the width and a merged child's missing rows are
 // zeroed.  A diagonal tile loads one row set for both sides and skips the
 // six blocks above the diagonal; edge and deferred tiles skip the blocks
-// past m or past the column cut.  Scatter as in k_update: column bases from
-// a wave-private LDS copy of tcol / tmap, relative rows from rel, atomics.
+// past m or past the column cut.  The scatter takes column bases from a
+// wave-private LDS copy of tcol / tmap and relative rows from rel, as k_schur
+// does, and always atomics.
 // ---------------------------------------------------------------------------
 template <typename T, bool LDL, int SHAPE>
 __device__ __forceinline__ void w1_products(typename Mfma<T>::v4 (&acc)[4][4], const T (&ra)[4], const T (&rb)[4],
@@ -1457,7 +1459,7 @@ void k_schur_w1(const SnInfo* __restrict__ sn, const Task4* __restrict__ tasks, 
     sTm[wv][lane] = tmap[s.upd + bc];
   }
   // k runs in MFMA steps of 4; chunks of KC = 32 (8 steps) are the unit of
-  // the k split, as in k_update
+  // the k split, as in k_schur
   constexpr int SPC = KC / 4;
   const int nq1 = (K + KC - 1) / KC, nq = nq1 + (K2 + KC - 1) / KC;
   const int q_lo = (int)((int64_t)p * nq / np), q_hi = (int)((int64_t)(p + 1) * nq / np);

@@ -407,8 +407,6 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
       });
     for (Int I : sns) each_target(I, [&](const RelGroup& g) { return writers[g.J] = 0, true; });
     const size_t level_first = p.factor_seq.size();
-    int smax = 0;
-    for (Int I : sns) smax = std::max<int>(smax, (int)ceil_div(p.sn[I].w, kStep));
     // Levels of single-step supernodes with at most kFuseMaxTasks row
     // tiles in all: one fused block-factor + TRSM launch (every row-tile
     // workgroup factors the block again) instead of two dependent launches.
@@ -433,7 +431,7 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
       p.factor_seq.push_back(nr);
       block_sns.erase(mid, block_sns.end());
     }
-    smax = 0;
+    int smax = 0;
     for (Int I : block_sns) smax = std::max<int>(smax, (int)ceil_div(p.sn[I].w, kStep));
     if (smax == 1)
       for (Int I : block_sns) fuse_tasks += std::max<int64_t>(1, ceil_div(p.sn[I].r - p.sn[I].w, kTrsmRows));

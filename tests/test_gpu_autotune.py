@@ -1,6 +1,6 @@
 """The Schur-launch autotuner: on the first factorization of a large enough
 structure every etree level's Schur launch is timed under each Schur kernel
-(64 x 64 tiles staged through LDS, 128 x 64 tiles, 64 x 64 tiles with one
+(64 x 64 tiles staged through LDS, 128 x 128 tiles, 64 x 64 tiles with one
 wave per tile), task order and k split and the fastest is kept.  The tuned factorization must give the
 oracle's solution (1e-10 relative, the parity bar), and so must the
 refactorizations that replay the recaptured launch sequence; the tuner's
@@ -83,8 +83,8 @@ def test_small_structures_are_not_tuned():
     assert m.autotune_log() == []
 
 
-# Each Schur kernel forced on every level (schur_kernel 2: 128 x 64 tiles,
-# k_schur_wide; 3: 64 x 64 tiles with one wave per tile, k_schur_w1): plain
+# Each Schur kernel forced on every level (schur_kernel 2: 128 x 128
+# tiles; 3: 64 x 64 tiles with one wave per tile, k_schur_w1): plain
 # updates, merged chain updates (merge_updates=2 makes every qualifying chain
 # child defer into its parent) and deferred column cuts, LL^T and static
 # LDL^T, FP64 and FP32 + refinement.  Parity bar: solutions within 1e-10

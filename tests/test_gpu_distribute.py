@@ -1,6 +1,6 @@
 """DistributeMatrix on the GPU: equilibration scaling and ||A||_inf (FP32
-factor mode) at sizes around the kernel's block of 256 rows, from host and
-device values.
+factor mode) at sizes around a multiple of the kernel's blocks of 64 rows, from
+host and device values.
 
 One CG step from an FP32 factor leaves a backward error far above rounding;
 the library reports max |r| / (||A||_inf max |x| + max |b|).  The residual's
