@@ -176,8 +176,9 @@ class Engine {
   // is refined or has a limit of kStep columns per supernode:
   // - a plan with wider supernodes substitutes, panel by panel, with corrected
   //   tile solves, in either precision (24^3, MMD, any width, values + factor +
-  //   solve: 1.84 ms, 1.43 ms with inverses at eight times the error); nor does
-  //   it hold a second arena beside a fill that can take most of the memory;
+  //   solve: 1.84 ms, with inverses 1.43 ms and a backward error 1.2 times as
+  //   large there, 1e6 times on a covariance); nor does it hold a second arena
+  //   beside a fill that can take most of the memory;
   // - FP64 static LDL^T substitutes: explicit inverses of its unit-lower
   //   diagonal blocks (indefinite, static pivots) raise the backward error
   //   several times over block substitution (80^3-like shifted Laplacians: 6x
