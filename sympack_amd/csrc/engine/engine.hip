@@ -1264,7 +1264,9 @@ void Engine::ensure_ginv(const T* arena) {
 // diagonal blocks): 16 rows per workgroup, or 64 where narrow panels make
 // many tiles: little of the time is latency there, and four times the
 // workgroups cost more to start (60^3 27-point, level 0, 6,931 tiles of at
-// most 32 columns: 45 against 60 us).  Right-hand-side blocks of 16 per
+// most 32 columns: 45 against 60 us; 16 columns or fewer always with 64 rows:
+// solve of 200^2 at most 8 wide 512 -> 499 us, but 64^2 153 -> 159 and 40^2 RCM 971
+// -> 1017).  Right-hand-side blocks of 16 per
 // workgroup: a launch with at least kGinvGrid workgroups walks every block in
 // each (G read once); one with fewer spreads the blocks over up to kGinvGrid
 // workgroups.

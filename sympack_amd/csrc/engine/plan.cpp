@@ -25,7 +25,9 @@ struct BucketGroup {
   std::vector<Int> items;
 };
 // The next bucket has to be four times as wide: 627 supernodes of two blocks
-// beside one of six cost 37 us together and 61 us apart.
+// beside one of six cost 37 us together and 61 us apart.  Solve of 315^2, one
+// right-hand side: 222 us, 231 from twice as wide on, 235 never; 30^3 7-point 234,
+// 242, 234; eight other structures within 2% either way.
 template <class BucketOf, class UnitsOf>
 std::vector<BucketGroup> bucket_groups(const std::vector<Int>& items, int64_t enough, BucketOf&& bucket_of,
                                        UnitsOf&& units_of) {
@@ -252,7 +254,10 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
   // dissection grids) and no other child of P comes near it in rows: where
   // two separators of similar size meet, their parent's columns are outside
   // both chains.  Members narrower than one k chunk are left out in mode 1:
-  // a segment costs a whole chunk's staging.
+  // a segment costs a whole chunk's staging.  The two limits decide little:
+  // factor of 48^3 4.73 ms, 4.77 and 4.74 with 0.25 and 0.8 for siblings, 60^3
+  // 27-point 12.05, 12.09 and 12.03; 0.7 and 0.95 of fill change nothing beyond
+  // 0.3% there, on LDL^T 60^3 or under AMD.
   constexpr double kChainMinFill = 0.85, kChainMaxSibling = 0.5;
   std::vector<int32_t> par(ns, -1), n1(ns, 0);
   std::vector<int32_t> link(ns, -1), prev(ns, -1);  // next / previous member of the chain
@@ -414,7 +419,9 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     int64_t fuse_tasks = 0;
     // Supernodes that fit one wave, in launches of their own where they are
     // many or all that is left of the level (otherwise they ride along with
-    // the wider ones).
+    // the wider ones).  Few that are all of a level, factor against the fused
+    // block factor and TRSM: 40^2 RCM, at most 8 wide, 1613 against 2070 us, 64^2
+    // 267 against 291, 8^2 63.5 against 61.5.
     std::vector<Int> block_sns = sns;
     for (int N : {8, 16}) {
       const auto mid = std::stable_partition(block_sns.begin(), block_sns.end(), [&](Int I) {
@@ -503,8 +510,10 @@ void build_plan(const Symbolic& s, Int n, const Ptr* colptr, const Idx* rowind, 
     // A head with a long k loop (a chain's last member) is split into parts of
     // at least kPartChunks chunks, so that every resident workgroup gets
     // about four: 1,827 tiles of 60 chunks on 1,024 slots (60^3 27-point,
-    // level 36) 541 us whole, 529 us in two parts.  Shorter parts cost more
-    // in atomics than the balance gains.
+    // level 36) 541 us whole, 529 us in two parts.  Whole factorizations move
+    // by 1% either way: with 10, 20, 40 and no parts 27-point 60^3 12.06, 12.05,
+    // 12.13, 12.15 ms, 27-point 40^3 2.70, 2.73, 2.73, 2.73, 48^3 4.73, 4.73, 4.68,
+    // 4.68.
     constexpr int64_t kPartChunks = 20, kSlots = 1024;
     int64_t units = 0;  // chunks of all tiles of the level
     for (Int I : sns) {
